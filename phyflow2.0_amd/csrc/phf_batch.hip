@@ -219,75 +219,27 @@ __global__ void batch_gather(const BatchSys *__restrict__ sys, const int64_t *__
 __global__ void batch_clear_flag(int32_t *flag) { flag[0] = 0; }
 
 // --------------------------------------------------------------- P2M ------
-template <class T>
-__global__ __launch_bounds__(64) void batch_p2m(const BatchSys *__restrict__ sys,
-                                                const int64_t *__restrict__ loff,
-                                                const int64_t *__restrict__ lvl, int S,
-                                                const BatchDom *__restrict__ dom,
-                                                const void *__restrict__ src_,
-                                                const int32_t *__restrict__ start, int p1,
-                                                typename C2<T>::type *__restrict__ M)
+// one wave per leaf (p2m_leaf), four leaves per workgroup
+template <class T, int NI>
+__global__ __launch_bounds__(256) void batch_p2m(const BatchSys *__restrict__ sys,
+                                                 const int64_t *__restrict__ loff,
+                                                 const int64_t *__restrict__ lvl, int S,
+                                                 const BatchDom *__restrict__ dom,
+                                                 const void *__restrict__ src,
+                                                 const int32_t *__restrict__ start, int64_t nleaf,
+                                                 int p1, typename C2<T>::type *__restrict__ M)
 {
-    using V = typename C2<T>::type;
-    extern __shared__ unsigned char lds_raw[];
-    V *tab = reinterpret_cast<V *>(lds_raw);
-    const int lane = threadIdx.x;
-    const int64_t g = blockIdx.x;
+    const int64_t g = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (g >= nleaf) return;
     const int s = find_seg(loff, S, g);
     const int L = sys[s].L;
     if (L < 2) return;  // no far field in this system
     const uint32_t b = (uint32_t)(g - sys[s].leafbase);
-    const int32_t s0 = start[g], s1 = start[g + 1];
-    V acc = cmk<T>(0, 0);
-    if (s1 > s0) {
-        const BatchDom d = dom[s];
-        double cx, cy;
-        leaf_center(b, d.x0, d.y0, d.s, cx, cy);
-        const T inv_s = (T)(1.0 / d.s);
-        for (int32_t c0 = s0; c0 < s1; c0 += 64) {
-            const int32_t j = c0 + lane;
-            V z = cmk<T>(0, 0), q = cmk<T>(0, 0);
-            if (j < s1) {
-                if (sizeof(T) == 4) {
-                    const float4 p = reinterpret_cast<const float4 *>(src_)[j];
-                    z = cmk<T>((T)p.x * inv_s, (T)p.y * inv_s);
-                    q = cmk<T>((T)p.z, 0);
-                } else {
-                    const double4 p = reinterpret_cast<const double4 *>(src_)[j];
-                    z = cmk<T>((T)((p.x - cx) * (double)inv_s), (T)((p.y - cy) * (double)inv_s));
-                    q = cmk<T>((T)p.z, 0);
-                }
-            }
-            for (int k = 0; k < p1; ++k) {
-                tab[lane * p1 + k] = q;
-                q = cmul(q, z);
-            }
-            __syncthreads();
-            // term k summed by 64 / W lanes (k, k + W, ...), each over every
-            // (64 / W)-th point, then combined by shuffles: a chain of
-            // cnt W / 64 adds per lane instead of cnt
-            const int cnt = min(64, s1 - c0);
-            const int W = p1 <= 16 ? 16 : (p1 <= 32 ? 32 : 64);
-            const int k = lane & (W - 1), R = 64 / W;
-            V part = cmk<T>(0, 0);
-            if (k < p1)
-                for (int jj = lane / W; jj < cnt; jj += R) {
-                    const V t = tab[jj * p1 + k];
-                    part.x += t.x;
-                    part.y += t.y;
-                }
-            for (int o = W; o < 64; o <<= 1) {
-                part.x += __shfl_xor(part.x, o);
-                part.y += __shfl_xor(part.y, o);
-            }
-            if (lane < p1) {
-                acc.x += part.x;
-                acc.y += part.y;
-            }
-            __syncthreads();
-        }
-    }
-    if (lane < p1) M[(lvl[L * (S + 1) + s] + b) * p1 + lane] = acc;
+    const BatchDom d = dom[s];
+    double cx, cy;
+    leaf_center(b, d.x0, d.y0, d.s, cx, cy);
+    p2m_leaf<T, NI>(src, start[g], start[g + 1], cx, cy, (T)(1.0 / d.s), p1,
+                    M + (lvl[L * (S + 1) + s] + b) * p1);
 }
 
 // --------------------------------------------------------- M2M / L2L ------
@@ -1093,8 +1045,10 @@ static int batch_enqueue_typed(Lane *L, const BatchPlan &P, BatchBuffers &Bf, co
     const VC *m2m = reinterpret_cast<const VC *>(Bf.m2m);
     const VC *l2l = reinterpret_cast<const VC *>(Bf.l2l);
     if (P.Lmax >= 2) {
-        batch_p2m<T><<<(unsigned)P.nleaf, 64, (size_t)64 * p1 * sizeof(V), L->stream>>>(
-            Bf.sys, Bf.loff, Bf.lvl, S, Bf.dom, Bf.src, sp, p1, M);
+        PHF_TRY(p2m_dispatch(p1, [&](auto ni) {
+            batch_p2m<T, decltype(ni)::value><<<div_up(P.nleaf, 4), 256, 0, L->stream>>>(
+                Bf.sys, Bf.loff, Bf.lvl, S, Bf.dom, Bf.src, sp, P.nleaf, p1, M);
+        }));
         for (int l = P.Lmax - 1; l >= 2; --l) {
             const int64_t nb = P.lvl[(size_t)l * (S + 1) + S] - P.lvl[(size_t)l * (S + 1)];
             if (nb > 0)

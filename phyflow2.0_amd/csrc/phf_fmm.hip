@@ -78,55 +78,19 @@ __global__ void gather_tgt_f64(const double *__restrict__ x, const double *__res
 }
 
 // ---------------------------------------------------------------- P2M ----
-// One wave per leaf.  Lane j forms w_j z_j^k (k = 0..p) into an LDS table,
-// lane k then adds column k over the wave's points in index order.
-template <class T>
-__global__ __launch_bounds__(64) void p2m_kernel(const void *__restrict__ src_,
-                                                 const int32_t *__restrict__ start, int p1,
-                                                 const double4 *__restrict__ org, double s,
-                                                 int Lvl, typename C2<T>::type *__restrict__ M)
+// One wave per leaf (p2m_leaf), four leaves per workgroup.
+template <class T, int NI>
+__global__ __launch_bounds__(256) void p2m_kernel(const void *__restrict__ src,
+                                                  const int32_t *__restrict__ start,
+                                                  uint32_t nleaf, int p1,
+                                                  const double4 *__restrict__ org, double s,
+                                                  typename C2<T>::type *__restrict__ M)
 {
-    using V = typename C2<T>::type;
-    extern __shared__ unsigned char lds_raw[];
-    V *tab = reinterpret_cast<V *>(lds_raw);  // [64][p1]
-    const int lane = threadIdx.x;
-    const uint32_t b = blockIdx.x;
-    const int32_t s0 = start[b], s1 = start[b + 1];
-    V acc = cmk<T>(0, 0);
-    if (s1 > s0) {
-        double cx = 0, cy = 0;
-        if (sizeof(T) == 8) leaf_center(b, org->x, org->z, s, cx, cy);
-        const T inv_s = (T)(1.0 / s);
-        for (int32_t c0 = s0; c0 < s1; c0 += 64) {
-            const int32_t j = c0 + lane;
-            V z = cmk<T>(0, 0), g = cmk<T>(0, 0);
-            if (j < s1) {
-                if (sizeof(T) == 4) {
-                    float4 q = reinterpret_cast<const float4 *>(src_)[j];
-                    z = cmk<T>((T)q.x * inv_s, (T)q.y * inv_s);
-                    g = cmk<T>((T)q.z, 0);
-                } else {
-                    double4 q = reinterpret_cast<const double4 *>(src_)[j];
-                    z = cmk<T>((T)((q.x - cx) * (double)inv_s), (T)((q.y - cy) * (double)inv_s));
-                    g = cmk<T>((T)q.z, 0);
-                }
-            }
-            for (int k = 0; k < p1; ++k) {
-                tab[lane * p1 + k] = g;
-                g = cmul(g, z);
-            }
-            __syncthreads();
-            const int cnt = min(64, s1 - c0);
-            if (lane < p1)
-                for (int jj = 0; jj < cnt; ++jj) {
-                    V t = tab[jj * p1 + lane];
-                    acc.x += t.x;
-                    acc.y += t.y;
-                }
-            __syncthreads();
-        }
-    }
-    if (lane < p1) M[(int64_t)b * p1 + lane] = acc;
+    const uint32_t b = blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (b >= nleaf) return;
+    double cx, cy;
+    leaf_center(b, org->x, org->z, s, cx, cy);
+    p2m_leaf<T, NI>(src, start[b], start[b + 1], cx, cy, (T)(1.0 / s), p1, M + (int64_t)b * p1);
 }
 
 // ---------------------------------------------------------- M2M / L2L ----
@@ -1389,8 +1353,10 @@ static int run_fmm_typed(Lane *L, const FmmArgs &a, const Domain &dom, const Lis
         // P2M
         tm.begin(PHF_STAGE_P2M);
         used[PHF_STAGE_P2M] = true;
-        p2m_kernel<T><<<nleaf, 64, (size_t)64 * p1 * sizeof(V), L->stream>>>(
-            src, sp, p1, dom.org, dom.s, Lv, M + off[Lv] * p1);
+        PHF_TRY(p2m_dispatch(p1, [&](auto ni) {
+            p2m_kernel<T, decltype(ni)::value><<<(nleaf + 3) / 4, 256, 0, L->stream>>>(
+                src, sp, nleaf, p1, dom.org, dom.s, M + off[Lv] * p1);
+        }));
         PHF_HIP(hipGetLastError());
         tm.end(PHF_STAGE_P2M);
         // M2M up to level 2, three levels per launch

@@ -3,6 +3,9 @@
 #pragma once
 
 #include "phf_device.hpp"
+#include "phyflow_amd.h"
+
+#include <type_traits>
 
 namespace phf {
 
@@ -32,6 +35,95 @@ __device__ __forceinline__ void leaf_center(uint32_t key, double x0, double y0, 
 __device__ __forceinline__ int box_count(const int32_t *__restrict__ start, uint32_t b, int shift)
 {
     return start[(int64_t)(b + 1) << shift] - start[(int64_t)b << shift];
+}
+
+// ----------------------------------------------------------------- P2M --
+// Multipole expansion sum_j w_j ((z_j - c) inv_s)^k, k < p1 <= 4 NI, of the
+// points [s0, s1) by one wave, without LDS.  Lane 4 r + q takes the points
+// j = r (mod 16) and the powers k = q (mod 4): it forms z^q from z and z^2,
+// steps by z^4 through its NI powers and keeps their sums in registers; the
+// sixteen lanes of a power are then added by a butterfly.  Four residues of
+// k balance the products repeated in every lane of a point (2 squarings, 2
+// selected) against the butterfly (4 steps of NI).  (With a table of
+// 64 x p1 powers in LDS and each column added by one lane, a leaf was a
+// serial chain of 64 LDS reads with 64 - p1 lanes idle.)
+// Beside the near field of 1M blobs, order 13: 47 us against 70; of 120k
+// blobs, float64 order 29: 139 against 155 us (it waits for the near field's
+// workgroups there).
+// float32 records are relative to the leaf centre; (cx, cy) is the centre
+// for float64 ones.
+template <class T, int NI>
+__device__ __forceinline__ void p2m_leaf(const void *__restrict__ src, int32_t s0, int32_t s1,
+                                         double cx, double cy, T inv_s, int p1,
+                                         typename C2<T>::type *__restrict__ out)
+{
+    using V = typename C2<T>::type;
+    const int lane = threadIdx.x & 63, q = lane & 3, r = lane >> 2;
+    V acc[NI];
+#pragma unroll
+    for (int i = 0; i < NI; ++i) acc[i] = cmk<T>(0, 0);
+    // the loads of U points go out together (16 U points of the leaf)
+    constexpr int U = 4;
+    using R = std::conditional_t<sizeof(T) == 4, float4, double4>;
+    const R *rec = reinterpret_cast<const R *>(src);
+    for (int32_t j0 = s0 + r; j0 < s1; j0 += 16 * U) {
+        R pt[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int32_t j = j0 + 16 * u;
+            pt[u] = rec[j < s1 ? j : s0];
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (j0 + 16 * u >= s1) break;
+            V z;
+            if (sizeof(T) == 4)
+                z = cmk<T>((T)pt[u].x * inv_s, (T)pt[u].y * inv_s);
+            else
+                z = cmk<T>((T)((pt[u].x - cx) * inv_s), (T)((pt[u].y - cy) * inv_s));
+            V t = cmk<T>((T)pt[u].z, 0);
+            const V z2 = cmul(z, z), z4 = cmul(z2, z2);
+            if (q & 1) t = cmul(t, z);
+            if (q & 2) t = cmul(t, z2);
+#pragma unroll
+            for (int i = 0; i < NI; ++i) {
+                acc[i].x += t.x;
+                acc[i].y += t.y;
+                if (i + 1 < NI) t = cmul(t, z4);
+            }
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+#pragma unroll
+        for (int d = 4; d < 64; d <<= 1) {
+            acc[i].x += __shfl_xor(acc[i].x, d);
+            acc[i].y += __shfl_xor(acc[i].y, d);
+        }
+        const int k = 4 * i + q;
+        if (r == i && k < p1) out[k] = acc[i];
+    }
+}
+
+// f(integral constant NI) for the compiled NI that holds p1 powers
+template <class F>
+inline int p2m_dispatch(int p1, const F &f)
+{
+    if (p1 <= 12)
+        f(std::integral_constant<int, 3>());
+    else if (p1 <= 16)
+        f(std::integral_constant<int, 4>());
+    else if (p1 <= 20)
+        f(std::integral_constant<int, 5>());
+    else if (p1 <= 24)
+        f(std::integral_constant<int, 6>());
+    else if (p1 <= 32)
+        f(std::integral_constant<int, 8>());
+    else if (p1 <= 44)
+        f(std::integral_constant<int, 11>());
+    else
+        return PHF_ERR_UNSUPPORTED;
+    return PHF_OK;
 }
 
 // ------------------------------------------------------ domain choice --
