@@ -41,18 +41,17 @@ __device__ __forceinline__ void two_sum_add(float &hi, float &lo, float x)
     lo += err;
 }
 
-// float64 reciprocal: hardware estimate refined by two Newton steps.  On
-// gfx950 the estimate (v_rcp_f64) is good to 2^-24.4 relative, one step
-// leaves up to 20 ulp and two gave the correctly rounded 1/x for 4M inputs
-// spread over 2^-80 .. 2^80 (max relative error against IEEE division).
-__device__ __forceinline__ double rcp_f64(double x)
+// w / x in float64: with y0 the hardware estimate and e = 1 - x y0 its error
+// (|e| < 2^-24), w / x = w y0 (1 + e + e^2 + ...); the terms dropped are
+// below 2^-72.  On gfx950 the estimate (v_rcp_f64) is good to 2^-24.4.  Within
+// 1 ulp, as the product of w with a rounded 1 / x, and one operation fewer
+// than two Newton steps and that product.
+__device__ __forceinline__ double div_f64(double w, double x)
 {
-    double y = __builtin_amdgcn_rcp(x);
-    double e = __builtin_fma(-x, y, 1.0);
-    y = __builtin_fma(y, e, y);
-    e = __builtin_fma(-x, y, 1.0);
-    y = __builtin_fma(y, e, y);
-    return y;
+    const double y = __builtin_amdgcn_rcp(x);
+    const double e = __builtin_fma(-x, y, 1.0);
+    const double q = w * y;
+    return __builtin_fma(q, __builtin_fma(e, e, e), q);
 }
 
 __device__ __forceinline__ float rcp_f32(float x) { return __builtin_amdgcn_rcpf(x); }
@@ -150,11 +149,11 @@ __device__ __forceinline__ double fma3_f64(double a, double b, double c)
     return d;
 }
 
-__device__ __forceinline__ double expm1_neg_f64(double x)
+// x = k ln2 + r and (expm1(r)) / r of the reduced argument
+__device__ __forceinline__ double expm1_reduced_f64(double x, double &k, double &r)
 {
-    x = __builtin_fmax(x, -40.0);
-    const double k = __builtin_rint(x * 1.4426950408889634);
-    double r = __builtin_fma(-k, 0x1.62e42ff000000p-1, x);
+    k = __builtin_rint(x * 1.4426950408889634);
+    r = __builtin_fma(-k, 0x1.62e42ff000000p-1, x);
     r = __builtin_fma(-k, -0x1.718432a1b0e26p-35, r);
     // q = sum_{j=0..12} r^j / (j+1)!
     double q = 1.6059043836821613e-10;
@@ -169,9 +168,24 @@ __device__ __forceinline__ double expm1_neg_f64(double x)
     q = fma3_f64(q, r, 4.1666666666666664e-02);
     q = fma3_f64(q, r, 1.6666666666666666e-01);
     q = fma3_f64(q, r, 0.5);
-    q = fma3_f64(q, r, 1.0);
+    return fma3_f64(q, r, 1.0);
+}
+
+__device__ __forceinline__ double expm1_neg_f64(double x)
+{
+    double k, r;
+    const double q = expm1_reduced_f64(__builtin_fmax(x, -40.0), k, r);
     const double t = __builtin_amdgcn_ldexp(1.0, (int)k);
     return __builtin_fma(t, r * q, t - 1.0);
+}
+
+// exp(x) for x <= 0 in float64 by the same reduction: 2^k (1 + r q), within
+// an ulp; subnormal results and 0 below -745 come out of the final scaling.
+__device__ __forceinline__ double exp_neg_f64(double x)
+{
+    double k, r;
+    const double q = expm1_reduced_f64(__builtin_fmax(x, -800.0), k, r);
+    return __builtin_amdgcn_ldexp(__builtin_fma(r, q, 1.0), (int)k);
 }
 
 template <int KIND>
@@ -180,18 +194,18 @@ __device__ __forceinline__ double pair_f64(double dx, double dy, double w, const
     if (KIND == PAIR_GAUSS_EPS) {
         // 1 - exp(-r2/ks) as -expm1 (agrees with the subtraction to an ulp
         // of 1, without its cancellation at small r2)
-        const double r2 = __builtin_fma(dx, dx, dy * dy) + pp.eps;
-        return (w * rcp_f64(r2)) * -expm1_neg_f64(-r2 * pp.inv_ks);
+        const double r2 = __builtin_fma(dx, dx, __builtin_fma(dy, dy, pp.eps));
+        return div_f64(w, r2) * -expm1_neg_f64(-r2 * pp.inv_ks);
     } else if (KIND == PAIR_CUTOFF) {
-        const double r2 = __builtin_fma(dx, dx, dy * dy) + pp.eps;
-        return w * rcp_f64(r2);
+        const double r2 = __builtin_fma(dx, dx, __builtin_fma(dy, dy, pp.eps));
+        return div_f64(w, r2);
     } else {
         // scale (1 - e) rises through 1 exactly at r2 = c2 (scale =
         // 1/(1 - exp(-shape c2))), so the cutoff branch is a min; with
         // cutoff 0 the scale is +inf and every r2 > 0 gives 1
         const double r2 = __builtin_fma(dx, dx, dy * dy);
         const double om = __builtin_fmin(-expm1_neg_f64(-pp.inv_ks * r2) * pp.scale, 1.0);
-        const double P = (w * rcp_f64(r2)) * om;
+        const double P = div_f64(w, r2) * om;
         return r2 > 0.0 ? P : 0.0;
     }
 }

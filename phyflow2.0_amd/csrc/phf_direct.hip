@@ -20,6 +20,7 @@
 //         arithmetic in float32 (v_exp_f32, v_rcp_f32), sums in blocks of
 //         16 terms folded into a TwoSum (hi, lo) accumulator per target.
 #include "phf_ops.hpp"
+#include "phf_tree.hpp"
 
 #include <algorithm>
 #include <cmath>
@@ -193,6 +194,71 @@ __global__ __launch_bounds__(64) void direct_f64(
     }
 }
 
+// ------------------------------------- F64 kernel, targets in Morton order --
+// The smoothing factor 1 - exp(-r2/ks) costs more than the rest of a pair
+// and rounds to 1 beyond r2 = 40 ks (Gaussian) or is 1 beyond the cutoff
+// (Oseen), which a wave of scattered targets rarely agrees on.  With the
+// targets of a wave close together (perm: target t of the sorted order is
+// xt[perm[t]]) most sources are beyond it for all 64: four sources at a time
+// are tested and, when no lane is inside, their pairs skip the factor; the
+// same P either way.  The partials are in sorted target order.
+// Bound by float64 issue: 15 operations and a reciprocal estimate per pair
+// beyond it, 36 inside.  20,011 sources, 30,017 targets: 731 us for the call's
+// kernels in input order, 439 us sorted (45 us of it the sort); 40,000 x
+// 80,000: 3,829 against 1,928 us.
+template <int KIND>
+__global__ __launch_bounds__(64) void direct_f64_sorted(
+    const double *__restrict__ xb, const double *__restrict__ yb, const double *__restrict__ wb,
+    int64_t nb, const double *__restrict__ xt, const double *__restrict__ yt,
+    const int32_t *__restrict__ perm, int64_t nt, int64_t chunk_len, PairParams pp,
+    double2 *__restrict__ part)
+{
+    const int64_t t = (int64_t)blockIdx.x * kWave + threadIdx.x;
+    const int32_t o = perm[t < nt ? t : nt - 1];
+    const double tx = xt[o], ty = yt[o];
+    // a pair at distance 0 (Oseen) always takes the full form
+    const double in2 = KIND == PAIR_GAUSS_EPS ? 40.0 / pp.inv_ks : fmax(pp.c2, 1e-300);
+    const double eps = KIND == PAIR_GAUSS_EPS ? pp.eps : 0.0;
+    double au = 0.0, av = 0.0;
+    const int64_t j0 = (int64_t)blockIdx.y * chunk_len;
+    const int64_t j1 = min(nb, j0 + chunk_len);
+    int64_t j = j0;
+    for (; j + 4 <= j1; j += 4) {
+        double dx[4], dy[4], r2[4], w[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            w[k] = wb[j + k];
+            dx[k] = tx - xb[j + k];
+            dy[k] = ty - yb[j + k];
+            r2[k] = __builtin_fma(dx[k], dx[k], fma3_f64(dy[k], dy[k], eps));
+        }
+        const double least = __builtin_fmin(__builtin_fmin(r2[0], r2[1]),
+                                            __builtin_fmin(r2[2], r2[3]));
+        if (__ballot(least < in2)) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const double P = pair_f64<KIND>(dx[k], dy[k], w[k], pp);
+                au = __builtin_fma(P, dx[k], au);
+                av = __builtin_fma(P, dy[k], av);
+            }
+        } else {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const double P = div_f64(w[k], r2[k]);
+                au = __builtin_fma(P, dx[k], au);
+                av = __builtin_fma(P, dy[k], av);
+            }
+        }
+    }
+    for (; j < j1; ++j) {
+        const double dx = tx - xb[j], dy = ty - yb[j];
+        const double P = pair_f64<KIND>(dx, dy, wb[j], pp);
+        au = __builtin_fma(P, dx, au);
+        av = __builtin_fma(P, dy, av);
+    }
+    if (t < nt) part[(int64_t)blockIdx.y * nt + t] = make_double2(au, av);
+}
+
 // Adds the chunk partials and maps (A, B) = (sum P dx, sum P dy) to the
 // reference outputs:
 //   Gaussian: vx = inv_2pi * (-B), vy = inv_2pi * A  (vv2parGauss_C_cpu.c:150-151)
@@ -201,10 +267,11 @@ __global__ __launch_bounds__(64) void direct_f64(
 // A workgroup of 4 waves serves 64 targets: wave w adds the w-th quarter of
 // the chunks in chunk order (coalesced rows, eight loads in flight), and
 // the four quarter sums are added in wave order, so the result is fixed
-// for a given chunking.
+// for a given chunking.  perm (nullable): partials of target perm[t].
 constexpr int FIN_T = 64;  // targets per finishing workgroup
 __global__ __launch_bounds__(256) void direct_finish(const double2 *__restrict__ part,
                                                      int nchunk, int64_t nt, int kind,
+                                                     const int32_t *__restrict__ perm,
                                                      double *__restrict__ o0,
                                                      double *__restrict__ o1)
 {
@@ -237,13 +304,14 @@ __global__ __launch_bounds__(256) void direct_finish(const double2 *__restrict__
     if (w != 0 || t >= nt) return;
     a = ((red[0][l].x + red[1][l].x) + red[2][l].x) + red[3][l].x;
     b = ((red[0][l].y + red[1][l].y) + red[2][l].y) + red[3][l].y;
+    const int64_t o = perm ? perm[t] : t;
     if (kind == PAIR_GAUSS_EPS || kind == PAIR_CUTOFF) {
         const double inv_2pi = 0.5 / 3.141592653589793;
-        o0[t] = inv_2pi * (-b);
-        o1[t] = inv_2pi * a;
+        o0[o] = inv_2pi * (-b);
+        o1[o] = inv_2pi * a;
     } else {
-        o0[t] = -a;
-        o1[t] = b;
+        o0[o] = -a;
+        o1[o] = b;
     }
 }
 
@@ -327,7 +395,7 @@ __global__ __launch_bounds__(64) void vort_f64(const double *__restrict__ xb,
         for (int i = 0; i < TPL; ++i) {
             const double dx = tx[i] - s.x, dy = ty[i] - s.y;
             const double r2 = dx * dx + dy * dy + pp.eps;
-            a[i] += CUT ? s.w / sqrt(r2) : s.w * exp(-r2 * pp.inv_ks);
+            a[i] += CUT ? s.w / sqrt(r2) : s.w * exp_neg_f64(-r2 * pp.inv_ks);
         }
     }
     double *out = part + (int64_t)blockIdx.y * nt;
@@ -364,6 +432,193 @@ __global__ void vort_finish(const double *__restrict__ part, int nchunk, int64_t
     }
 }
 
+// ------------------------------------ vorticity of near sources only -----
+// A Gaussian term of a source at r2 > kVortCut ks is below 2^-100 |w|, so all
+// of them together are below 2^-100 W, W = sum |w|: they cannot change a sum
+// of at least 2^-46 W beyond 2^-54 of its value.  Sources and targets are
+// sorted in Morton order; a wave of 64 targets takes only the blocks of 64
+// sources whose box comes within that radius of its own, and the few targets
+// whose sum is too small for the argument (empty regions, cancellation) are
+// summed again over every source.
+// 20,011 sources, 40,401 targets in float64: the call 1,015 us with every
+// pair, 331 us this way; 100,000 x 100,000: 11.2 against 0.70 ms.
+constexpr double kVortCut = 69.4;  // exp(-69.4) < 2^-100
+constexpr int kVortBlk = 64;       // sources per block
+
+// Sorted source records of block b (padded with zero circulations at the last
+// source), their box {xmin, xmax, ymin, ymax} and sum |w|: one wave each.
+__global__ __launch_bounds__(256) void vort_pack(const double *__restrict__ xb,
+                                                 const double *__restrict__ yb,
+                                                 const double *__restrict__ wb,
+                                                 const int32_t *__restrict__ perm, int64_t nb,
+                                                 int nblk, double4 *__restrict__ rec,
+                                                 double4 *__restrict__ box,
+                                                 double *__restrict__ wabs)
+{
+    const int lane = threadIdx.x & 63;
+    const int b = (int)(blockIdx.x * 4 + (threadIdx.x >> 6));
+    if (b >= nblk) return;
+    const int64_t q = (int64_t)b * kVortBlk + lane;
+    const int32_t j = perm[q < nb ? q : nb - 1];
+    const double x = xb[j], y = yb[j], w = q < nb ? wb[j] : 0.0;
+    rec[q] = make_double4(x, y, w, 0.0);
+    double4 bx = make_double4(x, x, y, y);
+    double s = fabs(w);
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) {
+        bx.x = fmin(bx.x, __shfl_xor(bx.x, d));
+        bx.y = fmax(bx.y, __shfl_xor(bx.y, d));
+        bx.z = fmin(bx.z, __shfl_xor(bx.z, d));
+        bx.w = fmax(bx.w, __shfl_xor(bx.w, d));
+        s += __shfl_xor(s, d);
+    }
+    if (lane == 0) {
+        box[b] = bx;
+        wabs[b] = s;
+    }
+}
+
+// Partial sums of 64 sorted targets over the near blocks b = blockIdx.y (mod
+// gridDim.y), so that neighbouring blocks go to different waves.  F32: the
+// arithmetic of vort_f32c, 16 terms to a TwoSum.
+template <bool F32>
+__global__ __launch_bounds__(64) void vort_near(const double4 *__restrict__ rec,
+                                                const double4 *__restrict__ box, int nblk,
+                                                const double *__restrict__ xt,
+                                                const double *__restrict__ yt,
+                                                const int32_t *__restrict__ perm, int64_t nt,
+                                                PairParams pp, double *__restrict__ part)
+{
+    const int lane = threadIdx.x;
+    const int64_t t = (int64_t)blockIdx.x * kWave + lane;
+    const int32_t o = perm[t < nt ? t : nt - 1];
+    const double tx = xt[o], ty = yt[o];
+    double x0 = tx, x1 = tx, y0 = ty, y1 = ty;
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) {
+        x0 = fmin(x0, __shfl_xor(x0, d));
+        x1 = fmax(x1, __shfl_xor(x1, d));
+        y0 = fmin(y0, __shfl_xor(y0, d));
+        y1 = fmax(y1, __shfl_xor(y1, d));
+    }
+    const double cut2 = kVortCut / pp.inv_ks;
+    const int ny = (int)gridDim.y;
+    double a = 0.0;
+    float h = 0.f, l = 0.f;
+    for (int b0 = (int)blockIdx.y; b0 < nblk; b0 += ny * kWave) {
+        const int bl = b0 + lane * ny;
+        bool near = false;
+        if (bl < nblk) {
+            const double4 bx = box[bl];
+            const double gx = fmax(fmax(bx.x - x1, x0 - bx.y), 0.0);
+            const double gy = fmax(fmax(bx.z - y1, y0 - bx.w), 0.0);
+            near = gx * gx + gy * gy < cut2;
+        }
+        for (unsigned long long m = __ballot(near); m; m &= m - 1) {
+            const int b = b0 + (__ffsll((long long)m) - 1) * ny;  // the same in every lane
+            const double4 *rb = rec + (int64_t)__builtin_amdgcn_readfirstlane(b) * kVortBlk;
+            if (F32) {
+#pragma unroll 1
+                for (int k0 = 0; k0 < kVortBlk; k0 += 16) {
+                    float s = 0.f;
+#pragma unroll
+                    for (int k = 0; k < 16; ++k) {
+                        const double4 q = rb[k0 + k];
+                        const float dx = (float)(tx - q.x), dy = (float)(ty - q.y);
+                        const float r2 = __builtin_fmaf(dx, dx, __builtin_fmaf(dy, dy, pp.eps_f));
+                        s = __builtin_fmaf((float)q.z, exp2_f32(r2 * pp.nlog2e_ks_f), s);
+                    }
+                    two_sum_add(h, l, s);
+                }
+            } else {
+#pragma unroll 1
+                for (int k0 = 0; k0 < kVortBlk; k0 += 4) {
+                    double r2[4], w[4];
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        const double4 q = rb[k0 + k];
+                        const double dx = tx - q.x, dy = ty - q.y;
+                        w[k] = q.z;
+                        r2[k] = __builtin_fma(dx, dx, fma3_f64(dy, dy, pp.eps));
+                    }
+                    const double least = __builtin_fmin(__builtin_fmin(r2[0], r2[1]),
+                                                        __builtin_fmin(r2[2], r2[3]));
+                    if (__ballot(least < cut2)) {
+#pragma unroll
+                        for (int k = 0; k < 4; ++k)
+                            a = __builtin_fma(w[k], exp_neg_f64(-r2[k] * pp.inv_ks), a);
+                    }
+                }
+            }
+        }
+    }
+    if (t < nt) part[(int64_t)blockIdx.y * nt + t] = F32 ? (double)h + (double)l : a;
+}
+
+// The partials of sorted target t, scaled, to w[perm[t]]; targets whose sum
+// is below 2^-46 W go on the list instead.
+__global__ __launch_bounds__(256) void vort_near_finish(
+    const double *__restrict__ part, int nchunk, int64_t nt, const int32_t *__restrict__ perm,
+    const double *__restrict__ wabs, int nblk, double ks, double *__restrict__ w,
+    int32_t *__restrict__ list, uint32_t *__restrict__ count)
+{
+    __shared__ double sh[256];
+    double s = 0.0;
+    for (int b = threadIdx.x; b < nblk; b += 256) s += wabs[b];
+    sh[threadIdx.x] = s;
+    __syncthreads();
+    for (int d = 128; d > 0; d >>= 1) {
+        if ((int)threadIdx.x < d) sh[threadIdx.x] += sh[threadIdx.x + d];
+        __syncthreads();
+    }
+    const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (t >= nt) return;
+    double a = 0.0;
+    for (int c = 0; c < nchunk; ++c) a += part[(int64_t)c * nt + t];
+    const int32_t o = perm[t];
+    if (fabs(a) >= sh[0] * 0x1p-46) {
+        const double inv_pi = 1.0 / 3.141592653589793;
+        w[o] = inv_pi * a / ks;
+    } else {
+        list[atomicAdd(count, 1u)] = o;
+    }
+}
+
+// every source for the listed targets, one workgroup each
+__global__ __launch_bounds__(256) void vort_rest(const double4 *__restrict__ rec, int64_t nrec,
+                                                 const double *__restrict__ xt,
+                                                 const double *__restrict__ yt, PairParams pp,
+                                                 double ks, const int32_t *__restrict__ list,
+                                                 const uint32_t *__restrict__ count,
+                                                 double *__restrict__ w)
+{
+    __shared__ double sh[256];
+    for (uint32_t q = blockIdx.x; q < *count; q += gridDim.x) {
+        const int32_t o = list[q];
+        const double tx = xt[o], ty = yt[o];
+        double a = 0.0;
+        for (int64_t j = threadIdx.x; j < nrec; j += 256) {
+            const double4 r = rec[j];
+            const double dx = tx - r.x, dy = ty - r.y;
+            const double r2 = __builtin_fma(dx, dx, __builtin_fma(dy, dy, pp.eps));
+            a = __builtin_fma(r.z, exp_neg_f64(-r2 * pp.inv_ks), a);
+        }
+        sh[threadIdx.x] = a;
+        __syncthreads();
+        for (int d = 128; d > 0; d >>= 1) {
+            if ((int)threadIdx.x < d) sh[threadIdx.x] += sh[threadIdx.x + d];
+            __syncthreads();
+        }
+        if (threadIdx.x == 0) {
+            const double inv_pi = 1.0 / 3.141592653589793;
+            w[o] = inv_pi * sh[0] / ks;
+        }
+        __syncthreads();
+    }
+}
+
+__global__ void zero_u32(uint32_t *p) { *p = 0u; }
+
 // ------------------------------------------------------------- host ------
 int upload(Lane *L, const double *host, int64_t n, double **dev)
 {
@@ -380,6 +635,44 @@ int download(Lane *L, const double *dev, int64_t n, double *host)
     if (n > 0)
         PHF_HIP(hipMemcpyAsync(host, dev, sizeof(double) * n, hipMemcpyDeviceToHost, L->stream));
     return PHF_OK;
+}
+
+// Cell of every target on a 2^B x 2^B grid over the targets' bounding box, in
+// Morton order, and its index.
+__global__ __launch_bounds__(256) void target_cells(const double *__restrict__ xt,
+                                                    const double *__restrict__ yt, int64_t nt,
+                                                    const double4 *__restrict__ bb, int B,
+                                                    uint32_t *__restrict__ keys,
+                                                    int32_t *__restrict__ vals)
+{
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= nt) return;
+    const double4 b = *bb;
+    const double ext = fmax(b.y - b.x, b.w - b.z);
+    const double scale = ext > 0.0 ? ldexp(1.0, B) / ext : 0.0;
+    const double hi = (double)((1u << B) - 1u);
+    const double fx = fmin(fmax(floor((xt[i] - b.x) * scale), 0.0), hi);
+    const double fy = fmin(fmax(floor((yt[i] - b.z) * scale), 0.0), hi);
+    keys[i] = morton2((uint32_t)fx, (uint32_t)fy);
+    vals[i] = (int32_t)i;
+}
+
+// The points' Morton order on a grid over the box bb (device; a stable sort,
+// so a fixed order): perm[t] is the t-th point.  Cells of some 64 points (a
+// wave's targets) at most, in whole 8-bit passes of the sort.
+static int target_order(Lane *L, const double *xt, const double *yt, int64_t nt,
+                        const double4 *bb, int32_t **perm)
+{
+    uint32_t *k0, *k1, *ks;
+    int32_t *v0, *v1;
+    PHF_ALLOC(k0, L->arena, uint32_t, (size_t)nt);
+    PHF_ALLOC(k1, L->arena, uint32_t, (size_t)nt);
+    PHF_ALLOC(v0, L->arena, int32_t, (size_t)nt);
+    PHF_ALLOC(v1, L->arena, int32_t, (size_t)nt);
+    const int B = nt <= 64 * 1024 ? 4 : 8;
+    target_cells<<<div_up(nt, 256), 256, 0, L->stream>>>(xt, yt, nt, bb, B, k0, v0);
+    PHF_HIP(hipGetLastError());
+    return device_radix_sort(L, k0, v0, k1, v1, nt, 2 * B, &ks, perm);
 }
 
 // Source chunks of a direct sum over nt targets in groups of 64 * tpl:
@@ -412,14 +705,23 @@ __global__ __launch_bounds__(256) void zero_part(double2 *__restrict__ part, int
 
 constexpr int DIRECT_TPL32 = 2, DIRECT_TPL64 = 1;
 
+// Pairs from which a float64 velocity sum sorts its targets (six launches,
+// some 45 us).  Call with its kernels, unsorted against sorted: 6.4e7 pairs
+// 91 against 97 us, 1.4e8 193 against 149, 6e8 731 against 439.
+constexpr double kSortPairs = 1e8;
+// Pairs from which the vorticity takes near sources only (a dozen launches).
+// Whole calls: float64 1.1e8 pairs 257 against 222 us, 8e8 1045 against 338;
+// float32 pairs cost less, 1.4e8 192 against 215 us, 8e8 425 against 285.
+constexpr double kNearPairs64 = 1e8, kNearPairs32 = 4e8;
+
 // Enqueue the pair kernel and the finishing kernel on stream st with the
 // partial sums in part (nchunk * nt double2; nchunk, chunk_len from
-// direct_split).
+// direct_split).  perm (float64 only): the targets' Morton order.
 template <int KIND>
 static int enqueue_direct(hipStream_t st, int prec, const PairParams &pp, const double *xb,
                           const double *yb, const double *wb, int64_t nb, const double *xt,
                           const double *yt, int64_t nt, int64_t nchunk, int64_t chunk_len,
-                          double2 *part, double *o0, double *o1)
+                          double2 *part, double *o0, double *o1, const int32_t *perm = nullptr)
 {
     const int tpl = prec == PHF_PREC_F32C ? DIRECT_TPL32 : DIRECT_TPL64;
     const int64_t tblock = (int64_t)kWave * tpl;
@@ -431,6 +733,9 @@ static int enqueue_direct(hipStream_t st, int prec, const PairParams &pp, const 
         // sources read in place: every lane of a wave reads the same one
         direct_f32c<KIND, DIRECT_TPL32><<<grid, kWave, 0, st>>>(xb, yb, wb, nb, xt, yt, nt,
                                                                 chunk_len, pp, part);
+    } else if (perm) {
+        direct_f64_sorted<KIND><<<grid, kWave, 0, st>>>(xb, yb, wb, nb, xt, yt, perm, nt,
+                                                        chunk_len, pp, part);
     } else {
         direct_f64<KIND, DIRECT_TPL64><<<grid, kWave, 0, st>>>(xb, yb, wb, nb, xt, yt, nt,
                                                                chunk_len, pp, part);
@@ -438,7 +743,7 @@ static int enqueue_direct(hipStream_t st, int prec, const PairParams &pp, const 
     PHF_HIP(hipGetLastError());
     direct_finish<<<div_up(nt, FIN_T), 256, 0, st>>>(
         part, nb == 0 ? 1 : (int)nchunk, nt,
-        (KIND == PAIR_GAUSS_EPS || KIND == PAIR_CUTOFF) ? KIND : PAIR_OSEEN, o0, o1);
+        (KIND == PAIR_GAUSS_EPS || KIND == PAIR_CUTOFF) ? KIND : PAIR_OSEEN, perm, o0, o1);
     PHF_HIP(hipGetLastError());
     return PHF_OK;
 }
@@ -453,8 +758,54 @@ static int launch_direct(Lane *L, int prec, const PairParams &pp, const double *
     direct_split(nt, tpl, nb, &nchunk, &chunk_len);
     double2 *part;
     PHF_ALLOC(part, L->arena, double2, (size_t)nchunk * (size_t)nt);
+    int32_t *perm = nullptr;
+    if (prec == PHF_PREC_F64 && KIND != PAIR_CUTOFF && nt < (int64_t(1) << 31) &&
+        (double)nb * (double)nt >= kSortPairs) {
+        double4 *bb;
+        PHF_ALLOC(bb, L->arena, double4, 1);
+        PHF_TRY(device_bbox(L, xt, yt, nt, nullptr, nullptr, 0, bb));
+        PHF_TRY(target_order(L, xt, yt, nt, bb, &perm));
+    }
     return enqueue_direct<KIND>(L->stream, prec, pp, xb, yb, wb, nb, xt, yt, nt, nchunk,
-                                chunk_len, part, o0, o1);
+                                chunk_len, part, o0, o1, perm);
+}
+
+static int vorticity_near(Lane *L, int prec, double ks, const PairParams &pp, const double *xb,
+                          const double *yb, const double *wb, int64_t nb, const double *xt,
+                          const double *yt, int64_t nt, double *w)
+{
+    const int nblk = (int)div_up(nb, kVortBlk);
+    const int64_t ngroups = div_up(nt, kWave);
+    // some 8 waves per SIMD, each with at least 8 blocks to look at
+    const int nchunk = (int)std::max<int64_t>(
+        1, std::min<int64_t>((8192 + ngroups - 1) / ngroups, nblk / 8));
+    double4 *bb, *rec, *box;
+    double *wabs, *part;
+    int32_t *ps, *pt, *list;
+    uint32_t *count;
+    PHF_ALLOC(bb, L->arena, double4, 1);
+    PHF_ALLOC(rec, L->arena, double4, (size_t)nblk * kVortBlk);
+    PHF_ALLOC(box, L->arena, double4, (size_t)nblk);
+    PHF_ALLOC(wabs, L->arena, double, (size_t)nblk);
+    PHF_ALLOC(part, L->arena, double, (size_t)nchunk * (size_t)nt);
+    PHF_ALLOC(list, L->arena, int32_t, (size_t)nt);
+    PHF_ALLOC(count, L->arena, uint32_t, 1);
+    PHF_TRY(device_bbox(L, xb, yb, nb, xt, yt, nt, bb));
+    PHF_TRY(target_order(L, xb, yb, nb, bb, &ps));
+    PHF_TRY(target_order(L, xt, yt, nt, bb, &pt));
+    zero_u32<<<1, 1, 0, L->stream>>>(count);
+    vort_pack<<<div_up(nblk, 4), 256, 0, L->stream>>>(xb, yb, wb, ps, nb, nblk, rec, box, wabs);
+    const dim3 grid((unsigned)ngroups, (unsigned)nchunk);
+    if (prec == PHF_PREC_F32C)
+        vort_near<true><<<grid, kWave, 0, L->stream>>>(rec, box, nblk, xt, yt, pt, nt, pp, part);
+    else
+        vort_near<false><<<grid, kWave, 0, L->stream>>>(rec, box, nblk, xt, yt, pt, nt, pp, part);
+    vort_near_finish<<<div_up(nt, 256), 256, 0, L->stream>>>(part, nchunk, nt, pt, wabs, nblk, ks,
+                                                             w, list, count);
+    vort_rest<<<1024, 256, 0, L->stream>>>(rec, (int64_t)nblk * kVortBlk, xt, yt, pp, ks, list,
+                                           count, w);
+    PHF_HIP(hipGetLastError());
+    return PHF_OK;
 }
 
 int vorticity_device(Lane *L, int prec, double ksigmasqr, const double *xb, const double *yb,
@@ -467,6 +818,9 @@ int vorticity_device(Lane *L, int prec, double ksigmasqr, const double *xb, cons
         pp.eps = ksigmasqr;
         pp.eps_f = (float)ksigmasqr;
     }
+    if (!cutoff && nb < (int64_t(1) << 31) && nt < (int64_t(1) << 31) &&
+        (double)nb * (double)nt >= (prec == PHF_PREC_F64 ? kNearPairs64 : kNearPairs32))
+        return vorticity_near(L, prec, ksigmasqr, pp, xb, yb, wb, nb, xt, yt, nt, w);
     constexpr int TPL32 = 2, TPL64 = 1;
     const int tpl = prec == PHF_PREC_F32C ? TPL32 : TPL64;
     const int64_t tblock = (int64_t)kWave * tpl;

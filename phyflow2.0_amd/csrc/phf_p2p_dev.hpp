@@ -367,7 +367,7 @@ __device__ __forceinline__ void p2p_sweep_f64(const double4 *__restrict__ st, in
                 double om = 1.0;
                 if (__ballot(r2 < pp.c2))
                     om = __builtin_fmin(-expm1_neg_f64(-pp.inv_ks * r2) * pp.scale, 1.0);
-                P = (q.z * rcp_f64(r2)) * om;
+                P = div_f64(q.z, r2) * om;
             } else {
                 P = pair_f64<KIND>(dx, dy, q.z, pp);
             }

@@ -45,3 +45,61 @@ def test_population_control_chunks(n, O):
     w[n // 3] = np.inf
     got = PopulationControl(x, y, w, 1e-8, 1e300)
     assert np.array_equal(got[0], x[~(np.abs(w) < 1e-8)])
+
+
+def _flow_and_targets(nb, nt, seed, spread=1.0):
+    s = W.uniform_system(nb, seed=seed)
+    p = np.random.default_rng(seed + 1).random((nt, 2)) * spread
+    return s["x"], s["y"], s["w"], p[:, 0].copy(), p[:, 1].copy(), 2.0 * s["sigma"] ** 2
+
+
+@pytest.mark.parametrize("nb,nt", [(9999, 10000), (10001, 10007), (3001, 65537), (70001, 1501)])
+def test_direct_sorted_targets(nb, nt, O):
+    """Both sides of the pair count from which targets are sorted, and of the
+    second sorting pass; targets on sources and a cutoff of 0.  float64 sums of
+    nb terms in another order: nb 2^-53 relative to the terms' sizes, far less
+    in practice."""
+    x, y, w, xt, yt, ks = _flow_and_targets(nb, nt, nb)
+    m = min(nb, nt) // 2
+    xt[:m], yt[:m] = x[:m], y[:m]
+    sub = np.arange(0, nt, 7)
+    got = gauss.vv2parGauss_gpu(x, y, w, xt, yt, ks, 128)
+    ref = O.vv2par_gauss(x, y, w, xt[sub], yt[sub], ks)
+    assert O.rel_l2([g[sub] for g in got], ref) <= 1e-13
+    xopt = (1.2564312086261696770 * ks) ** 0.5
+    for cutoff in (5.0 * xopt, 0.0):
+        got = gauss.fmm2d_gpu(x, y, w, xt, yt, 35, xopt, cutoff, 0.0)
+        if cutoff == 0.0:  # the oracle divides 0 by 0 where a target is a source
+            assert np.all(np.isfinite(got))
+            sub = sub[sub >= m]
+        ref = O.direct_oseen(x, y, w, xt[sub], yt[sub], xopt, cutoff)
+        assert O.rel_l2([g[sub] for g in got], ref) <= 1e-13
+
+
+def test_direct_sorted_degenerate(O):
+    """All targets in one point or on a line: one cell, or one row of them."""
+    x, y, w, xt, yt, ks = _flow_and_targets(10007, 10007, 5)
+    for xs, ys in ((np.full(10007, 0.25), np.full(10007, 0.5)), (xt, np.full(10007, 0.5))):
+        got = gauss.vv2parGauss_gpu(x, y, w, xs, ys, ks, 128)
+        ref = O.vv2par_gauss(x, y, w, xs[:500], ys[:500], ks)
+        assert O.rel_l2([g[:500] for g in got], ref) <= 1e-13
+
+
+@pytest.mark.parametrize("prec,tol", [(F64, 1e-14), (F32C, 1e-6)])
+@pytest.mark.parametrize("nb,nt,spread", [(9999, 10000, 1.0), (10001, 10007, 1.0),
+                                          (20011, 20021, 1.0), (2003, 200003, 1.6),
+                                          (300007, 1501, 3.0)])
+def test_vorticity_near(prec, tol, nb, nt, spread, O):
+    """Both sides of the pair counts; with spread > 1 many targets lie where
+    every term is below 2^-100: each value is held to the value itself (down to
+    where float64 runs out), float32 ones to the field's size."""
+    x, y, w, xt, yt, ks = _flow_and_targets(nb, nt, nt, spread)
+    sub = np.arange(0, nt, max(1, nt // 700))
+    got = gauss.ww2parGauss_gpu(x, y, w, xt, yt, ks, 128, prec=prec)[sub]
+    ref = O.ww2par_gauss(x, y, w, xt[sub], yt[sub], ks)
+    assert O.rel_l2([got], [ref]) <= tol
+    if prec == F64:
+        # terms of both signs cancel: the bound is on the sum of their sizes,
+        # and exp's argument carries its own rounding, 2^-53 of r2 / ks <= 750
+        size = O.ww2par_gauss(x, y, np.abs(w), xt[sub], yt[sub], ks)
+        assert np.all(np.abs(got - ref) <= 750 * 2.0 ** -52 * size + 1e-300)
