@@ -48,7 +48,8 @@ def diffusion_tutty(dt, nu, h, xBlob, yBlob, wBlob, sigma, xBounds, yBounds, ove
     try:
         m = lib().phf_blobset_size(hset)
         xo, yo, wo = np.empty(m), np.empty(m), np.empty(m)
-        io, jo = np.empty(m, np.int64), np.empty(m, np.int64)
+        io = np.empty(m, np.int64) if return_indices else None
+        jo = np.empty(m, np.int64) if return_indices else None
         call("phf_blobset_copy", hset, ptr(xo), ptr(yo), ptr(wo), ptr(io), ptr(jo))
     finally:
         lib().phf_blobset_free(hset)

@@ -37,7 +37,8 @@ def Regrid(xBlob, yBlob, wBlob, sigma, overlap, xBounds, yBounds, interpKernel=0
     try:
         m = lib().phf_blobset_size(h)
         xo, yo, wo = np.empty(m), np.empty(m), np.empty(m)
-        io, jo = np.empty(m, np.int64), np.empty(m, np.int64)
+        io = np.empty(m, np.int64) if return_indices else None
+        jo = np.empty(m, np.int64) if return_indices else None
         call("phf_blobset_copy", h, ptr(xo), ptr(yo), ptr(wo), ptr(io), ptr(jo))
     finally:
         lib().phf_blobset_free(h)

@@ -22,6 +22,7 @@
 // is evaluated in float64 by every kernel that needs it, so P2P and M2L
 // agree on near/far by construction; the interaction list at level l is
 // {tau : near_{l-1}(floor((tau + parity)/2)) && !near_l(tau)}.
+#include "phf_host.hpp"
 #include "phf_batch.hpp"
 #include "phf_fmm.hpp"
 #include "phf_fmm_dev.hpp"
@@ -1273,12 +1274,8 @@ int phf_batch_get_velocity(phf_batch *b, int32_t s, double *vx, double *vy)
     std::lock_guard<std::mutex> lk(b->mu);
     const int64_t n = b->plan.sys[s].n, o = b->plan.sys[s].off;
     PHF_REQUIRE(n == 0 || (vx && vy), "output arrays are NULL");
-    if (n > 0) {
-        PHF_HIP(hipMemcpyAsync(vx, b->vx + o, sizeof(double) * n, hipMemcpyDeviceToHost, b->lane.stream));
-        PHF_HIP(hipMemcpyAsync(vy, b->vy + o, sizeof(double) * n, hipMemcpyDeviceToHost, b->lane.stream));
-    }
-    PHF_HIP(hipStreamSynchronize(b->lane.stream));
-    return PHF_OK;
+    return copy_out(&b->lane, {{vx, b->vx + o, sizeof(double) * (size_t)n},
+                               {vy, b->vy + o, sizeof(double) * (size_t)n}});
 }
 
 int phf_batch_set_remesh(phf_batch *b, const phf_batch_remesh_params *rp)
@@ -1428,14 +1425,9 @@ int phf_batch_get_remeshed(phf_batch *b, int32_t s, int64_t *m, double *x, doubl
     }
     const int64_t o = b->mo[2 * s];
     PHF_HIP(hipSetDevice(Context::get().device()));
-    PHF_HIP(hipMemcpyAsync(x, b->rbuf.xo + o, sizeof(double) * cnt, hipMemcpyDeviceToHost,
-                           b->lane.stream));
-    PHF_HIP(hipMemcpyAsync(y, b->rbuf.yo + o, sizeof(double) * cnt, hipMemcpyDeviceToHost,
-                           b->lane.stream));
-    PHF_HIP(hipMemcpyAsync(w, b->rbuf.wo + o, sizeof(double) * cnt, hipMemcpyDeviceToHost,
-                           b->lane.stream));
-    PHF_HIP(hipStreamSynchronize(b->lane.stream));
-    return PHF_OK;
+    const size_t nb = sizeof(double) * (size_t)cnt;
+    return copy_out(&b->lane, {{x, b->rbuf.xo + o, nb}, {y, b->rbuf.yo + o, nb},
+                               {w, b->rbuf.wo + o, nb}});
 }
 
 }  // extern "C"

@@ -258,22 +258,6 @@ void get_stage_times(double *ms_out)
 bool timing_enabled() { return g_timing; }
 void set_timing(bool on) { g_timing = on; }
 
-// ------------------------------------------------------------ validation --
-int check_host_array(const double *p, int64_t n, const char *name, bool finite)
-{
-    if (n > 0 && p == nullptr) {
-        set_error("%s is NULL but has %lld entries", name, (long long)n);
-        return PHF_ERR_INVALID;
-    }
-    if (finite)
-        for (int64_t i = 0; i < n; ++i)
-            if (!std::isfinite(p[i])) {
-                set_error("%s[%lld] is not finite", name, (long long)i);
-                return PHF_ERR_INVALID;
-            }
-    return PHF_OK;
-}
-
 }  // namespace phf
 
 // ------------------------------------------------------------- C entry ---

@@ -19,6 +19,7 @@
 //   F32C: coordinates differenced in float64 and rounded once, pair
 //         arithmetic in float32 (v_exp_f32, v_rcp_f32), sums in blocks of
 //         16 terms folded into a TwoSum (hi, lo) accumulator per target.
+#include "phf_host.hpp"
 #include "phf_ops.hpp"
 #include "phf_tree.hpp"
 
@@ -922,13 +923,9 @@ static int vv2par_entry(int kind, const double *xb, const double *yb, const doub
     tm.begin(PHF_STAGE_TOTAL);
     tm.begin(PHF_STAGE_UPLOAD);
     double *dxb, *dyb, *dwb, *dxt, *dyt, *o0, *o1;
-    PHF_TRY(upload(L, xb, nb, &dxb));
-    PHF_TRY(upload(L, yb, nb, &dyb));
-    PHF_TRY(upload(L, wb, nb, &dwb));
-    PHF_TRY(upload(L, xt, nt, &dxt));
-    PHF_TRY(upload(L, yt, nt, &dyt));
-    PHF_ALLOC(o0, L->arena, double, (size_t)nt);
-    PHF_ALLOC(o1, L->arena, double, (size_t)nt);
+    PHF_TRY(copy_points_in(L, xb, yb, wb, nb, xt, yt, nt, &dxb, &dyb, &dwb, &dxt, &dyt));
+    PHF_ALLOC(o0, L->arena, double, (size_t)nt * 2);
+    o1 = o0 + nt;
     tm.end(PHF_STAGE_UPLOAD);
     tm.begin(PHF_STAGE_P2P);
     PairParams pp = make_gauss_params(ksigmasqr);
@@ -939,11 +936,10 @@ static int vv2par_entry(int kind, const double *xb, const double *yb, const doub
     PHF_TRY(direct_device(L, kind, prec, pp, dxb, dyb, dwb, nb, dxt, dyt, nt, o0, o1));
     tm.end(PHF_STAGE_P2P);
     tm.begin(PHF_STAGE_DOWNLOAD);
-    PHF_TRY(download(L, o0, nt, vx));
-    PHF_TRY(download(L, o1, nt, vy));
+    PHF_TRY(copy_out(L, {{vx, o0, sizeof(double) * nt}, {vy, o1, sizeof(double) * nt}}));
     tm.end(PHF_STAGE_DOWNLOAD);
     tm.end(PHF_STAGE_TOTAL);
-    PHF_HIP(hipStreamSynchronize(L->stream));
+    if (tm.on) PHF_HIP(hipStreamSynchronize(L->stream));
     record_stage_times(L, used);
     return PHF_OK;
 }
@@ -989,16 +985,10 @@ static int ww2par_entry(bool cutoff, const double *xb, const double *yb, const d
     Lane *L = g.lane;
     PHF_TRY(reset_arena(L));
     double *dxb, *dyb, *dwb, *dxt, *dyt, *o;
-    PHF_TRY(upload(L, xb, nb, &dxb));
-    PHF_TRY(upload(L, yb, nb, &dyb));
-    PHF_TRY(upload(L, wb, nb, &dwb));
-    PHF_TRY(upload(L, xt, nt, &dxt));
-    PHF_TRY(upload(L, yt, nt, &dyt));
+    PHF_TRY(copy_points_in(L, xb, yb, wb, nb, xt, yt, nt, &dxb, &dyb, &dwb, &dxt, &dyt));
     PHF_ALLOC(o, L->arena, double, (size_t)nt);
     PHF_TRY(vorticity_device(L, prec, ksigmasqr, dxb, dyb, dwb, nb, dxt, dyt, nt, o, cutoff));
-    PHF_TRY(download(L, o, nt, w));
-    PHF_HIP(hipStreamSynchronize(L->stream));
-    return PHF_OK;
+    return copy_out(L, {{w, o, sizeof(double) * nt}});
 }
 
 // ------------------------------------------- allocation-free direct sum ---

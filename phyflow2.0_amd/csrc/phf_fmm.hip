@@ -31,6 +31,7 @@
 // per-target sums, P2M/M2L/L2P in float32, and M2M/L2L in float64 when the
 // order exceeds 16.
 #include "phf_fmm.hpp"
+#include "phf_host.hpp"
 #include "phf_fmm_dev.hpp"
 #include "phf_p2p_dev.hpp"
 
@@ -1849,18 +1850,9 @@ extern "C" int phf_fmm2d(const double *xb, const double *yb, const double *wb, i
     tm.begin(PHF_STAGE_TOTAL);
     tm.begin(PHF_STAGE_UPLOAD);
     double *dxb, *dyb, *dwb, *dxt, *dyt, *dqr, *dqi;
-    PHF_TRY(upload(L, xb, nb, &dxb));
-    PHF_TRY(upload(L, yb, nb, &dyb));
-    PHF_TRY(upload(L, wb, nb, &dwb));
-    if (same) {
-        dxt = dxb;
-        dyt = dyb;
-    } else {
-        PHF_TRY(upload(L, xt, nt, &dxt));
-        PHF_TRY(upload(L, yt, nt, &dyt));
-    }
-    PHF_ALLOC(dqr, L->arena, double, (size_t)nt);
-    PHF_ALLOC(dqi, L->arena, double, (size_t)nt);
+    PHF_TRY(copy_points_in(L, xb, yb, wb, nb, xt, yt, nt, &dxb, &dyb, &dwb, &dxt, &dyt));
+    PHF_ALLOC(dqr, L->arena, double, (size_t)nt * 2);
+    dqi = dqr + nt;
     tm.end(PHF_STAGE_UPLOAD);
     if (tol == 0.0) {
         // direct sum over all pairs (direct.cpp:1409-1450)
@@ -1884,11 +1876,10 @@ extern "C" int phf_fmm2d(const double *xb, const double *yb, const double *wb, i
         PHF_TRY(fmm_device(L, a, tm, used, nullptr));
     }
     tm.begin(PHF_STAGE_DOWNLOAD);
-    PHF_TRY(download(L, dqr, nt, qr));
-    PHF_TRY(download(L, dqi, nt, qi));
+    PHF_TRY(copy_out(L, {{qr, dqr, sizeof(double) * nt}, {qi, dqi, sizeof(double) * nt}}));
     tm.end(PHF_STAGE_DOWNLOAD);
     tm.end(PHF_STAGE_TOTAL);
-    PHF_HIP(hipStreamSynchronize(L->stream));
+    if (tm.on) PHF_HIP(hipStreamSynchronize(L->stream));
     record_stage_times(L, used);
     return PHF_OK;
 }

@@ -36,12 +36,14 @@
 // formulas; the cube |u|^3 is formed in double-double and rounded once (the
 // correctly rounded pow(|u|, 3.0) of the reference).
 #include "phf_remesh.hpp"
+#include "phf_host.hpp"
 #include "phf_m4_dev.hpp"
 
 #include <algorithm>
 #include <climits>
 #include <cmath>
 #include <cstring>
+#include <memory>
 #include <vector>
 
 namespace phf {
@@ -363,7 +365,7 @@ __global__ __launch_bounds__(RM_THREADS) void gather_cells(
     const int32_t *__restrict__ start, const double *__restrict__ V, int64_t n,
     const uint32_t *__restrict__ slot, RmGeom *__restrict__ g, double h, double x0, double y0,
     double *__restrict__ xo, double *__restrict__ yo, double *__restrict__ wo,
-    int64_t *__restrict__ io, int64_t *__restrict__ jo)
+    uint32_t *__restrict__ co)
 {
     if (!g->ok) return;
     const int64_t ncell = g->ncell;
@@ -381,10 +383,12 @@ __global__ __launch_bounds__(RM_THREADS) void gather_cells(
         base_starts(start, i, j, bi, bj, st, rowok);
         const long long I = i + imin, J = j + jmin;  // absolute cell indices
         wo[o] = cell_sum_dense(st, rowok, j, bj, V, n);
+        if (co) {  // the host forms the coordinates from the cell
+            co[o] = (uint32_t)cidx;
+            continue;
+        }
         xo[o] = ((double)I * h + hh) + x0;
         yo[o] = ((double)J * h + hh) + y0;
-        if (io) io[o] = I;
-        if (jo) jo[o] = J;
     }
 }
 
@@ -626,7 +630,7 @@ static int remesh_sparse(Lane *L, const double *x, const double *y, const double
     PHF_ALLOC(xo, L->arena, double, mm);
     PHF_ALLOC(yo, L->arena, double, mm);
     PHF_ALLOC(wo, L->arena, double, mm);
-    if (out->want_indices) {
+    if (out->want_cells) {
         PHF_ALLOC(io, L->arena, int64_t, mm);
         PHF_ALLOC(jo, L->arena, int64_t, mm);
     }
@@ -688,14 +692,15 @@ int remesh_device(Lane *L, const double *x, const double *y, const double *w, in
     // outputs sized for the most cells n blobs can touch
     const size_t cap = (size_t)std::min<int64_t>(16 * n, ccap);
     double *V, *xo, *yo, *wo;
-    int64_t *io = nullptr, *jo = nullptr;
+    uint32_t *co = nullptr;
     PHF_ALLOC(V, L->arena, double, 16 * nn);
-    PHF_ALLOC(xo, L->arena, double, cap);
-    PHF_ALLOC(yo, L->arena, double, cap);
     PHF_ALLOC(wo, L->arena, double, cap);
-    if (out->want_indices) {
-        PHF_ALLOC(io, L->arena, int64_t, cap);
-        PHF_ALLOC(jo, L->arena, int64_t, cap);
+    if (out->want_cells) {
+        PHF_ALLOC(co, L->arena, uint32_t, cap);
+        xo = yo = nullptr;
+    } else {
+        PHF_ALLOC(xo, L->arena, double, cap);
+        PHF_ALLOC(yo, L->arena, double, cap);
     }
     RmGeom hg;
     for (int radix = 0; radix < 2; ++radix) {
@@ -725,7 +730,7 @@ int remesh_device(Lane *L, const double *x, const double *y, const double *w, in
         PHF_TRY(device_exclusive_scan_ws(L, flag, ccap + 1, slot, sums, &g->nscan));
         // 5. sums
         gather_cells<<<RM_GRID, RM_THREADS, 0, L->stream>>>(start, V, n, slot, g, h, x0, y0, xo,
-                                                            yo, wo, io, jo);
+                                                            yo, wo, co);
         PHF_HIP(hipGetLastError());
         // the one synchronisation: the layout with the output count, and what
         // the caller asked to read back
@@ -748,8 +753,10 @@ int remesh_device(Lane *L, const double *x, const double *y, const double *w, in
     out->x = xo;
     out->y = yo;
     out->w = wo;
-    out->i = io;
-    out->j = jo;
+    out->cell = co;
+    out->imin = hg.imin;
+    out->jmin = hg.jmin;
+    out->nj = hg.nj;
     out->cells = hg.ncell;
     return PHF_OK;
 }
@@ -1034,10 +1041,18 @@ int population_control_device(Lane *L, const double *x, const double *y, const d
 // ------------------------------------------------------------ C entry ----
 using namespace phf;
 
+// A remesh keeps each blob's weight and its cell, c = (i - imin) nj + (j -
+// jmin) in ascending order, in place of coordinates and indices that follow
+// from it; phf_blobset_copy forms them in the caller's arrays by the kernel's
+// own expressions.  Population control, and a range too wide for 32-bit cells,
+// keep the arrays themselves.
 struct phf_blobset_s {
     int64_t m = 0;
-    std::vector<double> x, y, w;
-    std::vector<int64_t> i, j;
+    std::unique_ptr<double[]> x, y, w;
+    std::unique_ptr<int64_t[]> i, j;
+    std::unique_ptr<uint32_t[]> cell;
+    long long imin = 0, jmin = 0, nj = 1;
+    double h = 0.0, x0 = 0.0, y0 = 0.0;
 };
 
 extern "C" {
@@ -1115,31 +1130,35 @@ static int regrid_entry(int kind, const double *x, const double *y, const double
         used[PHF_STAGE_REMESH] = used[PHF_STAGE_TOTAL] = true;
         tm.begin(PHF_STAGE_TOTAL);
         double *dx, *dy, *dw;
-        PHF_TRY(upload(L, x, n, &dx));
-        PHF_TRY(upload(L, y, n, &dy));
-        PHF_TRY(upload(L, w, n, &dw));
+        PHF_TRY(copy_in(L, {{x, n, &dx}, {y, n, &dy}, {w, n, &dw}}));
         tm.begin(PHF_STAGE_REMESH);
         RemeshOut ro;
-        ro.want_indices = true;
+        ro.want_cells = true;
         PHF_TRY(remesh_device(L, dx, dy, dw, n, sigma, overlap, x0, y0, c, &ro, kind));
         tm.end(PHF_STAGE_REMESH);
+        const size_t m = (size_t)ro.m;
         res->m = ro.m;
-        res->x.resize(ro.m);
-        res->y.resize(ro.m);
-        res->w.resize(ro.m);
-        res->i.resize(ro.m);
-        res->j.resize(ro.m);
-        if (ro.m > 0) {
-            PHF_TRY(download(L, ro.x, ro.m, res->x.data()));
-            PHF_TRY(download(L, ro.y, ro.m, res->y.data()));
-            PHF_TRY(download(L, ro.w, ro.m, res->w.data()));
-            PHF_HIP(hipMemcpyAsync(res->i.data(), ro.i, sizeof(int64_t) * ro.m,
-                                   hipMemcpyDeviceToHost, L->stream));
-            PHF_HIP(hipMemcpyAsync(res->j.data(), ro.j, sizeof(int64_t) * ro.m,
-                                   hipMemcpyDeviceToHost, L->stream));
+        res->w.reset(new double[m]);
+        if (ro.sparse) {
+            res->x.reset(new double[m]);
+            res->y.reset(new double[m]);
+            res->i.reset(new int64_t[m]);
+            res->j.reset(new int64_t[m]);
+            PHF_TRY(copy_out(L, {{res->x.get(), ro.x, 8 * m}, {res->y.get(), ro.y, 8 * m},
+                                 {res->w.get(), ro.w, 8 * m}, {res->i.get(), ro.i, 8 * m},
+                                 {res->j.get(), ro.j, 8 * m}}));
+        } else {
+            res->cell.reset(new uint32_t[m]);
+            res->imin = ro.imin;
+            res->jmin = ro.jmin;
+            res->nj = ro.nj;
+            res->h = sigma * overlap;
+            res->x0 = x0;
+            res->y0 = y0;
+            PHF_TRY(copy_out(L, {{res->w.get(), ro.w, 8 * m}, {res->cell.get(), ro.cell, 4 * m}}));
         }
         tm.end(PHF_STAGE_TOTAL);
-        PHF_HIP(hipStreamSynchronize(L->stream));
+        if (tm.on) PHF_HIP(hipStreamSynchronize(L->stream));
         record_stage_times(L, used);
         return PHF_OK;
     }();
@@ -1159,11 +1178,30 @@ int phf_blobset_copy(const phf_blobset *b, double *x, double *y, double *w, int6
     clear_error();
     PHF_REQUIRE(b != nullptr, "blob set is NULL");
     if (b->m == 0) return PHF_OK;
-    if (x) std::memcpy(x, b->x.data(), sizeof(double) * b->m);
-    if (y) std::memcpy(y, b->y.data(), sizeof(double) * b->m);
-    if (w) std::memcpy(w, b->w.data(), sizeof(double) * b->m);
-    if (i && !b->i.empty()) std::memcpy(i, b->i.data(), sizeof(int64_t) * b->m);
-    if (j && !b->j.empty()) std::memcpy(j, b->j.data(), sizeof(int64_t) * b->m);
+    constexpr int64_t kPart = 1 << 14;
+    host_parallel((int)((b->m + kPart - 1) / kPart), [&](int part) {
+        const int64_t lo = (int64_t)part * kPart, hi = std::min(b->m, lo + kPart);
+        if (w) std::memcpy(w + lo, b->w.get() + lo, sizeof(double) * (size_t)(hi - lo));
+        if (!b->cell) {
+            const size_t nb = sizeof(double) * (size_t)(hi - lo);
+            if (x) std::memcpy(x + lo, b->x.get() + lo, nb);
+            if (y) std::memcpy(y + lo, b->y.get() + lo, nb);
+            if (i && b->i) std::memcpy(i + lo, b->i.get() + lo, nb);
+            if (j && b->j) std::memcpy(j + lo, b->j.get() + lo, nb);
+            return;
+        }
+        const double h = b->h, hh = 0.5 * h, x0 = b->x0, y0 = b->y0;
+        long long row = (long long)b->cell[lo] / b->nj;
+        for (int64_t k = lo; k < hi; ++k) {
+            const long long c = (long long)b->cell[k];
+            while (c >= (row + 1) * b->nj) ++row;
+            const long long I = b->imin + row, J = b->jmin + (c - row * b->nj);
+            if (x) x[k] = ((double)I * h + hh) + x0;
+            if (y) y[k] = ((double)J * h + hh) + y0;
+            if (i) i[k] = I;
+            if (j) j[k] = J;
+        }
+    });
     return PHF_OK;
 }
 
@@ -1195,9 +1233,7 @@ int phf_population_control(const double *x, const double *y, const double *w, in
     int rc = [&]() -> int {
         PHF_TRY(reset_arena(L));
         double *dx, *dy, *dw, *xo, *yo, *wo;
-        PHF_TRY(upload(L, x, n, &dx));
-        PHF_TRY(upload(L, y, n, &dy));
-        PHF_TRY(upload(L, w, n, &dw));
+        PHF_TRY(copy_in(L, {{x, n, &dx}, {y, n, &dy}, {w, n, &dw}}));
         PHF_ALLOC(xo, L->arena, double, (size_t)n);
         PHF_ALLOC(yo, L->arena, double, (size_t)n);
         PHF_ALLOC(wo, L->arena, double, (size_t)n);
@@ -1205,16 +1241,11 @@ int phf_population_control(const double *x, const double *y, const double *w, in
         PHF_TRY(population_control_device(L, dx, dy, dw, n, wThreshold, wTotalThreshold, xo, yo,
                                           wo, &m, nullptr));
         res->m = m;
-        res->x.resize(m);
-        res->y.resize(m);
-        res->w.resize(m);
-        if (m > 0) {
-            PHF_TRY(download(L, xo, m, res->x.data()));
-            PHF_TRY(download(L, yo, m, res->y.data()));
-            PHF_TRY(download(L, wo, m, res->w.data()));
-        }
-        PHF_HIP(hipStreamSynchronize(L->stream));
-        return PHF_OK;
+        res->x.reset(new double[(size_t)m]);
+        res->y.reset(new double[(size_t)m]);
+        res->w.reset(new double[(size_t)m]);
+        const size_t b = sizeof(double) * (size_t)m;
+        return copy_out(L, {{res->x.get(), xo, b}, {res->y.get(), yo, b}, {res->w.get(), wo, b}});
     }();
     if (rc != PHF_OK) {
         delete res;

@@ -6,7 +6,9 @@
 namespace phf {
 
 struct RemeshOut {
-    bool want_indices = false;  // input: also return the cell indices
+    // input: the weights and cells only (cell; x, y stay null), or, on the
+    // sparse path, everything and the cell indices (i, j)
+    bool want_cells = false;
     // input: device bytes read back to the host with the output count
     const void *read_src = nullptr;
     size_t read_bytes = 0;
@@ -15,6 +17,9 @@ struct RemeshOut {
     int64_t m = 0;
     double *x = nullptr, *y = nullptr, *w = nullptr;
     int64_t *i = nullptr, *j = nullptr;
+    // cell (i - imin) nj + (j - jmin) of every output, ascending
+    uint32_t *cell = nullptr;
+    long long imin = 0, jmin = 0, nj = 1;
     int64_t cells = 0;    // cells scanned (dense touched range, or the sparse list)
     bool sparse = false;  // the range was too large for the dense layout
 };

@@ -14,6 +14,7 @@
 // second-order scheme, x1 = x0 + dt k(x0), x = x0 + dt/2 (k(x0) + k(x1)),
 // with every stage evaluated at its own positions (the reference RK4 reuses
 // aliased positions, a defect not reproduced here).
+#include "phf_host.hpp"
 #include "phf_panel.hpp"
 #include "phf_remesh.hpp"
 #include "phf_system.hpp"
@@ -513,12 +514,9 @@ int phf_panels_solve(phf_panels *P, const double *vx, const double *vy, double *
     Lane *L = g.lane;
     PHF_TRY(reset_arena(L));
     double *dvx, *dvy;
-    PHF_TRY(upload(L, vx, P->m, &dvx));
-    PHF_TRY(upload(L, vy, P->m, &dvy));
+    PHF_TRY(copy_in(L, {{vx, P->m, &dvx}, {vy, P->m, &dvy}}));
     PHF_TRY(panels_solve_device(L, P, dvx, dvy, 0.0, 0.0));
-    PHF_HIP(hipMemcpyAsync(strength, P->s, sizeof(double) * P->m, hipMemcpyDeviceToHost,
-                           L->stream));
-    PHF_HIP(hipStreamSynchronize(L->stream));
+    PHF_TRY(copy_out(L, {{strength, P->s, sizeof(double) * P->m}}));
     if (iterations) *iterations = P->last_iterations;
     return PHF_OK;
 }

@@ -1,6 +1,7 @@
 // phf_system.cpp -- device-resident blob systems (one stream + workspace
 // each), velocity evaluation on resident data.
 #include "phf_system.hpp"
+#include "phf_host.hpp"
 
 #include <cmath>
 #include <mutex>
@@ -193,13 +194,8 @@ int phf_system_get(phf_system *h, double *x, double *y, double *w)
     PHF_REQUIRE(h != nullptr, "system is NULL");
     System *s = reinterpret_cast<System *>(h);
     std::lock_guard<std::mutex> lk(s->mu);
-    if (s->n > 0) {
-        if (x) PHF_HIP(hipMemcpyAsync(x, s->x, sizeof(double) * s->n, hipMemcpyDeviceToHost, s->lane.stream));
-        if (y) PHF_HIP(hipMemcpyAsync(y, s->y, sizeof(double) * s->n, hipMemcpyDeviceToHost, s->lane.stream));
-        if (w) PHF_HIP(hipMemcpyAsync(w, s->w, sizeof(double) * s->n, hipMemcpyDeviceToHost, s->lane.stream));
-    }
-    PHF_HIP(hipStreamSynchronize(s->lane.stream));
-    return PHF_OK;
+    const size_t b = sizeof(double) * (size_t)s->n;
+    return copy_out(&s->lane, {{x, s->x, x ? b : 0}, {y, s->y, y ? b : 0}, {w, s->w, w ? b : 0}});
 }
 
 int phf_system_set(phf_system *h, const double *x, const double *y, const double *w, int64_t n)
@@ -251,10 +247,8 @@ int phf_system_velocity(phf_system *h, const phf_vel_params *p, double *vx, doub
         if (vx && vy && s->n > 0) {
             tm.begin(PHF_STAGE_DOWNLOAD);
             used[PHF_STAGE_DOWNLOAD] = true;
-            PHF_HIP(hipMemcpyAsync(vx, s->vx, sizeof(double) * s->n, hipMemcpyDeviceToHost,
-                                   L->stream));
-            PHF_HIP(hipMemcpyAsync(vy, s->vy, sizeof(double) * s->n, hipMemcpyDeviceToHost,
-                                   L->stream));
+            PHF_TRY(copy_out(L, {{vx, s->vx, sizeof(double) * s->n},
+                                 {vy, s->vy, sizeof(double) * s->n}}));
             tm.end(PHF_STAGE_DOWNLOAD);
         }
         tm.end(PHF_STAGE_TOTAL);
@@ -297,12 +291,8 @@ int phf_system_get_velocity(phf_system *h, double *vx, double *vy)
         set_error("no velocity has been evaluated for this system");
         return PHF_ERR_INVALID;
     }
-    if (s->n > 0) {
-        PHF_HIP(hipMemcpyAsync(vx, s->vx, sizeof(double) * s->n, hipMemcpyDeviceToHost, s->lane.stream));
-        PHF_HIP(hipMemcpyAsync(vy, s->vy, sizeof(double) * s->n, hipMemcpyDeviceToHost, s->lane.stream));
-    }
-    PHF_HIP(hipStreamSynchronize(s->lane.stream));
-    return PHF_OK;
+    return copy_out(&s->lane, {{vx, s->vx, sizeof(double) * (size_t)s->n},
+                               {vy, s->vy, sizeof(double) * (size_t)s->n}});
 }
 
 }  // extern "C"

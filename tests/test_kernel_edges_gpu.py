@@ -103,3 +103,44 @@ def test_vorticity_near(prec, tol, nb, nt, spread, O):
         # and exp's argument carries its own rounding, 2^-53 of r2 / ks <= 750
         size = O.ww2par_gauss(x, y, np.abs(w), xt[sub], yt[sub], ks)
         assert np.all(np.abs(got - ref) <= 750 * 2.0 ** -52 * size + 1e-300)
+
+
+@pytest.mark.parametrize("n", [1, 5461, 5462, 87381, 87382, 131072, 131073, 800001])
+def test_blobs_come_back_whole(n):
+    """Results by one packed transfer, by the runtime's copies and through the
+    pinned slots (24 n bytes: 128 KiB, 2 MiB, whole and odd slots, more slots
+    than a ring has), from several threads at once."""
+    import threading
+    from phyflow_amd.system import BlobSystem
+    rng = np.random.default_rng(n)
+    data = [tuple(rng.random(n) for _ in range(3)) for _ in range(3)]
+    systems = [BlobSystem(*d) for d in data]
+    wrong = []
+
+    def check(k):
+        for _ in range(3):
+            for a, b in zip(systems[k].get(), data[k]):
+                if not np.array_equal(a, b):
+                    wrong.append(k)
+
+    threads = [threading.Thread(target=check, args=(k,)) for k in range(3)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong
+
+
+@pytest.mark.parametrize("n", [1, 7, 65536, 65537, 300001])
+@pytest.mark.parametrize("bad", [np.nan, np.inf, -np.inf])
+def test_not_finite_is_refused_anywhere(n, bad):
+    from phyflow_amd._native import PhfError
+    from phyflow_amd.system import BlobSystem
+    x = np.zeros(n)
+    x[:4] = [5e-324, 1.7976931348623157e308, -0.0, 1.0][:min(4, n)]
+    BlobSystem(x, x, x).close()
+    for at in {0, n // 2, n - 1, min(n - 1, 65535), min(n - 1, 65536)}:
+        y = x.copy()
+        y[at] = bad
+        with pytest.raises(PhfError, match=r"y\[%d\] is not finite" % at):
+            BlobSystem(x, y, x)
