@@ -123,6 +123,7 @@ struct Pinned {
 
 // ---------------------------------------------------------------- lanes --
 struct FmmGraphCache;
+struct FmmPlanCache;
 
 struct Lane {
     hipStream_t stream = nullptr;
@@ -136,6 +137,7 @@ struct Lane {
     // second stream (default priority) the FMM near field runs on while the
     // far field runs on `stream`, with the events that fork and join them
     FmmGraphCache *fmm_graphs = nullptr;
+    FmmPlanCache *fmm_plans = nullptr;  // tables of the tree shapes last used
     hipStream_t stream2 = nullptr;
     hipEvent_t fork_ev = nullptr, join_ev = nullptr;
     // start, end of convection, end of a time step (its stage times)

@@ -40,6 +40,7 @@
 #include <complex>
 #include <cstring>
 #include <functional>
+#include <memory>
 #include <vector>
 
 namespace phf {
@@ -901,40 +902,36 @@ Domain choose_domain(const double4 &hb, int L, double nb, double nt, double cuto
     }
 }
 
-// All small host tables of one call are packed into the lane's pinned
-// staging buffer and sent with a single asynchronous copy; the buffer is
-// owned by the call until its final stream synchronisation.
+// The small host tables of a plan, packed into the lane's pinned staging
+// buffer and sent with a single copy.
 struct TableBlob {
     std::vector<char> host;
     std::vector<std::pair<size_t, void **>> fix;
-    template <class T, class Dev>
-    void add(const std::vector<T> &v, Dev **d)
+    template <class T>
+    void add(const std::vector<T> &v, void **d)
     {
         size_t at = (host.size() + 255) & ~size_t(255);
         host.resize(at + std::max<size_t>(sizeof(T) * v.size(), 1));
         if (!v.empty()) std::memcpy(host.data() + at, v.data(), sizeof(T) * v.size());
-        fix.push_back({at, reinterpret_cast<void **>(d)});
+        fix.push_back({at, d});
     }
-    // keep != nullptr (launches being recorded into a graph): the tables
-    // go once to a device buffer of their own handed to *keep, copied on
-    // the side stream (not recorded) and waited for, so the graph holds no
-    // copy (the tables depend only on what keys the graph)
-    int send(Lane *L, char **keep = nullptr, hipStream_t side = nullptr)
+    // To a device buffer of their own, handed to *keep, copied on stream st;
+    // wait: the copy is complete on return (launches being recorded into a
+    // graph then hold no copy), else it is ordered on st.
+    int send(Lane *L, char **keep, hipStream_t st, bool wait)
     {
         if (host.empty()) return PHF_OK;
         char *dev;
-        if (keep) {
-            PHF_HIP(hipMalloc(&dev, host.size()));
-            *keep = dev;
-            PHF_HIP(hipMemcpyAsync(dev, host.data(), host.size(), hipMemcpyHostToDevice, side));
-            PHF_HIP(hipStreamSynchronize(side));
+        PHF_HIP(hipMalloc(&dev, host.size()));
+        *keep = dev;
+        if (wait) {
+            PHF_HIP(hipMemcpyAsync(dev, host.data(), host.size(), hipMemcpyHostToDevice, st));
+            PHF_HIP(hipStreamSynchronize(st));
         } else {
             PHF_TRY(L->pin.ensure(host.size()));
             std::memcpy(L->pin.ptr, host.data(), host.size());
-            PHF_ALLOC(dev, L->arena, char, host.size());
-            PHF_HIP(hipMemcpyAsync(dev, L->pin.ptr, host.size(), hipMemcpyHostToDevice,
-                                   L->stream));
-            PHF_TRY(L->pin.mark(L->stream));
+            PHF_HIP(hipMemcpyAsync(dev, L->pin.ptr, host.size(), hipMemcpyHostToDevice, st));
+            PHF_TRY(L->pin.mark(st));
         }
         for (auto &f : fix) *f.second = dev + f.first;
         return PHF_OK;
@@ -1079,10 +1076,13 @@ using P2PLaunch = std::function<int(hipStream_t)>;
 // the near field (fmm_far_fork / fmm_far_done / fmm_far_join), so that the
 // near field follows the tree on the lane's stream with no cross-stream
 // wait in between.  An empty near launch runs everything in order.
+struct FmmPlan;
 struct FmmSplit {
+    ~FmmSplit();
     std::function<int()> mid;
     P2PLaunch near, finish;
     char **tables_keep = nullptr;  // device tables kept for replays
+    std::unique_ptr<FmmPlan> plan;  // and their layout, while recording
     hipStream_t side = nullptr;    // their upload stream while recording
 };
 
@@ -1126,10 +1126,174 @@ static int fmm_near(Lane *L, const P2PLaunch &near, StageTimer &tm)
     return rc;
 }
 
+// Tables of one tree shape on the device: near list, interaction lists,
+// binomials and powers.  They depend on the order, the precision, the leaf
+// level and which box offsets are near at each level (key), not on the points
+// or the domain's place and size.  A lane keeps the last kPlans it used, so a
+// time step or a call with new points of a like spread neither builds nor
+// sends them again (45 us less between the bounding box and the near field of
+// 120k blobs).
+struct FmmPlan {
+    std::vector<uint8_t> key;
+    char *dev = nullptr;
+    void *near = nullptr, *pas = nullptr, *bin = nullptr, *U = nullptr, *il = nullptr,
+         *iloff = nullptr;
+    int nnear = 0, ninner = 0, R = 1;
+    std::vector<int> il_base, il_max;
+    uint64_t last = 0;
+};
+
+FmmSplit::~FmmSplit() = default;
+
+struct FmmPlanCache {
+    std::vector<std::unique_ptr<FmmPlan>> v;
+    uint64_t clock = 0;
+};
+
+constexpr size_t kPlans = 6;
+
+// What the tables depend on: near sets are symmetric and shrink with |dy|, so
+// the reach in x for every dy >= 0 describes one.
+static std::vector<uint8_t> plan_key(const FmmArgs &a, const Domain &dom, int type, bool far,
+                                     double shape_log2)
+{
+    std::vector<uint8_t> k = {(uint8_t)type, (uint8_t)dom.L,      (uint8_t)a.p,
+                              (uint8_t)(a.p >> 8), (uint8_t)a.ws, (uint8_t)far};
+    const double c2 = a.cutoff * a.cutoff;
+    auto reach = [&k](int R, auto in) {
+        for (int dy = 0; dy <= R; ++dy) {
+            int dx = -1;
+            while (dx < R && in(dx + 1, dy)) ++dx;
+            if (dx < 0) break;
+            k.push_back((uint8_t)(dx + 1));
+        }
+        k.push_back(0);
+    };
+    for (int l = far ? 0 : dom.L; l <= dom.L; ++l) {
+        const double s = dom.D / std::ldexp(1.0, l);
+        reach(near_window(s, c2, a.ws, l),
+              [&](int dx, int dy) { return near_offset(dx, dy, a.ws, s, c2); });
+    }
+    reach(near_window(dom.s, c2, a.ws, dom.L), [&](int dx, int dy) {
+        return near_offset(dx, dy, a.ws, dom.s, c2) && near_offset_core(dx, dy, dom.s, shape_log2);
+    });
+    return k;
+}
+
+void fmm_plans_release(Lane *L)
+{
+    if (!L->fmm_plans) return;
+    for (auto &q : L->fmm_plans->v)
+        if (q->dev) (void)hipFree(q->dev);
+    delete L->fmm_plans;
+    L->fmm_plans = nullptr;
+}
+
+// The plan of (a, dom): the lane's own, or a new one.  While a graph is being
+// recorded (spl) the tables go to the recording instead, which owns them.
 template <class T, class TC>
-static int run_fmm_typed(Lane *L, const FmmArgs &a, const Domain &dom, const Lists &ls,
-                         const SortedPoints &S, const SortedPoints &Tg, StageTimer &tm,
-                         bool *used, FmmInfo *info, FmmSplit *spl)
+static int fmm_plan(Lane *L, const FmmArgs &a, const Domain &dom, const PairParams &pp, bool far,
+                    FmmSplit *spl, const FmmPlan **out)
+{
+    using V = typename C2<T>::type;
+    const int Lv = dom.L, p1 = a.p + 1;
+    const double shape_log2 = 1.4426950408889634074 * pp.inv_ks;
+    if (!L->fmm_plans) L->fmm_plans = new FmmPlanCache;
+    FmmPlanCache &c = *L->fmm_plans;
+    std::vector<uint8_t> key =
+        plan_key(a, dom, (int)(sizeof(T) + 16 * sizeof(TC)), far, shape_log2);
+    if (!spl)
+        for (auto &q : c.v)
+            if (q->key == key) {
+                q->last = ++c.clock;
+                *out = q.get();
+                return PHF_OK;
+            }
+    std::unique_ptr<FmmPlan> pl(new FmmPlan);
+    pl->key = std::move(key);
+    const Lists ls = make_lists(dom, a.cutoff * a.cutoff, a.ws);
+    // near list at the leaf level, offsets that can hold pairs inside the
+    // smoothing core first: for the others the box gap g satisfies
+    // shape g^2 log2(e) >= 26 with a 2% margin for float32 rounding of the
+    // point offsets, so exp(-shape r2) <= 2^-26 for every pair
+    std::vector<int2> near_ord, outer;
+    for (const int2 &o : ls.near_leaf)
+        (near_offset_core(o.x, o.y, dom.s, shape_log2) ? near_ord : outer).push_back(o);
+    pl->ninner = (int)near_ord.size();
+    near_ord.insert(near_ord.end(), outer.begin(), outer.end());
+    pl->nnear = (int)near_ord.size();
+    TableBlob blob;
+    blob.add(near_ord, &pl->near);
+    pl->il_base.assign(Lv + 1, 0);
+    pl->il_max.assign(Lv + 1, 0);
+    const int R = pl->R = std::max(ls.R, 1);
+    if (far) {
+        // Pascal triangle C(m, k) for the multi-level shifts
+        std::vector<TC> pas((size_t)p1 * p1);
+        for (int m = 0; m < p1; ++m)
+            for (int k = 0; k < p1; ++k) pas[(size_t)m * p1 + k] = (TC)binom_d(m, k);
+        blob.add(pas, &pl->pas);
+        // M2L: binomial rows C(k+m, k) and powers u^k, u = -1/offset
+        std::vector<T> bin((size_t)p1 * p1);
+        for (int m = 0; m < p1; ++m)
+            for (int k = 0; k < p1; ++k) bin[(size_t)m * p1 + k] = (T)binom_d(k + m, k);
+        const int W2 = 2 * R + 1;
+        std::vector<V> U((size_t)W2 * W2 * (p1 + 1));
+        for (int oy = -R; oy <= R; ++oy)
+            for (int ox = -R; ox <= R; ++ox) {
+                std::complex<double> u = 0.0;
+                if (ox || oy) u = -1.0 / std::complex<double>(ox, oy);
+                std::complex<double> pw = 1.0;
+                for (int k = 0; k <= p1; ++k) {
+                    U[((size_t)(oy + R) * W2 + (ox + R)) * (p1 + 1) + k] =
+                        V{(T)pw.real(), (T)pw.imag()};
+                    pw *= u;
+                }
+            }
+        blob.add(bin, &pl->bin);
+        blob.add(U, &pl->U);
+        std::vector<int2> il_all;
+        std::vector<int32_t> il_offs;
+        for (int l = 2; l <= Lv; ++l) {
+            pl->il_base[l] = (int)il_offs.size();
+            for (int q = 0; q < 5; ++q) il_offs.push_back((int32_t)il_all.size() + ls.il_off[l][q]);
+            for (int q = 0; q < 4; ++q)
+                pl->il_max[l] = std::max(pl->il_max[l], ls.il_off[l][q + 1] - ls.il_off[l][q]);
+            il_all.insert(il_all.end(), ls.il[l].begin(), ls.il[l].end());
+        }
+        blob.add(il_all, &pl->il);
+        blob.add(il_offs, &pl->iloff);
+    }
+    if (spl) {
+        PHF_TRY(blob.send(L, spl->tables_keep, spl->side, true));
+        spl->plan = std::move(pl);
+        *out = spl->plan.get();
+        return PHF_OK;
+    }
+    if (c.v.size() >= kPlans) {
+        auto lru = std::min_element(c.v.begin(), c.v.end(), [](const auto &x, const auto &y) {
+            return x->last < y->last;
+        });
+        PHF_TRY(lane_quiesce(L));  // launches in flight may still read its tables
+        if ((*lru)->dev) (void)hipFree((*lru)->dev);
+        c.v.erase(lru);
+    }
+    pl->last = ++c.clock;
+    c.v.push_back(std::move(pl));
+    FmmPlan *q = c.v.back().get();
+    const int rc = blob.send(L, &q->dev, L->stream, false);
+    if (rc != PHF_OK) {
+        if (q->dev) (void)hipFree(q->dev);
+        c.v.pop_back();
+        return rc;
+    }
+    *out = q;
+    return PHF_OK;
+}
+
+template <class T, class TC>
+static int run_fmm_typed(Lane *L, const FmmArgs &a, const Domain &dom, const SortedPoints &S, const SortedPoints &Tg, StageTimer &tm,
+                         bool *used, FmmInfo *info, FmmSplit *spl, int *nnear_out)
 {
     using V = typename C2<T>::type;
     const int Lv = dom.L, p1 = a.p + 1;
@@ -1164,80 +1328,29 @@ static int run_fmm_typed(Lane *L, const FmmArgs &a, const Domain &dom, const Lis
     }
     PHF_HIP(hipGetLastError());
 
-    // near list at the leaf level, offsets that can hold pairs inside the
-    // smoothing core first: for the others the box gap g satisfies
-    // shape g^2 log2(e) >= 26 with a 2% margin for float32 rounding of the
-    // point offsets, so exp(-shape r2) <= 2^-26 for every pair
-    std::vector<int2> near_ord;
-    int ninner = 0;
-    {
-        const double shape_log2 = 1.4426950408889634074 * pp.inv_ks;
-        std::vector<int2> far;
-        for (const int2 &o : ls.near_leaf)
-            (near_offset_core(o.x, o.y, dom.s, shape_log2) ? near_ord : far).push_back(o);
-        ninner = (int)near_ord.size();
-        near_ord.insert(near_ord.end(), far.begin(), far.end());
-    }
-    // near list and the far-field tables, uploaded together
-    TableBlob blob;
-    int2 *d_near = nullptr;
-    blob.add(near_ord, &d_near);
+    // the near list (offsets that can hold pairs inside the smoothing core
+    // first) and the far field's tables
     const bool far = Lv >= 2 && a.nb > 0;
-    // level offsets in the coefficient arrays
-    std::vector<int64_t> off(Lv + 2, 0);
+    std::vector<int64_t> off(Lv + 2, 0);  // level offsets in the coefficient arrays
     for (int l = 0; l <= Lv; ++l) off[l + 1] = off[l] + (int64_t(1) << (2 * l));
-    TC *d_pas = nullptr;
-    T *d_bin = nullptr;
-    V *d_U = nullptr;
-    int2 *d_il = nullptr;
-    int32_t *d_iloff = nullptr;
-    std::vector<int> il_base(Lv + 1, 0), il_max(Lv + 1, 0);
-    const int R = std::max(ls.R, 1);
-    if (far) {
-        // Pascal triangle C(m, k) for the multi-level shifts
-        std::vector<TC> pas((size_t)p1 * p1);
-        for (int m = 0; m < p1; ++m)
-            for (int k = 0; k < p1; ++k) pas[(size_t)m * p1 + k] = (TC)binom_d(m, k);
-        blob.add(pas, &d_pas);
-        // M2L: binomial rows C(k+m, k) and powers u^k, u = -1/offset
-        std::vector<T> bin((size_t)p1 * p1);
-        for (int m = 0; m < p1; ++m)
-            for (int k = 0; k < p1; ++k) bin[(size_t)m * p1 + k] = (T)binom_d(k + m, k);
-        const int W2 = 2 * R + 1;
-        std::vector<V> U((size_t)W2 * W2 * (p1 + 1));
-        for (int oy = -R; oy <= R; ++oy)
-            for (int ox = -R; ox <= R; ++ox) {
-                std::complex<double> u = 0.0;
-                if (ox || oy) u = -1.0 / std::complex<double>(ox, oy);
-                std::complex<double> pw = 1.0;
-                for (int k = 0; k <= p1; ++k) {
-                    U[((size_t)(oy + R) * W2 + (ox + R)) * (p1 + 1) + k] =
-                        V{(T)pw.real(), (T)pw.imag()};
-                    pw *= u;
-                }
-            }
-        blob.add(bin, &d_bin);
-        blob.add(U, &d_U);
-        std::vector<int2> il_all;
-        std::vector<int32_t> il_offs;
-        for (int l = 2; l <= Lv; ++l) {
-            il_base[l] = (int)il_offs.size();
-            for (int q = 0; q < 5; ++q) il_offs.push_back((int32_t)il_all.size() + ls.il_off[l][q]);
-            for (int q = 0; q < 4; ++q)
-                il_max[l] = std::max(il_max[l], ls.il_off[l][q + 1] - ls.il_off[l][q]);
-            il_all.insert(il_all.end(), ls.il[l].begin(), ls.il[l].end());
-        }
-        blob.add(il_all, &d_il);
-        blob.add(il_offs, &d_iloff);
-    }
-    PHF_TRY(blob.send(L, spl ? spl->tables_keep : nullptr, spl ? spl->side : nullptr));
+    const FmmPlan *pl;
+    PHF_TRY((fmm_plan<T, TC>(L, a, dom, pp, far, spl, &pl)));
+    const int2 *d_near = (const int2 *)pl->near;
+    const int nnear = pl->nnear, ninner = pl->ninner;
+    const TC *d_pas = (const TC *)pl->pas;
+    const T *d_bin = (const T *)pl->bin;
+    const V *d_U = (const V *)pl->U;
+    const int2 *d_il = (const int2 *)pl->il;
+    const int32_t *d_iloff = (const int32_t *)pl->iloff;
+    const std::vector<int> &il_base = pl->il_base, &il_max = pl->il_max;
+    const int R = pl->R;
+    *nnear_out = nnear;
     V *M = nullptr, *B = nullptr;
     if (far) {
         PHF_ALLOC(M, L->arena, V, (size_t)off[Lv + 1] * p1);
         PHF_ALLOC(B, L->arena, V, (size_t)off[Lv + 1] * p1);
     }
     const uint32_t nleaf = 1u << (2 * Lv);
-    const int nnear = (int)near_ord.size();
     if (info && info->want_counts) {
         for (int l = 2; far && l <= Lv; ++l)
             count_m2l_links<<<div_up(int64_t(1) << (2 * l), 256), 256, 0, L->stream>>>(
@@ -1446,9 +1559,6 @@ static int run_fmm_typed(Lane *L, const FmmArgs &a, const Domain &dom, const Lis
 static int fmm_enqueue(Lane *L, const FmmArgs &a, const Domain &dom_in, StageTimer &tm,
                        bool *used, FmmInfo *info, FmmSplit *spl, int *nnear)
 {
-    const double c2 = a.cutoff * a.cutoff;
-    const Lists ls = make_lists(dom_in, c2, a.ws);
-    *nnear = (int)ls.near_leaf.size();
     // points in Morton order inside the leaves too, with the key bits the
     // radix passes leave free: targets that share a wave, and sources taken
     // together, sit close, so that more pair batches skip the smoothing
@@ -1486,10 +1596,10 @@ static int fmm_enqueue(Lane *L, const FmmArgs &a, const Domain &dom_in, StageTim
     }
     if (a.prec == PHF_PREC_F32C) {
         if (a.p > 16)
-            return run_fmm_typed<float, double>(L, a, dom, ls, S, Tg, tm, used, info, spl);
-        return run_fmm_typed<float, float>(L, a, dom, ls, S, Tg, tm, used, info, spl);
+            return run_fmm_typed<float, double>(L, a, dom, S, Tg, tm, used, info, spl, nnear);
+        return run_fmm_typed<float, float>(L, a, dom, S, Tg, tm, used, info, spl, nnear);
     }
-    return run_fmm_typed<double, double>(L, a, dom, ls, S, Tg, tm, used, info, spl);
+    return run_fmm_typed<double, double>(L, a, dom, S, Tg, tm, used, info, spl, nnear);
 }
 
 // ------------------------------------------------------ captured graphs --
@@ -1549,6 +1659,7 @@ void fmm_graphs_release(Lane *L)
         (void)hipStreamDestroy(L->stream2);
         L->stream2 = nullptr;
     }
+    fmm_plans_release(L);
     if (L->fork_ev) (void)hipEventDestroy(L->fork_ev);
     if (L->join_ev) (void)hipEventDestroy(L->join_ev);
     L->fork_ev = L->join_ev = nullptr;

@@ -105,6 +105,8 @@ __device__ __forceinline__ void p2m_leaf(const void *__restrict__ src, int32_t s
     }
 }
 
+void set_error(const char *fmt, ...) __attribute__((format(printf, 1, 2)));
+
 // f(integral constant NI) for the compiled NI that holds p1 powers
 template <class F>
 inline int p2m_dispatch(int p1, const F &f)
@@ -121,8 +123,10 @@ inline int p2m_dispatch(int p1, const F &f)
         f(std::integral_constant<int, 8>());
     else if (p1 <= 44)
         f(std::integral_constant<int, 11>());
-    else
+    else {
+        set_error("expansion order %d too large (max 40)", p1 - 1);
         return PHF_ERR_UNSUPPORTED;
+    }
     return PHF_OK;
 }
 

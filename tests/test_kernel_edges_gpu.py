@@ -144,3 +144,36 @@ def test_not_finite_is_refused_anywhere(n, bad):
         y[at] = bad
         with pytest.raises(PhfError, match=r"y\[%d\] is not finite" % at):
             BlobSystem(x, y, x)
+
+
+def test_tree_shapes_in_turn(O):
+    """More tree shapes than a lane keeps tables for, in changing order: the
+    same bits every time a shape comes back, each against the direct sum.
+    Shapes differ in one thing at a time: order, precision, leaf level, box
+    separation, the cutoff against the leaf, targets apart from the sources."""
+    n = 4000
+    s = W.uniform_system(n, seed=3)
+    x, y, w = s["x"], s["y"], s["w"]
+    xopt, cutoff = W.oseen_params(s["sigma"])
+    t = np.random.default_rng(4).random((2, 700))
+    base = dict(prec=F64, order=20, leaf=16, ws=1)
+    shapes = [dict(base), dict(base, order=21), dict(base, order=12), dict(base, prec=F32C),
+              dict(base, prec=F32C, order=16), dict(base, prec=F32C, order=17),
+              dict(base, leaf=64), dict(base, ws=2), dict(base, cut=0.3), dict(base, cut=0.5),
+              dict(base, targets=True), dict(base, leaf=4000)]
+
+    def run(kw):
+        kw = dict(kw)
+        c = cutoff * kw.pop("cut", 1.0)
+        xt, yt = t if kw.pop("targets", False) else (x, y)
+        return np.array(gauss.fmm2d_gpu(x, y, w, xt, yt, 35, xopt, c, 1e-6, **kw)), (xt, yt, c)
+
+    first = []
+    for kw in shapes:
+        got, (xt, yt, c) = run(kw)
+        ref = O.direct_oseen(x, y, w, xt, yt, xopt, c)
+        assert O.rel_l2(got, ref) <= (1e-4 if kw["order"] < 16 else 1e-6), kw
+        first.append(got)
+    rng = np.random.default_rng(5)
+    for k in rng.integers(0, len(shapes), 40):
+        assert np.array_equal(run(shapes[k])[0], first[k]), shapes[k]
