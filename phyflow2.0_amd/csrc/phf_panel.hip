@@ -1641,10 +1641,43 @@ static int dense_inverse(Lane *L, DenseFactors *f)
     return PHF_OK;
 }
 
-int dense_factor_enqueue(Lane *L, const double *B, int64_t rows, int64_t n, DenseFactors *f,
-                         hipEvent_t *marks)
+// A square system through its normal matrix (via_normal).  The pivoted LU is a
+// chain of n pivot searches, 1.8 us a column, and its inverse one of 2 n / 16
+// blocks; the Cholesky of B^T B needs no search and its inverse doubles.  The
+// refinement x += (B^T B)^-1 B^T (c - B x), float64 in the residual and its
+// projection, converges to the same x while 2^-24 cond(B)^2 < 1; a factor
+// whose diagonal spans more than 10^3 (cond(B^T B) >= 10^6, singular matrices
+// among them), or a refinement that does not converge, takes the pivoted LU
+// of B instead, as before, and keeps it for later rebuilds.
+// A rebuild and solve of 301 panels: 955 us by the pivoted LU, 676 us this way.
+__global__ __launch_bounds__(256) void chol_check(const float *__restrict__ dg, int n,
+                                                  int32_t *__restrict__ info)
 {
-    const bool normal = rows > n;
+    __shared__ float lo[256], hi[256];
+    float a = INFINITY, b = 0.0f;
+    for (int k = threadIdx.x; k < n; k += 256) {
+        a = fminf(a, dg[k]);
+        b = fmaxf(b, dg[k]);
+    }
+    lo[threadIdx.x] = a;
+    hi[threadIdx.x] = b;
+    __syncthreads();
+    for (int s = 128; s > 0; s >>= 1) {
+        if ((int)threadIdx.x < s) {
+            lo[threadIdx.x] = fminf(lo[threadIdx.x], lo[threadIdx.x + s]);
+            hi[threadIdx.x] = fmaxf(hi[threadIdx.x], hi[threadIdx.x + s]);
+        }
+        __syncthreads();
+    }
+    if (threadIdx.x == 0 && *info == 0 && !(lo[0] > 1e-3f * hi[0])) *info = n;
+}
+
+int dense_factor_enqueue(Lane *L, const double *B, int64_t rows, int64_t n, DenseFactors *f,
+                         hipEvent_t *marks, bool via_normal)
+{
+    const bool square = rows == n;
+    via_normal = via_normal && square && n <= LU_TMAX;
+    const bool normal = rows > n || (via_normal && !f->lu_only);
     if (!(f->LU && f->rows == rows && f->n == n)) {
         f->rows = rows;
         f->n = n;
@@ -1654,8 +1687,9 @@ int dense_factor_enqueue(Lane *L, const double *B, int64_t rows, int64_t n, Dens
         PHF_ALLOC(f->info, L->arena, int32_t, 1);
         PHF_ALLOC(f->Xinv, L->arena, float, (size_t)(n * n));
         PHF_ALLOC(f->dg, L->arena, float, (size_t)n);
-        if (normal) PHF_ALLOC(f->N64, L->arena, double, (size_t)(n * n));
-        if (normal && n <= LU_TMAX) {
+        const bool ws = rows > n || via_normal;
+        if (ws) PHF_ALLOC(f->N64, L->arena, double, (size_t)(n * n));
+        if (ws && n <= LU_TMAX) {
             const size_t np = (size_t)(SI_B * div_up(n, SI_B));
             PHF_ALLOC(f->Lt, L->arena, float, np * np);
             PHF_ALLOC(f->Wc, L->arena, float, np * np);
@@ -1681,7 +1715,11 @@ int dense_factor_enqueue(Lane *L, const double *B, int64_t rows, int64_t n, Dens
     if (chol)
         PHF_TRY(chol_factor_f32(L, f->LU, (int)n, f->ipiv, f->info, f->dg, f->Lt,
                                 SI_B * (int)div_up(n, SI_B)));
-    else
+    if (chol && square) {
+        chol_check<<<1, 256, 0, L->stream>>>(f->dg, (int)n, f->info);
+        PHF_HIP(hipGetLastError());
+    }
+    if (!chol)
         PHF_TRY(lu_factor_f32(L, f->LU, (int)n, f->ipiv, f->info, f->lu_work));
     if (marks) PHF_HIP(hipEventRecord(marks[1], L->stream));
     if (chol)
@@ -1691,12 +1729,28 @@ int dense_factor_enqueue(Lane *L, const double *B, int64_t rows, int64_t n, Dens
     if (marks) PHF_HIP(hipEventRecord(marks[2], L->stream));
     f->Br = B;
     f->cholesky = chol;
+    f->normal = normal;
     return PHF_OK;
+}
+
+int dense_factor_lu(Lane *L, DenseFactors *f)
+{
+    const int64_t n = f->n;
+    f->lu_only = true;
+    f->normal = f->cholesky = false;
+    to_f32<<<div_up(n * n, 256), 256, 0, L->stream>>>(f->Bc, n * n, f->LU);
+    PHF_TRY(lu_factor_f32(L, f->LU, (int)n, f->ipiv, f->info, f->lu_work));
+    PHF_TRY(dense_inverse(L, f));
+    int32_t hinfo = 0;
+    PHF_HIP(hipMemcpyAsync(&hinfo, f->info, sizeof(int32_t), hipMemcpyDeviceToHost, L->stream));
+    PHF_HIP(hipStreamSynchronize(L->stream));
+    return dense_factor_finish(L, f, hinfo);
 }
 
 int dense_factor_finish(Lane *L, DenseFactors *f, int32_t hinfo)
 {
     const int64_t n = f->n;
+    if (f->cholesky && hinfo != 0 && f->rows == n) return dense_factor_lu(L, f);
     if (f->cholesky && hinfo != 0) {
         // not positive definite in float32: the pivoted LU of the same matrix
         to_f32<<<div_up(n * n, 256), 256, 0, L->stream>>>(f->N64, n * n, f->LU);
@@ -1729,7 +1783,7 @@ int dense_refine_device(Lane *L, const DenseFactors &f, const double *c, double 
                         SolveStats *st, bool warm, int first_burst)
 {
     const int64_t rows = f.rows, n = f.n;
-    const bool normal = rows > n;
+    const bool normal = f.normal;
     double *r, *g;
     RefineState *dst;
     PHF_ALLOC(r, L->arena, double, (size_t)rows);

@@ -36,7 +36,7 @@ struct DenseFactors {
     double *Bc = nullptr;
     float *LU = nullptr;
     float *Xinv = nullptr;       // float32 (P L U)^-1, row-major
-    double *N64 = nullptr;       // B^T B (rows > n)
+    double *N64 = nullptr;       // B^T B (normal)
     void *lu_work = nullptr;
     float *dg = nullptr;         // diagonal of the Cholesky factor
     // Cholesky path: the unit lower factor row-major (Lt), its inverse
@@ -44,6 +44,8 @@ struct DenseFactors {
     // npad x npad with npad = n rounded up to 32
     float *Lt = nullptr, *Wc = nullptr, *Wr = nullptr, *Wt = nullptr;
     bool cholesky = false;       // B^T B factored by Cholesky (else pivoted LU)
+    bool normal = false;         // the factors are of B^T B, not of B
+    bool lu_only = false;        // a square B whose B^T B did not serve
     int32_t *ipiv = nullptr, *info = nullptr;
     int singular_at = 0;
 };
@@ -57,8 +59,13 @@ int dense_factor_device(Lane *L, const double *B, int64_t rows, int64_t n, Dense
 // synchronisation; f->info on the device holds the result), then, once that
 // work is complete and hinfo holds f->info, finish: the pivoted LU if the
 // Cholesky met a non-positive pivot, and the error for a singular matrix.
+// via_normal: a square B of at most 1,024 rows may be solved through B^T B as
+// well (see phf_panel.hip).
 int dense_factor_enqueue(Lane *L, const double *B, int64_t rows, int64_t n, DenseFactors *f,
-                         hipEvent_t *marks = nullptr);
+                         hipEvent_t *marks = nullptr, bool via_normal = false);
+// The pivoted LU of a square B in place of the factors of B^T B, also for
+// later calls on f.  One host synchronisation.
+int dense_factor_lu(Lane *L, DenseFactors *f);
 int dense_factor_finish(Lane *L, DenseFactors *f, int32_t hinfo);
 // Refinement sweeps from x = 0, or from the x given (warm); sweeps go in
 // bursts between host checks, the first of first_burst sweeps.

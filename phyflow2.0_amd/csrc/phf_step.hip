@@ -164,6 +164,11 @@ static int panels_solve_device(Lane *L, Panels *P, const double *vx_cp, const do
     P->have_solution = false;
     PHF_TRY(dense_refine_device(L, P->f, rhs, P->s, &st, warm,
                                 warm ? std::min(6, P->last_iterations + 1) : 6));
+    if (!st.converged && P->f.normal && rows == P->m) {
+        // a square system whose normal matrix is too ill-conditioned
+        PHF_TRY(dense_factor_lu(L, &P->f));
+        PHF_TRY(dense_refine_device(L, P->f, rhs, P->s, &st, false, 6));
+    }
     P->last_iterations = st.iterations;
     P->have_solution = st.converged;
     if (!st.converged) {
@@ -313,7 +318,7 @@ static int panels_rebuild_enqueue(Panels *P, const PanelGeomHost &g)
                                    hipMemcpyDeviceToDevice, L->stream));
         PHF_HIP(hipEventRecord(ev[1], L->stream));
         const int64_t rows = P->problem == PHF_PANELS_PRESCRIBED ? m + 1 : m;
-        PHF_TRY(dense_factor_enqueue(L, P->A, rows, m, &P->f, ev + 2));
+        PHF_TRY(dense_factor_enqueue(L, P->A, rows, m, &P->f, ev + 2, true));
         PHF_TRY(panel_series_geom_device(L, m, P->xs, P->ys, P->xe, P->ye, P->cosA, P->sinA,
                                          &P->sg));
         PHF_HIP(hipEventRecord(ev[5], L->stream));

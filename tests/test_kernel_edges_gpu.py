@@ -177,3 +177,38 @@ def test_tree_shapes_in_turn(O):
     rng = np.random.default_rng(5)
     for k in rng.integers(0, len(shapes), 40):
         assert np.array_equal(run(shapes[k])[0], first[k]), shapes[k]
+
+
+def _ellipse(m, thin, turn=0.1):
+    t = np.linspace(np.pi, -np.pi, m + 1) + turn
+    return np.cos(t), thin * np.sin(t)
+
+
+@pytest.mark.parametrize("problem", ["fixed", "moving"])
+@pytest.mark.parametrize("m,thin", [(3, 1.0), (31, 1.0), (32, 0.5), (33, 0.9), (65, 0.3),
+                                    (300, 1.0), (512, 0.7), (1024, 1.0), (1025, 1.0),
+                                    (200, 0.02), (400, 0.003)])
+def test_square_body_solve(m, thin, problem):
+    """Square panel systems at block edges and at the size where the pivoted LU
+    takes over, from round bodies to thin ones (whose condition number sends
+    them there); after a move as after the creation.  numpy's float64 solve of
+    the body's own matrix, to its condition number times 2^-52 sqrt(m)."""
+    from phyflow_amd.lagrangian import PanelBody
+    xp, yp = _ellipse(m, thin)
+    body = PanelBody(xp, yp, problem)
+    k = 2 * np.pi * np.arange(m) / m
+    vx, vy = 1.0 + 0.2 * np.sin(3 * k), 0.3 * np.cos(2 * k)
+    for move in range(3):
+        if move:
+            body.updateBody((0.1 * move, -0.2), 0.3 * move)
+            c, s = np.cos(0.3 * move), np.sin(0.3 * move)
+            x, y = c * xp - s * yp + 0.1 * move, s * xp + c * yp - 0.2
+        else:
+            x, y = xp, yp
+        g = W.panel_geometry(x, y)
+        A = body.A
+        rhs = -(vx * g["cosA"] + vy * g["sinA"])
+        ref = np.linalg.solve(A, rhs)
+        got = body.solve(vx, vy)
+        cond = np.linalg.cond(A)
+        assert np.linalg.norm(got - ref) <= 4 * cond * 2.0 ** -52 * m ** 0.5 * np.linalg.norm(ref)
