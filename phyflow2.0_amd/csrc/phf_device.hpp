@@ -137,15 +137,15 @@ __device__ __forceinline__ float pair_f32_far(float dx, float dy, float w, const
 // relative at |r| = ln2/2); expm1(x) = 2^k expm1(r) + (2^k - 1), whose
 // second term is exact for k >= -53.  x is clamped at -40, where expm1
 // rounds to -1.
-// a b + c as the three-operand v_fma_f64.  With c a constant held in a
-// register (a Horner coefficient hoisted out of a loop) the compiler
-// otherwise copies c into the destination and uses the two-address
-// v_fmac_f64: one extra move per Horner step.  The same operation, so the
-// same result.
+// a b + c as the three-operand v_fma_f64 with c, the same in every lane, read
+// from a scalar register.  Otherwise the compiler copies c into the
+// destination and uses the two-address v_fmac_f64, or moves it into a vector
+// register before each use: an instruction more per Horner step.  The same
+// operation, so the same result.
 __device__ __forceinline__ double fma3_f64(double a, double b, double c)
 {
     double d;
-    asm("v_fma_f64 %0, %1, %2, %3" : "=v"(d) : "v"(a), "v"(b), "v"(c));
+    asm("v_fma_f64 %0, %1, %2, %3" : "=v"(d) : "v"(a), "v"(b), "s"(c));
     return d;
 }
 

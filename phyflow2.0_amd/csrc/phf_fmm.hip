@@ -491,9 +491,11 @@ __device__ __forceinline__ void p2p_near_leaf_f32s(
     const float4 *__restrict__ src, const int32_t *__restrict__ sp,
     const float2 *__restrict__ tgt, const int32_t *__restrict__ start_t, int Lvl, uint32_t b,
     const int2 *__restrict__ near, int nnear, int ninner, const PairParams &pp, float s_f,
-    double2 *__restrict__ nsum, float4 *st, float4 *acc)
+    double2 *__restrict__ nsum, float4 *st, float4 *acc, int q, int P)
 {
-    const int32_t t0 = start_t[b], t1 = start_t[b + 1];
+    const int32_t tl = start_t[b];
+    int32_t t0 = tl, t1 = start_t[b + 1];
+    p2p_part(t0, t1, q, P);
     if (t1 <= t0) return;
     const int n = 1 << Lvl;
     const NearList nf{near, ninner, (int)compact_bits(b), (int)compact_bits(b >> 1), n, s_f};
@@ -502,8 +504,8 @@ __device__ __forceinline__ void p2p_near_leaf_f32s(
     const int32_t ts = sp[b];
     auto tpos = [&](int32_t i) {
         if (tgt) return tgt[i];
-        const float4 q = src[ts + (i - t0)];  // targets are the sources
-        return make_float2(q.x, q.y);
+        const float4 r = src[ts + (i - tl)];  // targets are the sources
+        return make_float2(r.x, r.y);
     };
     auto out = [&](int32_t i, float ha, float la, float hb, float lb) {
         nsum[i] = make_double2(((double)ha + (double)la) * (double)lam,
@@ -517,15 +519,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void p
     const float4 *__restrict__ src, const int32_t *__restrict__ sp,
     const float2 *__restrict__ tgt, const int32_t *__restrict__ start_t, int Lvl,
     const int32_t *__restrict__ split, const int2 *__restrict__ near, int nnear, int ninner,
-    PairParams pp, float s_f, double2 *__restrict__ nsum)
+    PairParams pp, float s_f, int P, double2 *__restrict__ nsum)
 {
     __shared__ float4 st[P2P_STAGE];
     __shared__ float4 acc[P2P_CHUNKS * 4 * 16];
-    const int32_t hi = split[(blockIdx.x & 7u) + 1];
-    for (int32_t bl = split[blockIdx.x & 7u] + (int32_t)(blockIdx.x >> 3); bl < hi;
-         bl += (int32_t)(gridDim.x >> 3))
-        p2p_near_leaf_f32s<KIND>(src, sp, tgt, start_t, Lvl, (uint32_t)bl, near, nnear, ninner,
-                                 pp, s_f, nsum, st, acc);
+    const int32_t lo = split[blockIdx.x & 7u];
+    const int32_t items = (split[(blockIdx.x & 7u) + 1] - lo) * P;  // P parts of each leaf
+    for (int32_t it = (int32_t)(blockIdx.x >> 3); it < items; it += (int32_t)(gridDim.x >> 3))
+        p2p_near_leaf_f32s<KIND>(src, sp, tgt, start_t, Lvl, (uint32_t)(lo + it / P), near, nnear,
+                                 ninner, pp, s_f, nsum, st, acc, it % P, P);
 }
 
 // L2P on the far side (the far field's last kernel, beside the near
@@ -610,26 +612,26 @@ __global__ void out_scatter_f32(const float4 *__restrict__ src, const int32_t *_
 // the XCD leaf ranges split by target count, written in sorted target
 // order: nsum[i] = (a, b) of target i.  Absolute coordinates and
 // pair_f64's operation order.
-template <int KIND>
-__global__ __launch_bounds__(256) void p2p_near_f64s(
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void p2p_near_f64s(
     const double4 *__restrict__ src, const int32_t *__restrict__ start_s,
     const double2 *__restrict__ tgt, const int32_t *__restrict__ start_t, int Lvl,
     const int32_t *__restrict__ split, const int2 *__restrict__ near, int nnear, PairParams pp,
-    double2 *__restrict__ nsum)
+    int P, double2 *__restrict__ nsum)
 {
     __shared__ double4 st[P2P_STAGE_F64];
     __shared__ double2 acc[P2P_CHUNKS * 4 * 16];
-    const int32_t hi = split[(blockIdx.x & 7u) + 1];
+    const int32_t lo = split[blockIdx.x & 7u];
+    const int32_t items = (split[(blockIdx.x & 7u) + 1] - lo) * P;  // P parts of each leaf
     const int n = 1 << Lvl;
-    for (int32_t bl = split[blockIdx.x & 7u] + (int32_t)(blockIdx.x >> 3); bl < hi;
-         bl += (int32_t)(gridDim.x >> 3)) {
-        const uint32_t b = (uint32_t)bl;
-        const int32_t t0 = start_t[b], t1 = start_t[b + 1];
+    for (int32_t it = (int32_t)(blockIdx.x >> 3); it < items; it += (int32_t)(gridDim.x >> 3)) {
+        const uint32_t b = (uint32_t)(lo + it / P);
+        int32_t t0 = start_t[b], t1 = start_t[b + 1];
+        p2p_part(t0, t1, it % P, P);
         if (t1 <= t0) continue;
         const NearList nf{near, nnear, (int)compact_bits(b), (int)compact_bits(b >> 1), n, 0.f};
         auto tpos = [&](int32_t i) { return tgt[i]; };
         auto out = [&](int32_t i, double a, double bb) { nsum[i] = make_double2(a, bb); };
-        p2p_leaf_f64<KIND>(src, start_s, st, acc, nnear, nf, t0, t1, tpos, pp, out);
+        p2p_leaf_f64(src, start_s, st, acc, nnear, nf, t0, t1, tpos, pp, out);
     }
 }
 
@@ -1365,7 +1367,8 @@ static int run_fmm_typed(Lane *L, const FmmArgs &a, const Domain &dom, const Sor
     // order (beside the far field), then the leaf expansions are added and
     // the outputs written in input order
     const int vout = a.velocity_out ? 1 : 0;
-    const uint32_t nl8 = (nleaf + 7) / 8;
+    const int P = p2p_parts(dom.occupied, (double)a.nt);
+    const uint32_t nl8 = (nleaf * (uint32_t)P + 7) / 8;
     const int32_t *split = Tg.split;  // XCD leaf ranges of the targets
     const int32_t *ts = Tg.start;
     double *qr = a.qr, *qi = a.qi;
@@ -1383,10 +1386,10 @@ static int run_fmm_typed(Lane *L, const FmmArgs &a, const Domain &dom, const Sor
         near = [=](hipStream_t st) {
             if (pp.f32_nocut)
                 p2p_near_f32s<PAIR_OSEEN_NOCUT><<<8 * nl8, 256, 0, st>>>(
-                    s4, sp, t2, ts, Lv, split, d_near, nnear, ninner, pp, s_f, nsum);
+                    s4, sp, t2, ts, Lv, split, d_near, nnear, ninner, pp, s_f, P, nsum);
             else
                 p2p_near_f32s<PAIR_OSEEN><<<8 * nl8, 256, 0, st>>>(
-                    s4, sp, t2, ts, Lv, split, d_near, nnear, ninner, pp, s_f, nsum);
+                    s4, sp, t2, ts, Lv, split, d_near, nnear, ninner, pp, s_f, P, nsum);
             PHF_HIP(hipGetLastError());
             return PHF_OK;
         };
@@ -1433,8 +1436,8 @@ static int run_fmm_typed(Lane *L, const FmmArgs &a, const Domain &dom, const Sor
         double2 *nsum;
         PHF_ALLOC(nsum, L->arena, double2, (size_t)std::max<int64_t>(a.nt, 1));
         near = [=](hipStream_t st) {
-            p2p_near_f64s<PAIR_OSEEN><<<8 * nl8, 256, 0, st>>>(s4, ss, t2, ts, Lv, split, d_near,
-                                                             nnear, pp, nsum);
+            p2p_near_f64s<<<8 * nl8, 256, 0, st>>>(s4, ss, t2, ts, Lv, split, d_near, nnear, pp, P,
+                                                   nsum);
             PHF_HIP(hipGetLastError());
             return PHF_OK;
         };

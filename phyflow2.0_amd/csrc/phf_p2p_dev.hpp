@@ -221,6 +221,28 @@ __device__ __forceinline__ void p2p_sweep(const float4 *__restrict__ st, int a, 
 
 constexpr int P2P_CHUNKS = 8;  // target chunks of 16 per round (128 targets)
 
+// Part q of P of the targets [t0, t1) of a leaf, in whole chunks of 16.
+__device__ __forceinline__ void p2p_part(int32_t &t0, int32_t &t1, int q, int P)
+{
+    const int32_t len = ((t1 - t0 + 15) / 16 + P - 1) / P * 16;
+    t0 += q * len;
+    t1 = min(t1, t0 + len);
+}
+
+// Workgroups per leaf of the near field: enough for eight on each of the 256
+// CUs, each with at least two chunks of targets.  With one per leaf, 768
+// leaves of 157 blobs kept the CUs busy for 67% of the kernel (the last leaves
+// run alone); staging a leaf's sources again costs little against its pairs.
+// 120k float64 blobs, 768 leaves: 323 us with one workgroup per leaf, 267 us
+// with two.
+inline int p2p_parts(double leaves, double targets)
+{
+    const double want = 2048.0 / (leaves > 1.0 ? leaves : 1.0);
+    const double most = targets / (leaves > 1.0 ? leaves : 1.0) / 32.0;
+    const double p = want < most ? want : most;
+    return p <= 1.0 ? 1 : p >= 8.0 ? 8 : (int)p;
+}
+
 // Near-field sums of the targets [t0, t1) of one leaf, in scaled
 // coordinates x' = lam x (pair_scaled).  nf(q, sb, ox, oy, core) gives near
 // index q's source leaf sb, its centre shift (exact in float32) and whether
@@ -339,48 +361,75 @@ __device__ __forceinline__ void p2p_leaf(const float4 *__restrict__ src,
 // ---------------------------------------------------------------- float64
 constexpr int P2P_STAGE_F64 = 768;  // staged sources (double4) per batch
 
-// float64 pair sweep over staged entries x in [a, b) with x = o (mod S)
+// E staged entries of stride S against NT targets: all E NT distances, then
+// one test of whether any pair of the wave is inside the cutoff, and the pairs
+// in one straight run, so that their chains of dependent float64 operations
+// overlap.  Outside, the smoothing factor is 1 exactly (the factor of a pair
+// beyond the cutoff comes out as 1 inside as well).
+//
+// The 1e-200 in r2 changes no pair at a distance (it is far below half an ulp
+// of any r2 above 1e-184) and makes a blob's pair with itself finite, so its
+// P dx is 0 as pair_f64's r2 > 0 test makes it, without that compare and two
+// selects per pair.
+template <int NT, int E, int S>
+__device__ __forceinline__ void p2p_pairs_f64(const double4 *__restrict__ st, int x,
+                                              const double *xt, const double *yt,
+                                              const PairParams &pp, double *ax, double *ay)
+{
+    double dx[E * NT], dy[E * NT], r2[E * NT], w[E];
+    double least = INFINITY;
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+        const double4 q = st[x + S * e];
+        w[e] = q.z;
+#pragma unroll
+        for (int u = 0; u < NT; ++u) {
+            const int k = e * NT + u;
+            dx[k] = xt[u] - q.x;
+            dy[k] = yt[u] - q.y;
+            r2[k] = __builtin_fma(dx[k], dx[k], fma3_f64(dy[k], dy[k], 1e-200));
+            least = k == 0 ? r2[k] : __builtin_fmin(least, r2[k]);
+        }
+    }
+    if (__ballot(least < pp.c2)) {
+        double om[E * NT];
+#pragma unroll
+        for (int k = 0; k < E * NT; ++k)
+            om[k] = __builtin_fmin(-expm1_neg_f64(-pp.inv_ks * r2[k]) * pp.scale, 1.0);
+#pragma unroll
+        for (int k = 0; k < E * NT; ++k) {
+            const double P = div_f64(w[k / NT], r2[k]) * om[k];
+            ax[k % NT] = __builtin_fma(P, dx[k], ax[k % NT]);
+            ay[k % NT] = __builtin_fma(P, dy[k], ay[k % NT]);
+        }
+    } else {
+#pragma unroll
+        for (int k = 0; k < E * NT; ++k) {
+            const double P = div_f64(w[k / NT], r2[k]);
+            ax[k % NT] = __builtin_fma(P, dx[k], ax[k % NT]);
+            ay[k % NT] = __builtin_fma(P, dy[k], ay[k % NT]);
+        }
+    }
+}
+
+// float64 Oseen pair sweep over staged entries x in [a, b) with x = o (mod S)
 // for NT targets at once (each staged record read once for all of them),
-// absolute coordinates, pair_f64's operation order.  (Reading the next
-// entry ahead of the current pairs was measured slower: 1.62 against
-// 1.55 ms at 1M blobs.)
-template <int KIND, int NT, int S = 16>
+// absolute coordinates.
+template <int NT, int S = 16>
 __device__ __forceinline__ void p2p_sweep_f64(const double4 *__restrict__ st, int a, int b, int o,
                                               const double *xt, const double *yt,
                                               const PairParams &pp, double *ax, double *ay)
 {
-    for (int x = a + ((o - a) & (S - 1)); x < b; x += S) {
-        const double4 q = st[x];
-#pragma unroll
-        for (int u = 0; u < NT; ++u) {
-            const double dx = xt[u] - q.x, dy = yt[u] - q.y;
-            double P;
-            if (KIND == PAIR_OSEEN || KIND == PAIR_OSEEN_NOCUT) {
-                // pair_f64's Oseen form; the smoothing factor is skipped
-                // (1 exactly) when no lane of the wave is inside the cutoff.
-                // The 1e-200 in r2 changes no pair at a distance (it is far
-                // below half an ulp of any r2 above 1e-184) and makes a
-                // blob's pair with itself finite, so its P dx is 0 as
-                // pair_f64's r2 > 0 test makes it, without that compare and
-                // two selects per pair.
-                const double r2 = __builtin_fma(dx, dx, __builtin_fma(dy, dy, 1e-200));
-                double om = 1.0;
-                if (__ballot(r2 < pp.c2))
-                    om = __builtin_fmin(-expm1_neg_f64(-pp.inv_ks * r2) * pp.scale, 1.0);
-                P = div_f64(q.z, r2) * om;
-            } else {
-                P = pair_f64<KIND>(dx, dy, q.z, pp);
-            }
-            ax[u] = __builtin_fma(P, dx, ax[u]);
-            ay[u] = __builtin_fma(P, dy, ay[u]);
-        }
-    }
+    constexpr int E = NT == 1 ? 2 : 1;
+    int x = a + ((o - a) & (S - 1));
+    for (; x + (E - 1) * S < b; x += E * S) p2p_pairs_f64<NT, E, S>(st, x, xt, yt, pp, ax, ay);
+    for (; x < b; x += S) p2p_pairs_f64<NT, 1, S>(st, x, xt, yt, pp, ax, ay);
 }
 
 // float64 near-field sums of the targets [t0, t1) of one leaf, the
 // float32 p2p_leaf's layout with float64 records and plain float64
 // partials: out(i, sum_a, sum_b).
-template <int KIND, class NearFn, class TgtFn, class OutFn>
+template <class NearFn, class TgtFn, class OutFn>
 __device__ __forceinline__ void p2p_leaf_f64(const double4 *__restrict__ src,
                                              const int32_t *__restrict__ sp, double4 *st,
                                              double2 *acc, int nnear, const NearFn &nf,
@@ -416,9 +465,9 @@ __device__ __forceinline__ void p2p_leaf_f64(const double4 *__restrict__ src,
                 }
                 const int nu = min(2, npair - c);
                 if (nu == 2)
-                    p2p_sweep_f64<KIND, 2>(st, 0, used, o, xt, yt, pp, ax, ay);
+                    p2p_sweep_f64<2>(st, 0, used, o, xt, yt, pp, ax, ay);
                 else
-                    p2p_sweep_f64<KIND, 1>(st, 0, used, o, xt, yt, pp, ax, ay);
+                    p2p_sweep_f64<1>(st, 0, used, o, xt, yt, pp, ax, ay);
                 for (int u = 0; u < nu; ++u) {
                     ax[u] += __shfl_xor(ax[u], 16);
                     ay[u] += __shfl_xor(ay[u], 16);
@@ -435,7 +484,7 @@ __device__ __forceinline__ void p2p_leaf_f64(const double4 *__restrict__ src,
                 const int32_t i = rc + 16 * c + th;
                 const double2 tp = i < t1 ? tgt(i) : make_double2(0.0, 0.0);
                 double xt[1] = {tp.x}, yt[1] = {tp.y}, ax[1] = {}, ay[1] = {};
-                p2p_sweep_f64<KIND, 1, 32>(st, 0, used, o + 16 * (t >> 3), xt, yt, pp, ax, ay);
+                p2p_sweep_f64<1, 32>(st, 0, used, o + 16 * (t >> 3), xt, yt, pp, ax, ay);
                 ax[0] += __shfl_xor(ax[0], 8);
                 ay[0] += __shfl_xor(ay[0], 8);
                 ax[0] += __shfl_xor(ax[0], 16);

@@ -128,6 +128,9 @@ Domain make_domain(double xmin, double xmax, double ymin, double ymax, int L, do
     d.L = L;
     d.s = d.D / std::ldexp(1.0, L);  // exact (power-of-two division)
     d.inv_s = std::ldexp(1.0, L) / d.D;
+    const double n = std::ldexp(1.0, L);
+    d.occupied = std::min(n, std::max(1.0, std::ceil((xmax - xmin) / d.s))) *
+                 std::min(n, std::max(1.0, std::ceil((ymax - ymin) / d.s)));
     return d;
 }
 

@@ -12,6 +12,7 @@ struct Domain {
     double s;       // leaf box side D / 2^L (exact)
     double inv_s;   // 2^L / D
     int L;
+    double occupied = 1.0;  // leaves that the bounding box touches
     // sort keys carry 2 * fine more bits below the leaf index, the Morton
     // order of a 2^fine x 2^fine grid inside each leaf (leaf = key >> 2 fine)
     int fine = 0;

@@ -212,3 +212,22 @@ def test_square_body_solve(m, thin, problem):
         got = body.solve(vx, vy)
         cond = np.linalg.cond(A)
         assert np.linalg.norm(got - ref) <= 4 * cond * 2.0 ** -52 * m ** 0.5 * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("n,leaf", [(70, 200), (500, 1000), (3001, 3001), (3001, 100),
+                                    (20011, 300), (60013, 230)])
+@pytest.mark.parametrize("prec,tol", [(F64, 1e-7), (F32C, 1e-6)])
+def test_leaves_in_parts(n, leaf, prec, tol, O):
+    """Few leaves of many targets, each split over one to eight workgroups; the
+    targets also apart from the sources.  Order 24 leaves the near field's own
+    error (and 1e-8 of the expansions')."""
+    s = W.uniform_system(n, seed=n)
+    x, y, w = s["x"], s["y"], s["w"]
+    xopt, cutoff = W.oseen_params(s["sigma"])
+    t = np.random.default_rng(n).random((2, n // 3 + 1))
+    for xt, yt in ((x, y), t):
+        got = gauss.fmm2d_gpu(x, y, w, xt, yt, 35, xopt, cutoff, 1e-6, prec=prec, order=24,
+                              leaf=leaf)
+        sub = np.arange(0, xt.size, max(1, xt.size // 2000))
+        ref = O.direct_oseen(x, y, w, xt[sub], yt[sub], xopt, cutoff)
+        assert O.rel_l2([g[sub] for g in got], ref) <= tol
