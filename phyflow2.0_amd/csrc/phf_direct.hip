@@ -205,8 +205,8 @@ __global__ __launch_bounds__(64) void direct_f64(
 // same P either way.  The partials are in sorted target order.
 // Bound by float64 issue: 15 operations and a reciprocal estimate per pair
 // beyond it, 36 inside.  20,011 sources, 30,017 targets: 731 us for the call's
-// kernels in input order, 439 us sorted (45 us of it the sort); 40,000 x
-// 80,000: 3,829 against 1,928 us.
+// kernels in input order, 430 us sorted (45 us of it the sort); 40,000 x
+// 80,000: 3,829 against 1,708 us.
 template <int KIND>
 __global__ __launch_bounds__(64) void direct_f64_sorted(
     const double *__restrict__ xb, const double *__restrict__ yb, const double *__restrict__ wb,
@@ -224,13 +224,33 @@ __global__ __launch_bounds__(64) void direct_f64_sorted(
     const int64_t j0 = (int64_t)blockIdx.y * chunk_len;
     const int64_t j1 = min(nb, j0 + chunk_len);
     int64_t j = j0;
-    for (; j + 4 <= j1; j += 4) {
-        double dx[4], dy[4], r2[4], w[4];
+    // the next four sources' scalar loads go out before the current pairs
+    double nx[4], ny[4], nw[4];
+    const int64_t jl = max(j0, j1 - 4);
+    if (j + 4 <= j1)
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
-            w[k] = wb[j + k];
-            dx[k] = tx - xb[j + k];
-            dy[k] = ty - yb[j + k];
+            nx[k] = xb[j + k];
+            ny[k] = yb[j + k];
+            nw[k] = wb[j + k];
+        }
+    for (; j + 4 <= j1; j += 4) {
+        double dx[4], dy[4], r2[4], w[4], sx[4], sy[4];
+        const int64_t jn = min(j + 4, jl);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            sx[k] = nx[k];
+            sy[k] = ny[k];
+            w[k] = nw[k];
+            nx[k] = xb[jn + k];
+            ny[k] = yb[jn + k];
+            nw[k] = wb[jn + k];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            dx[k] = tx - sx[k];
+            dy[k] = ty - sy[k];
             r2[k] = __builtin_fma(dx[k], dx[k], fma3_f64(dy[k], dy[k], eps));
         }
         const double least = __builtin_fmin(__builtin_fmin(r2[0], r2[1]),
@@ -677,7 +697,7 @@ static int target_order(Lane *L, const double *xt, const double *yt, int64_t nt,
 }
 
 // Source chunks of a direct sum over nt targets in groups of 64 * tpl:
-// enough chunks that the grid holds ~8 waves per SIMD of the chip, each of
+// enough chunks that the waves fill the chip in whole rounds, each of
 // at least 64 sources (a multiple of 16); one chunk once the target groups
 // alone fill the chip.  max_chunks caps the count (the partial sums take
 // nchunk * nt double2).
@@ -686,8 +706,21 @@ static void direct_split(int64_t nt, int tpl, int64_t nb, int64_t *nchunk_out,
 {
     const int64_t tblock = (int64_t)kWave * tpl;
     const int64_t ngroups = (nt + tblock - 1) / tblock;
-    const int64_t want_waves = 8192;
-    int64_t nchunk = std::max<int64_t>(1, (want_waves + ngroups - 1) / ngroups);
+    // whole rounds of the 8,192 waves the chip holds: the first count that
+    // leaves at most 5% of the last round empty, else the fullest (18 chunks
+    // of 470 groups left a second round of 268 waves)
+    const int64_t full = 8192;
+    int64_t nchunk = 1;
+    double best = 0.0;
+    for (int64_t c = 1; c * ngroups <= 5 * full || c == 1; ++c) {
+        const int64_t waves = c * ngroups, rounds = (waves + full - 1) / full;
+        const double eff = (double)waves / (double)(rounds * full);
+        if (eff > best) {
+            best = eff;
+            nchunk = c;
+        }
+        if (eff >= 0.95) break;
+    }
     nchunk = std::min<int64_t>(nchunk, std::max<int64_t>(1, nb / 64));
     nchunk = std::min<int64_t>(nchunk, std::max<int64_t>(1, std::min<int64_t>(max_chunks, 65535)));
     int64_t chunk_len = (nb + nchunk - 1) / nchunk;
