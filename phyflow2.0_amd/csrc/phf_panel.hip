@@ -14,6 +14,7 @@
 // at float64 resolution.  Over-determined systems (the 'prescribed' problem)
 // are solved through the normal equations B^T B x = B^T c, refined with the
 // float64 semi-normal residual B^T (c - B x).
+#include "phf_fmm_dev.hpp"
 #include "phf_panel.hpp"
 #include "phf_tree.hpp"
 
@@ -166,48 +167,54 @@ __global__ void to_colmajor(const double *__restrict__ B, int64_t rows, int64_t 
 }
 
 // N = B^T B (n x n, column-major, F64 and F32 copies); Bc column-major rows x n.
-// One workgroup per 32 x 32 tile of N: the 32 columns of B on each side are
-// staged in LDS 32 rows at a time and each thread adds 2 x 2 outputs, every
-// output summed over the rows in order (one FMA chain).
-constexpr int NM_T = 32;
+// One workgroup per 16 x 16 tile on and below the diagonal (the tile above is
+// its transpose), on v_mfma_f64_16x16x4f64 straight from memory: lane l holds
+// column l % 16 of either side at row l / 16 of a step of 4 rows, so the four
+// rows of a column are one 32-byte read.  The four waves take a quarter of the
+// rows each and are added in wave order.  Bound by the latency of the reads:
+// with 32 x 32 tiles staged in LDS by barriers, 301 columns took 35 us and 512
+// columns 55 us; now 8.6 us and, beside a near field, 22 us.
+constexpr int NM_T = 16;
+typedef double doublex4 __attribute__((ext_vector_type(4)));
 __global__ __launch_bounds__(256) void normal_matrix(const double *__restrict__ Bc, int64_t rows,
                                                      int64_t n, double *__restrict__ N64,
                                                      float *__restrict__ N32)
 {
-    __shared__ double Ti[NM_T][NM_T + 1];  // [column of the i side][row]
-    __shared__ double Tj[NM_T][NM_T + 1];
+    if (blockIdx.x < blockIdx.y) return;
+    __shared__ double part[4][256];
+    const int tid = threadIdx.x, wv = tid >> 6, lane = tid & 63, li = lane & 15, lk = lane >> 4;
     const int64_t i0 = (int64_t)blockIdx.x * NM_T, j0 = (int64_t)blockIdx.y * NM_T;
-    const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
-    double acc[2][2] = {{0.0, 0.0}, {0.0, 0.0}};
-    for (int64_t r0 = 0; r0 < rows; r0 += NM_T) {
-        for (int e = threadIdx.x; e < NM_T * NM_T; e += 256) {
-            const int c = e / NM_T, k = e % NM_T;
-            const int64_t r = r0 + k;
-            Ti[c][k] = (i0 + c < n && r < rows) ? Bc[(i0 + c) * rows + r] : 0.0;
-            Tj[c][k] = (j0 + c < n && r < rows) ? Bc[(j0 + c) * rows + r] : 0.0;
+    const double *ci = Bc + min(i0 + li, n - 1) * rows;
+    const double *cj = Bc + min(j0 + li, n - 1) * rows;
+    const int64_t quarter = ((rows + 15) / 16) * 4;
+    const int64_t r0 = wv * quarter, r1 = min(rows, r0 + quarter);
+    doublex4 acc = {0.0, 0.0, 0.0, 0.0};
+    for (int64_t r = r0; r < r1; r += 32) {
+        double a[8], b[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const int64_t k = r + 4 * u + lk;
+            const bool in = k < r1;
+            a[u] = in ? ci[k] : 0.0;
+            b[u] = in ? cj[k] : 0.0;
         }
-        __syncthreads();
-#pragma unroll 8
-        for (int k = 0; k < NM_T; ++k) {
-            const double a0 = Ti[tx][k], a1 = Ti[tx + 16][k];
-            const double b0 = Tj[ty][k], b1 = Tj[ty + 16][k];
-            acc[0][0] = __builtin_fma(a0, b0, acc[0][0]);
-            acc[1][0] = __builtin_fma(a1, b0, acc[1][0]);
-            acc[0][1] = __builtin_fma(a0, b1, acc[0][1]);
-            acc[1][1] = __builtin_fma(a1, b1, acc[1][1]);
-        }
-        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+            acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a[u], b[u], acc, 0, 0, 0);
     }
+    // result register v of lane l: row 4 v + l / 16, column l % 16
 #pragma unroll
-    for (int a = 0; a < 2; ++a)
-#pragma unroll
-        for (int b = 0; b < 2; ++b) {
-            const int64_t i = i0 + tx + 16 * a, j = j0 + ty + 16 * b;
-            if (i < n && j < n) {
-                N64[j * n + i] = acc[a][b];
-                N32[j * n + i] = (float)acc[a][b];
-            }
-        }
+    for (int v = 0; v < 4; ++v) part[wv][(4 * v + lk) * 16 + li] = acc[v];
+    __syncthreads();
+    const int64_t i = i0 + (tid >> 4), j = j0 + (tid & 15);
+    if (i >= n || j >= n) return;
+    const double s = ((part[0][tid] + part[1][tid]) + part[2][tid]) + part[3][tid];
+    N64[j * n + i] = s;
+    N32[j * n + i] = (float)s;
+    if (blockIdx.x != blockIdx.y) {
+        N64[i * n + j] = s;
+        N32[i * n + j] = (float)s;
+    }
 }
 
 // --------------------------------------------------------------- LU -------
@@ -1793,8 +1800,10 @@ int dense_refine_device(Lane *L, const DenseFactors &f, const double *c, double 
                                                                           dst);
     const int max_it = 60;
     RefineState hs{};
+    // sweeps are launched ahead of their verdict: a square system through its
+    // normal matrix takes 5 to 8 from cold (301 panels: 8), then 3 at a time
     for (int launched = 0, burst = std::max(1, first_burst); launched < max_it;
-         launched += burst, burst = 6) {
+         launched += burst, burst = 3) {
         for (int b = 0; b < burst && launched + b < max_it; ++b) {
             resid_rows<<<div_up(rows, 4), 256, 0, L->stream>>>(f.Br, rows, n, x, c, r, dst);
             const double *rhs = r;
@@ -1944,77 +1953,73 @@ __global__ __launch_bounds__(64) void panel_group_coeffs(
 // panel_group_coeffs without the strengths: the group headers, and per
 // panel p of the group and term k the factor geo[p * PG_TERMS + k] =
 // R_g / (2 pi) (s_p + i c_p) (zh2^(k+1) - zh1^(k+1)) / (k + 1), so that
-// b_k = sum_p gamma_p geo[p][k] (panel_group_apply).
-__global__ __launch_bounds__(64) void panel_group_geom(
+// b_k = sum_p gamma_p geo[p][k] (panel_group_apply).  One thread per panel and
+// term, powers by squaring (one thread per term, multiplying its way up for
+// the sixteen panels in turn, took 30 us).
+__global__ __launch_bounds__(PG_SIZE * 32) void panel_group_geom(
     int64_t M, const double *__restrict__ xs, const double *__restrict__ ys,
     const double *__restrict__ xe, const double *__restrict__ ye,
     const double *__restrict__ cosA, const double *__restrict__ sinA, PanelG *__restrict__ grp,
     double2 *__restrict__ geo)
 {
+    static_assert(PG_TERMS <= 32, "a panel's terms fill at most 32 threads");
     __shared__ double pd[PG_SIZE][6];  // xs, ys, xe, ye, cos, sin
-    __shared__ double sc[3];
-    const int g = blockIdx.x, k = threadIdx.x;
+    const int g = blockIdx.x, tid = threadIdx.x, q = tid >> 5, k = tid & 31;
     const int64_t p0 = (int64_t)g * PG_SIZE;
     const int cnt = (int)min((int64_t)PG_SIZE, M - p0);
-    if (k < cnt) {
-        const int64_t p = p0 + k;
-        pd[k][0] = xs[p];
-        pd[k][1] = ys[p];
-        pd[k][2] = xe[p];
-        pd[k][3] = ye[p];
-        pd[k][4] = cosA[p];
-        pd[k][5] = sinA[p];
+    if (tid < cnt) {
+        const int64_t p = p0 + tid;
+        pd[tid][0] = xs[p];
+        pd[tid][1] = ys[p];
+        pd[tid][2] = xe[p];
+        pd[tid][3] = ye[p];
+        pd[tid][4] = cosA[p];
+        pd[tid][5] = sinA[p];
     }
     __syncthreads();
-    if (k == 0) {
-        double cx = 0.0, cy = 0.0;
-        for (int q = 0; q < cnt; ++q) {
-            cx += 0.5 * (pd[q][0] + pd[q][2]);
-            cy += 0.5 * (pd[q][1] + pd[q][3]);
-        }
-        cx /= cnt;
-        cy /= cnt;
-        double r2 = 0.0;
-        for (int q = 0; q < cnt; ++q) {
-            const double a1 = pd[q][0] - cx, b1 = pd[q][1] - cy;
-            const double a2 = pd[q][2] - cx, b2 = pd[q][3] - cy;
-            r2 = fmax(r2, fmax(a1 * a1 + b1 * b1, a2 * a2 + b2 * b2));
-        }
-        const double R = sqrt(r2);
-        sc[0] = cx;
-        sc[1] = cy;
-        sc[2] = R;
+    // centre and radius, the same in every thread
+    double cx = 0.0, cy = 0.0;
+    for (int r = 0; r < cnt; ++r) {
+        cx += 0.5 * (pd[r][0] + pd[r][2]);
+        cy += 0.5 * (pd[r][1] + pd[r][3]);
+    }
+    cx /= cnt;
+    cy /= cnt;
+    double r2 = 0.0;
+    for (int r = 0; r < cnt; ++r) {
+        const double a1 = pd[r][0] - cx, b1 = pd[r][1] - cy;
+        const double a2 = pd[r][2] - cx, b2 = pd[r][3] - cy;
+        r2 = fmax(r2, fmax(a1 * a1 + b1 * b1, a2 * a2 + b2 * b2));
+    }
+    const double R = sqrt(r2), iR = 1.0 / R;
+    if (tid == 0) {
         PanelG pg;
         pg.zx = cx;
         pg.zy = cy;
         pg.far2 = 9.0 * r2;
         pg.R = R;
-        pg.inv_R = 1.0 / R;
+        pg.inv_R = iR;
         pg.first = (int32_t)p0;
         pg.count = cnt;
         pg.pad0 = pg.pad1 = 0;
         grp[g] = pg;
     }
-    __syncthreads();
-    if (k >= PG_TERMS) return;
-    const double cx = sc[0], cy = sc[1], R = sc[2], iR = 1.0 / R;
-    for (int q = 0; q < cnt; ++q) {
-        const double u1 = (pd[q][0] - cx) * iR, v1 = (pd[q][1] - cy) * iR;
-        const double u2 = (pd[q][2] - cx) * iR, v2 = (pd[q][3] - cy) * iR;
-        double p1r = u1, p1i = v1, p2r = u2, p2i = v2;
-        for (int e = 0; e < k; ++e) {
-            const double t1 = p1r * u1 - p1i * v1;
-            p1i = p1r * v1 + p1i * u1;
-            p1r = t1;
-            const double t2 = p2r * u2 - p2i * v2;
-            p2i = p2r * v2 + p2i * u2;
-            p2r = t2;
+    if (k >= PG_TERMS || q >= cnt) return;
+    auto power = [k](double2 z) {  // z^(k+1)
+        double2 r = make_double2(1.0, 0.0);
+#pragma unroll
+        for (int b = 0; b < 5; ++b) {
+            if ((k + 1) & (1 << b)) r = cmul(r, z);
+            z = cmul(z, z);
         }
-        const double dr = (p2r - p1r) / (k + 1), di = (p2i - p1i) / (k + 1);
-        const double f = R / (2.0 * M_PI);
-        const double fr = f * pd[q][5], fi = f * pd[q][4];
-        geo[(p0 + q) * PG_TERMS + k] = make_double2(fr * dr - fi * di, fr * di + fi * dr);
-    }
+        return r;
+    };
+    const double2 z1 = power(make_double2((pd[q][0] - cx) * iR, (pd[q][1] - cy) * iR));
+    const double2 z2 = power(make_double2((pd[q][2] - cx) * iR, (pd[q][3] - cy) * iR));
+    const double dr = (z2.x - z1.x) / (k + 1), di = (z2.y - z1.y) / (k + 1);
+    const double f = R / (2.0 * M_PI);
+    const double fr = f * pd[q][5], fi = f * pd[q][4];
+    geo[(p0 + q) * PG_TERMS + k] = make_double2(fr * dr - fi * di, fr * di + fi * dr);
 }
 
 // b_k of every group from the strengths: one thread per (group, term),
@@ -2050,7 +2055,7 @@ int panel_series_geom_device(Lane *L, int64_t m, const double *xs, const double 
         PHF_ALLOC(grp, L->arena, PanelG, (size_t)ng);
         PHF_ALLOC(geo, L->arena, double2, (size_t)m * PG_TERMS);
     }
-    panel_group_geom<<<(unsigned)ng, 64, 0, L->stream>>>(m, xs, ys, xe, ye, cosA, sinA, grp, geo);
+    panel_group_geom<<<(unsigned)ng, PG_SIZE * 32, 0, L->stream>>>(m, xs, ys, xe, ye, cosA, sinA, grp, geo);
     PHF_HIP(hipGetLastError());
     out->grp = grp;
     out->geo = geo;

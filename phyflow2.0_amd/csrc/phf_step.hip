@@ -163,7 +163,8 @@ static int panels_solve_device(Lane *L, Panels *P, const double *vx_cp, const do
     const bool warm = P->have_solution;
     P->have_solution = false;
     PHF_TRY(dense_refine_device(L, P->f, rhs, P->s, &st, warm,
-                                warm ? std::min(6, P->last_iterations + 1) : 6));
+                                warm ? std::min(6, P->last_iterations + 1)
+                                : P->f.normal && rows == P->m ? 8 : 6));
     if (!st.converged && P->f.normal && rows == P->m) {
         // a square system whose normal matrix is too ill-conditioned
         PHF_TRY(dense_factor_lu(L, &P->f));
@@ -299,13 +300,12 @@ static int panels_rebuild_enqueue(Panels *P, const PanelGeomHost &g)
     const int64_t m = P->m;
     const double *host[9] = {g.xs, g.ys, g.xe, g.ye, g.cs.data(), g.sn.data(), g.Ln.data(),
                              g.xc.data(), g.yc.data()};
-    double *dev[9] = {P->xs, P->ys, P->xe, P->ye, P->cosA, P->sinA, P->L, P->xcp, P->ycp};
     int rc = [&]() -> int {
-        for (int k = 0; k < 9; ++k) {
+        for (int k = 0; k < 9; ++k)
             std::memcpy(P->geom_pin + k * m, host[k], sizeof(double) * m);
-            PHF_HIP(hipMemcpyAsync(dev[k], P->geom_pin + k * m, sizeof(double) * m,
-                                   hipMemcpyHostToDevice, L->stream));
-        }
+        // one slice on the device, in this order
+        PHF_HIP(hipMemcpyAsync(P->xs, P->geom_pin, sizeof(double) * 9 * m, hipMemcpyHostToDevice,
+                               L->stream));
         PHF_HIP(hipEventRecord(P->ev_geom, L->stream));
         P->hxcp = g.xc;
         P->hycp = g.yc;
@@ -415,7 +415,9 @@ int phf_panels_create(const double *xs, const double *ys, const double *xe, cons
         P->gTotal = gTotal;
         double **bufs[9] = {&P->xs, &P->ys, &P->xe, &P->ye, &P->cosA, &P->sinA, &P->L, &P->xcp,
                             &P->ycp};
-        for (double **b : bufs) PHF_ALLOC(*b, L->arena, double, (size_t)m);
+        double *geom;
+        PHF_ALLOC(geom, L->arena, double, (size_t)m * 9);
+        for (int k = 0; k < 9; ++k) *bufs[k] = geom + k * m;
         const int64_t rows = problem == PHF_PANELS_PRESCRIBED ? m + 1 : m;
         PHF_ALLOC(P->A, L->arena, double, (size_t)(rows * m));
         PHF_ALLOC(P->s, L->arena, double, (size_t)m);
