@@ -220,8 +220,8 @@ __global__ void batch_gather(const BatchSys *__restrict__ sys, const int64_t *__
 __global__ void batch_clear_flag(int32_t *flag) { flag[0] = 0; }
 
 // --------------------------------------------------------------- P2M ------
-// one wave per leaf (p2m_leaf), four leaves per workgroup
-template <class T, int NI>
+// p2m_leaf for 64 / R leaves per workgroup
+template <class T, int NI, int R>
 __global__ __launch_bounds__(256) void batch_p2m(const BatchSys *__restrict__ sys,
                                                  const int64_t *__restrict__ loff,
                                                  const int64_t *__restrict__ lvl, int S,
@@ -230,7 +230,7 @@ __global__ __launch_bounds__(256) void batch_p2m(const BatchSys *__restrict__ sy
                                                  const int32_t *__restrict__ start, int64_t nleaf,
                                                  int p1, typename C2<T>::type *__restrict__ M)
 {
-    const int64_t g = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    const int64_t g = (int64_t)blockIdx.x * (64 / R) + threadIdx.x / (4 * R);
     if (g >= nleaf) return;
     const int s = find_seg(loff, S, g);
     const int L = sys[s].L;
@@ -239,7 +239,7 @@ __global__ __launch_bounds__(256) void batch_p2m(const BatchSys *__restrict__ sy
     const BatchDom d = dom[s];
     double cx, cy;
     leaf_center(b, d.x0, d.y0, d.s, cx, cy);
-    p2m_leaf<T, NI>(src, start[g], start[g + 1], cx, cy, (T)(1.0 / d.s), p1,
+    p2m_leaf<T, NI, R>(src, start[g], start[g + 1], cx, cy, (T)(1.0 / d.s), p1,
                     M + (lvl[L * (S + 1) + s] + b) * p1);
 }
 
@@ -1046,9 +1046,11 @@ static int batch_enqueue_typed(Lane *L, const BatchPlan &P, BatchBuffers &Bf, co
     const VC *m2m = reinterpret_cast<const VC *>(Bf.m2m);
     const VC *l2l = reinterpret_cast<const VC *>(Bf.l2l);
     if (P.Lmax >= 2) {
-        PHF_TRY(p2m_dispatch(p1, [&](auto ni) {
-            batch_p2m<T, decltype(ni)::value><<<div_up(P.nleaf, 4), 256, 0, L->stream>>>(
-                Bf.sys, Bf.loff, Bf.lvl, S, Bf.dom, Bf.src, sp, P.nleaf, p1, M);
+        PHF_TRY(p2m_dispatch(p1, (double)P.N, (double)P.nleaf, [&](auto ni, auto r) {
+            constexpr int R = decltype(r)::value;
+            batch_p2m<T, decltype(ni)::value, R>
+                <<<div_up(P.nleaf, 64 / R), 256, 0, L->stream>>>(
+                    Bf.sys, Bf.loff, Bf.lvl, S, Bf.dom, Bf.src, sp, P.nleaf, p1, M);
         }));
         for (int l = P.Lmax - 1; l >= 2; --l) {
             const int64_t nb = P.lvl[(size_t)l * (S + 1) + S] - P.lvl[(size_t)l * (S + 1)];

@@ -80,19 +80,20 @@ __global__ void gather_tgt_f64(const double *__restrict__ x, const double *__res
 }
 
 // ---------------------------------------------------------------- P2M ----
-// One wave per leaf (p2m_leaf), four leaves per workgroup.
-template <class T, int NI>
+// p2m_leaf for 64 / R leaves per workgroup; inv_s is 1 / s.
+template <class T, int NI, int R>
 __global__ __launch_bounds__(256) void p2m_kernel(const void *__restrict__ src,
                                                   const int32_t *__restrict__ start,
                                                   uint32_t nleaf, int p1,
                                                   const double4 *__restrict__ org, double s,
+                                                  double inv_s,
                                                   typename C2<T>::type *__restrict__ M)
 {
-    const uint32_t b = blockIdx.x * 4 + (threadIdx.x >> 6);
+    const uint32_t b = blockIdx.x * (64 / R) + threadIdx.x / (4 * R);
     if (b >= nleaf) return;
-    double cx, cy;
-    leaf_center(b, org->x, org->z, s, cx, cy);
-    p2m_leaf<T, NI>(src, start[b], start[b + 1], cx, cy, (T)(1.0 / s), p1, M + (int64_t)b * p1);
+    double cx = 0.0, cy = 0.0;
+    if (sizeof(T) == 8) leaf_center(b, org->x, org->z, s, cx, cy);
+    p2m_leaf<T, NI, R>(src, start[b], start[b + 1], cx, cy, (T)inv_s, p1, M + (int64_t)b * p1);
 }
 
 // ---------------------------------------------------------- M2M / L2L ----
@@ -495,7 +496,7 @@ __device__ __forceinline__ void p2p_near_leaf_f32s(
 {
     const int32_t tl = start_t[b];
     int32_t t0 = tl, t1 = start_t[b + 1];
-    p2p_part(t0, t1, q, P);
+    if (P > 1) p2p_part(t0, t1, q, P);
     if (t1 <= t0) return;
     const int n = 1 << Lvl;
     const NearList nf{near, ninner, (int)compact_bits(b), (int)compact_bits(b >> 1), n, s_f};
@@ -525,9 +526,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void p
     __shared__ float4 acc[P2P_CHUNKS * 4 * 16];
     const int32_t lo = split[blockIdx.x & 7u];
     const int32_t items = (split[(blockIdx.x & 7u) + 1] - lo) * P;  // P parts of each leaf
-    for (int32_t it = (int32_t)(blockIdx.x >> 3); it < items; it += (int32_t)(gridDim.x >> 3))
-        p2p_near_leaf_f32s<KIND>(src, sp, tgt, start_t, Lvl, (uint32_t)(lo + it / P), near, nnear,
-                                 ninner, pp, s_f, nsum, st, acc, it % P, P);
+    for (int32_t it = (int32_t)(blockIdx.x >> 3); it < items; it += (int32_t)(gridDim.x >> 3)) {
+        const int32_t k = P == 1 ? it : it / P;
+        p2p_near_leaf_f32s<KIND>(src, sp, tgt, start_t, Lvl, (uint32_t)(lo + k), near, nnear,
+                                 ninner, pp, s_f, nsum, st, acc, it - k * P, P);
+    }
 }
 
 // L2P on the far side (the far field's last kernel, beside the near
@@ -612,7 +615,11 @@ __global__ void out_scatter_f32(const float4 *__restrict__ src, const int32_t *_
 // the XCD leaf ranges split by target count, written in sorted target
 // order: nsum[i] = (a, b) of target i.  Absolute coordinates and
 // pair_f64's operation order.
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void p2p_near_f64s(
+// Three workgroups on a CU (141 VGPRs): held to 128 VGPRs four fit and the
+// kernel alone is faster (262k blobs in leaves of 16: 317 against 459 us), but
+// they fill the registers and the far field beside it waits for them: the
+// evaluation took 585 us against 564.
+__global__ __launch_bounds__(256) void p2p_near_f64s(
     const double4 *__restrict__ src, const int32_t *__restrict__ start_s,
     const double2 *__restrict__ tgt, const int32_t *__restrict__ start_t, int Lvl,
     const int32_t *__restrict__ split, const int2 *__restrict__ near, int nnear, PairParams pp,
@@ -624,9 +631,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void p
     const int32_t items = (split[(blockIdx.x & 7u) + 1] - lo) * P;  // P parts of each leaf
     const int n = 1 << Lvl;
     for (int32_t it = (int32_t)(blockIdx.x >> 3); it < items; it += (int32_t)(gridDim.x >> 3)) {
-        const uint32_t b = (uint32_t)(lo + it / P);
+        const int32_t k = P == 1 ? it : it / P;
+        const uint32_t b = (uint32_t)(lo + k);
         int32_t t0 = start_t[b], t1 = start_t[b + 1];
-        p2p_part(t0, t1, it % P, P);
+        if (P > 1) p2p_part(t0, t1, it - k * P, P);
         if (t1 <= t0) continue;
         const NearList nf{near, nnear, (int)compact_bits(b), (int)compact_bits(b >> 1), n, 0.f};
         auto tpos = [&](int32_t i) { return tgt[i]; };
@@ -756,21 +764,21 @@ __global__ void padded_counts(const int32_t *__restrict__ start, int64_t nleaf,
 }
 
 // Leaf ranges of the 8 XCDs holding equal numbers of targets: split[k]
-// (k = 0..8) is the leaf that holds target k ceil(nt/8), nleaf when there is
-// none.  Launched with nleaf + 1 threads; every entry has one writer.
+// (k = 0..8) is the leaf that holds target k ceil(nt/8); without such a target
+// the end of the last leaf that has any, so no XCD walks the empty leaves
+// behind it (600k blobs in the first 16k of 65k leaves: near field 406 ->
+// 337 us).  Every entry has one writer.
 __global__ void xcd_leaf_split(const int32_t *__restrict__ start, int64_t nleaf,
                                int32_t *__restrict__ split)
 {
     const int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (b > nleaf) return;
+    if (b >= nleaf) return;
     const int64_t nt = start[nleaf];
     const int64_t T = nt > 0 ? (nt + 7) / 8 : 1;
-    if (b == nleaf) {
-        for (int k = 0; k <= 8; ++k)
-            if (k == 8 || k * T >= nt) split[k] = (int32_t)nleaf;
-        return;
-    }
     const int64_t t0 = start[b], t1 = start[b + 1];
+    if (t1 == nt && (t0 < nt || (nt == 0 && b == 0)))
+        for (int k = 0; k <= 8; ++k)
+            if (k == 8 || k * T >= nt) split[k] = nt > 0 ? (int32_t)b + 1 : 0;
     for (int64_t k = (t0 + T - 1) / T; k < 8 && k * T < t1; ++k) split[k] = (int32_t)b;
 }
 
@@ -1367,7 +1375,7 @@ static int run_fmm_typed(Lane *L, const FmmArgs &a, const Domain &dom, const Sor
     // order (beside the far field), then the leaf expansions are added and
     // the outputs written in input order
     const int vout = a.velocity_out ? 1 : 0;
-    const int P = p2p_parts(dom.occupied, (double)a.nt);
+    const int P = p2p_parts(dom.occupied, (double)a.nt, sizeof(T) == 8 ? 1536.0 : 2048.0);
     const uint32_t nl8 = (nleaf * (uint32_t)P + 7) / 8;
     const int32_t *split = Tg.split;  // XCD leaf ranges of the targets
     const int32_t *ts = Tg.start;
@@ -1470,9 +1478,11 @@ static int run_fmm_typed(Lane *L, const FmmArgs &a, const Domain &dom, const Sor
         // P2M
         tm.begin(PHF_STAGE_P2M);
         used[PHF_STAGE_P2M] = true;
-        PHF_TRY(p2m_dispatch(p1, [&](auto ni) {
-            p2m_kernel<T, decltype(ni)::value><<<(nleaf + 3) / 4, 256, 0, L->stream>>>(
-                src, sp, nleaf, p1, dom.org, dom.s, M + off[Lv] * p1);
+        PHF_TRY(p2m_dispatch(p1, (double)a.nb, dom.occupied, [&](auto ni, auto r) {
+            constexpr int R = decltype(r)::value;
+            p2m_kernel<T, decltype(ni)::value, R>
+                <<<(nleaf + 64 / R - 1) / (64 / R), 256, 0, L->stream>>>(
+                    src, sp, nleaf, p1, dom.org, dom.s, 1.0 / dom.s, M + off[Lv] * p1);
         }));
         PHF_HIP(hipGetLastError());
         tm.end(PHF_STAGE_P2M);

@@ -39,10 +39,11 @@ __device__ __forceinline__ int box_count(const int32_t *__restrict__ start, uint
 
 // ----------------------------------------------------------------- P2M --
 // Multipole expansion sum_j w_j ((z_j - c) inv_s)^k, k < p1 <= 4 NI, of the
-// points [s0, s1) by one wave, without LDS.  Lane 4 r + q takes the points
-// j = r (mod 16) and the powers k = q (mod 4): it forms z^q from z and z^2,
-// steps by z^4 through its NI powers and keeps their sums in registers; the
-// sixteen lanes of a power are then added by a butterfly.  Four residues of
+// points [s0, s1) by 4 R lanes of a wave (R = 16 or 4), without LDS.  Lane
+// 4 r + q takes the points j = r (mod R) and the powers k = q (mod 4): it
+// forms z^q from z and z^2, steps by z^4 through its NI powers and keeps their
+// sums in registers; the R lanes of a power are then added by a butterfly.
+// Four residues of
 // k balance the products repeated in every lane of a point (2 squarings, 2
 // selected) against the butterfly (4 steps of NI).  (With a table of
 // 64 x p1 powers in LDS and each column added by one lane, a leaf was a
@@ -52,30 +53,30 @@ __device__ __forceinline__ int box_count(const int32_t *__restrict__ start, uint
 // workgroups there).
 // float32 records are relative to the leaf centre; (cx, cy) is the centre
 // for float64 ones.
-template <class T, int NI>
+template <class T, int NI, int R>
 __device__ __forceinline__ void p2m_leaf(const void *__restrict__ src, int32_t s0, int32_t s1,
                                          double cx, double cy, T inv_s, int p1,
                                          typename C2<T>::type *__restrict__ out)
 {
     using V = typename C2<T>::type;
-    const int lane = threadIdx.x & 63, q = lane & 3, r = lane >> 2;
+    const int lane = threadIdx.x & (4 * R - 1), q = lane & 3, r = lane >> 2;
     V acc[NI];
 #pragma unroll
     for (int i = 0; i < NI; ++i) acc[i] = cmk<T>(0, 0);
-    // the loads of U points go out together (16 U points of the leaf)
+    // the loads of U points go out together (R U points of the leaf)
     constexpr int U = 4;
-    using R = std::conditional_t<sizeof(T) == 4, float4, double4>;
-    const R *rec = reinterpret_cast<const R *>(src);
-    for (int32_t j0 = s0 + r; j0 < s1; j0 += 16 * U) {
-        R pt[U];
+    using Rec = std::conditional_t<sizeof(T) == 4, float4, double4>;
+    const Rec *rec = reinterpret_cast<const Rec *>(src);
+    for (int32_t j0 = s0 + r; j0 < s1; j0 += R * U) {
+        Rec pt[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const int32_t j = j0 + 16 * u;
+            const int32_t j = j0 + R * u;
             pt[u] = rec[j < s1 ? j : s0];
         }
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            if (j0 + 16 * u >= s1) break;
+            if (j0 + R * u >= s1) break;
             V z;
             if (sizeof(T) == 4)
                 z = cmk<T>((T)pt[u].x * inv_s, (T)pt[u].y * inv_s);
@@ -93,36 +94,51 @@ __device__ __forceinline__ void p2m_leaf(const void *__restrict__ src, int32_t s
             }
         }
     }
+    if (__ballot(s1 > s0) == 0) {  // nothing to add up
+#pragma unroll
+        for (int i = 0; i < NI; ++i)
+            if (r == i % R && 4 * i + q < p1) out[4 * i + q] = cmk<T>(0, 0);
+        return;
+    }
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
 #pragma unroll
-        for (int d = 4; d < 64; d <<= 1) {
+        for (int d = 4; d < 4 * R; d <<= 1) {
             acc[i].x += __shfl_xor(acc[i].x, d);
             acc[i].y += __shfl_xor(acc[i].y, d);
         }
         const int k = 4 * i + q;
-        if (r == i && k < p1) out[k] = acc[i];
+        if (r == i % R && k < p1) out[k] = acc[i];
     }
 }
 
 void set_error(const char *fmt, ...) __attribute__((format(printf, 1, 2)));
 
-// f(integral constant NI) for the compiled NI that holds p1 powers
+// f(integral constants NI, R) for the compiled NI that holds p1 powers and the
+// lanes of a leaf: a wave (R = 16), or sixteen lanes (R = 4) where the mean
+// leaf has fewer than 24 points, which a wave takes in little more than one
+// round of its 16 points and then spends on the butterfly.
 template <class F>
-inline int p2m_dispatch(int p1, const F &f)
+inline int p2m_dispatch(int p1, double points, double leaves, const F &f)
 {
+    auto lanes = [&](auto ni) {
+        if (points < 24.0 * leaves)
+            f(ni, std::integral_constant<int, 4>());
+        else
+            f(ni, std::integral_constant<int, 16>());
+    };
     if (p1 <= 12)
-        f(std::integral_constant<int, 3>());
+        lanes(std::integral_constant<int, 3>());
     else if (p1 <= 16)
-        f(std::integral_constant<int, 4>());
+        lanes(std::integral_constant<int, 4>());
     else if (p1 <= 20)
-        f(std::integral_constant<int, 5>());
+        lanes(std::integral_constant<int, 5>());
     else if (p1 <= 24)
-        f(std::integral_constant<int, 6>());
+        lanes(std::integral_constant<int, 6>());
     else if (p1 <= 32)
-        f(std::integral_constant<int, 8>());
+        lanes(std::integral_constant<int, 8>());
     else if (p1 <= 44)
-        f(std::integral_constant<int, 11>());
+        lanes(std::integral_constant<int, 11>());
     else {
         set_error("expansion order %d too large (max 40)", p1 - 1);
         return PHF_ERR_UNSUPPORTED;

@@ -567,7 +567,7 @@ int device_radix_sort_dbits(Lane *L, uint32_t *keys, int32_t *vals, uint32_t *kt
 // start[k] = first position of sorted keys with leaf (key >> fsh) >= k
 // (k = 0..nleaf); with split set, also the leaf ranges of the 8 XCDs
 // holding equal numbers of points: split[j] (j = 0..8) is the leaf of
-// sorted point j ceil(n/8), nleaf when there is none.
+// sorted point j ceil(n/8); without one, the end of the last leaf with points.
 __global__ void leaf_starts_kernel(const uint32_t *__restrict__ skeys, int64_t n, int64_t nleaf,
                                    int fsh, int32_t *__restrict__ start,
                                    int32_t *__restrict__ split)
@@ -575,7 +575,9 @@ __global__ void leaf_starts_kernel(const uint32_t *__restrict__ skeys, int64_t n
     int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (split && k <= 8) {
         const int64_t T = n > 0 ? (n + 7) / 8 : 1;
-        split[k] = (k < 8 && k * T < n) ? (int32_t)(skeys[k * T] >> fsh) : (int32_t)nleaf;
+        split[k] = n <= 0                ? 0
+                   : (k < 8 && k * T < n) ? (int32_t)(skeys[k * T] >> fsh)
+                                          : (int32_t)(skeys[n - 1] >> fsh) + 1;
     }
     if (k > nleaf) return;
     int64_t lo = 0, hi = n;  // first index with leaf >= k

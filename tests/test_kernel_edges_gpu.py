@@ -27,6 +27,24 @@ def test_multipole_orders(order, O):
     assert O.rel_l2(got, ref) <= (r / (2 - r)) ** (order + 1) + 1e-6
 
 
+@pytest.mark.parametrize("order", [2, 12, 19, 31, 40])
+@pytest.mark.parametrize("n", [5, 300, 9001])
+def test_small_and_empty_leaves(n, order, O):
+    """Leaves of few points (sixteen lanes each), most of them empty, among them
+    all the last ones in Morton order; the same bounds as above."""
+    rng = np.random.default_rng(n + order)
+    x, y = 0.3 * rng.random((2, n)) ** 2
+    x[0], y[0], x[1], y[1] = 1.0, 0.0, 0.0, 1.0  # the last quarter holds no point
+    w = rng.standard_normal(n)
+    xopt, cutoff = W.oseen_params(1e-3)
+    ref = O.direct_oseen(x, y, w, x, y, xopt, cutoff)
+    r = 0.5 ** 0.5
+    for prec, eps in ((F64, 1e-12), (F32C, 1e-6)):
+        got = gauss.fmm2d_gpu(x, y, w, x, y, 35, xopt, cutoff, 1e-6, prec=prec, order=order,
+                              leaf=1 if n < 1000 else 8)
+        assert O.rel_l2(got, ref) <= (r / (2 - r)) ** (order + 1) + eps
+
+
 @pytest.mark.parametrize("n", [1, 63, 65, 255, 257, 1025, 2047, 2048, 2049, 70001])
 def test_population_control_chunks(n, O):
     """Chunks of 2048 and waves of 64 blobs at their edges; few, most, all and
