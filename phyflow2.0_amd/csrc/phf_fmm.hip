@@ -79,6 +79,14 @@ __global__ void gather_tgt_f64(const double *__restrict__ x, const double *__res
     out[i] = make_double2(x[j], y[j]);
 }
 
+// The far field's kernels run beside the near field, whose waves keep the
+// vector units busy and which they outlast in small trees: a chain of short
+// kernels of few waves each, issued before the near field's (P2M of 1024 leaves
+// 54 -> 8 us, M2M 28 -> 9; the evaluation of 65k float64 blobs 246 -> 214 us,
+// of 120k float32 ones 179 -> 163; where the near field is the longer, no
+// change).
+__device__ __forceinline__ void far_priority() { __builtin_amdgcn_s_setprio(3); }
+
 // ---------------------------------------------------------------- P2M ----
 // p2m_leaf for 64 / R leaves per workgroup; inv_s is 1 / s.
 template <class T, int NI, int R>
@@ -89,6 +97,7 @@ __global__ __launch_bounds__(256) void p2m_kernel(const void *__restrict__ src,
                                                   double inv_s,
                                                   typename C2<T>::type *__restrict__ M)
 {
+    far_priority();
     const uint32_t b = blockIdx.x * (64 / R) + threadIdx.x / (4 * R);
     if (b >= nleaf) return;
     double cx = 0.0, cy = 0.0;
@@ -97,156 +106,224 @@ __global__ __launch_bounds__(256) void p2m_kernel(const void *__restrict__ src,
 }
 
 // ---------------------------------------------------------- M2M / L2L ----
-// Offset of the centre of descendant c (index within its ancestor's block
-// of 4^D boxes, D levels down) from the ancestor's centre, in units of the
-// ancestor's side (exact dyadic).
-template <class TC>
-__device__ __forceinline__ void descendant_offset(uint32_t c, int D, TC &dx, TC &dy)
-{
-    const uint32_t side = 1u << D;
-    const TC inv = (TC)1 / (TC)side;
-    dx = ((TC)compact_bits(c) + (TC)0.5) * inv - (TC)0.5;
-    dy = ((TC)compact_bits(c >> 1) + (TC)0.5) * inv - (TC)0.5;
-}
-
-// Upward pass over up to three levels in one launch: the multipole
-// expansion of a box at level a (from - nlev <= a < from) is the sum over
-// its 4^(from - a) descendants at level `from`, in Morton order, of
-// M_m += sum_{k <= m} C(m, k) d^(m-k) rho^k M_k (d: descendant centre from
-// the box centre in box units, rho = 2^-(from - a)), the composition of
-// the one-level shifts.  One workgroup per box: the descendants'
-// coefficients (contiguous) and the Pascal triangle are staged in LDS,
-// thread PW j + m sums coefficient m over descendants j, j + NG, ...
-// (NG = 256 / PW groups), and the group partials are added in group
-// order.  Empty boxes have zero expansions, so no box is skipped.
+// Upward pass over up to three levels in one launch: M_m = sum over the four
+// children (sum_{k <= m} C(m, k) d^(m-k) rho^k M_k), d the child's centre from
+// its parent's and rho = 1/2, both in the parent's side.  d = 2^(-3/2) e^(i
+// theta), theta an odd multiple of 45 degrees, so with M'_k = e^(-i theta k)
+// M_k the shift is one real matrix for every child of every box,
+// S[m][k] = C(m, k) 2^(-3 (m - k) / 2) 2^-k, and its result turns back by
+// e^(i theta m): S times the children's real and imaginary parts as columns,
+// on v_mfma_f64_16x16x4f64 (lane l holds A[l % 16][4 s + l / 16],
+// B[4 s + l / 16][l % 16] and, of the result, row 4 v + l / 16, column
+// l % 16; the probe of the layout is the multipole order test).  S stays in
+// registers, its zero tiles are left out; eight children are one tile of
+// columns, so a wave adds four siblings across its lanes.  One workgroup per
+// box of level lev0 takes the levels in turn, in float64 throughout, and keeps
+// the boxes between them in LDS.  Empty boxes have zero expansions, so no box
+// is skipped.
+// (Every level from the finest by complex shifts on the vector units took
+// 192 shifts of 6 p1^2 operations for 64 boxes, against 84 of p1^2 matrix
+// operations: 262k float64 blobs, order 29, beside the near field 57 us for
+// 192 and 45 for 84, and the evaluation 562 -> 515 us, the near field being
+// left the vector units; 600k float32 blobs in 16k leaves 431 -> 405.)
 struct UpLevels {
     int nlev, lev0, from;
-    int64_t blk[4];  // first workgroup of each level
     int64_t off[4];  // coefficient offset (boxes) of each level
     int64_t off_from;
 };
 
-template <class T, class TC, int PW>
-__global__ __launch_bounds__(256) void m2m_multi_kernel(UpLevels u, int p1,
-                                                        typename C2<T>::type *__restrict__ M,
-                                                        const TC *__restrict__ pas)
+typedef double doublex4 __attribute__((ext_vector_type(4)));
+
+// cos and sin of k 45 degrees
+__device__ __forceinline__ void eighth_turns(int k, double &c, double &s)
 {
-    using V = typename C2<T>::type;
-    using W = typename C2<TC>::type;
-    constexpr int NG = 256 / PW;
-    __shared__ V ch[64 * PW];
-    __shared__ W part[NG * PW];
-    __shared__ TC pl[PW * PW];
-    int i = 0;
-    while (i + 1 < u.nlev && (int64_t)blockIdx.x >= u.blk[i + 1]) ++i;
-    const int a = u.lev0 + i, D = u.from - a;
-    const int64_t box = (int64_t)blockIdx.x - u.blk[i];
-    const int tid = threadIdx.x, nd = 1 << (2 * D);
-    const V *src = M + (u.off_from + (box << (2 * D))) * p1;
-    for (int e = tid; e < nd * p1; e += 256) ch[e] = src[e];
-    for (int e = tid; e < p1 * p1; e += 256) pl[e] = pas[e];
-    __syncthreads();
-    const int j = tid / PW, m = tid - j * PW;
-    if (j < NG && m < p1) {
-        W acc = W{0, 0};
-        const TC rho = (TC)1 / (TC)(1u << D), irho = (TC)(1u << D);
-        TC rm = (TC)1;  // rho^m
-        for (int k = 0; k < m; ++k) rm *= rho;
-        for (int c = j; c < nd; c += NG) {
-            TC dx, dy;
-            descendant_offset<TC>((uint32_t)c, D, dx, dy);
-            const V *mc = ch + c * p1;
-            // k = m .. 0: d^(m-k) gains a factor d, rho^k loses one rho
-            TC rk = rm;
-            W dp = W{1, 0};
-            for (int k = m; k >= 0; --k) {
-                const V mk = mc[k];
-                const TC f = pl[m * p1 + k] * rk;
-                const TC tx = f * dp.x, ty = f * dp.y;
-                acc.x += tx * (TC)mk.x - ty * (TC)mk.y;
-                acc.y += tx * (TC)mk.y + ty * (TC)mk.x;
-                const TC nx = dp.x * dx - dp.y * dy;
-                dp.y = dp.x * dy + dp.y * dx;
-                dp.x = nx;
-                rk *= irho;
+    const double h = 0.70710678118654752440;
+    const double m = (k & 1) ? h : 1.0;
+    const int a = (k + 1) & 7, b = (k - 1) & 7;  // cos > 0 in a = 0..2, sin > 0 in b = 0..2
+    c = (k & 3) == 2 ? 0.0 : a < 3 ? m : -m;
+    s = (k & 3) == 0 ? 0.0 : b < 3 ? m : -m;
+}
+
+// S[m][k] of the shifts, 0 outside 0 <= k <= m < p1
+__device__ __forceinline__ double shift_term(const double *__restrict__ pas, int p1, int m, int k)
+{
+    const int n = m - k;
+    if (n < 0 || m >= p1) return 0.0;
+    return ldexp(pas[m * p1 + k] * ((n & 1) ? 1.41421356237309504880 : 1.0),
+                 -((3 * n + 1) >> 1) - k);
+}
+
+// cos and sin of k theta of child q (bit 0: east, bit 1: north)
+__device__ __forceinline__ void child_turn(int q, int k, double &c, double &s)
+{
+    const int turn = (q & 2) ? ((q & 1) ? 1 : 3) : ((q & 1) ? -1 : -3);
+    eighth_turns((turn * k) & 7, c, s);
+}
+
+template <class T, int MT>
+__global__ __launch_bounds__(256) void m2m_kernel(UpLevels u, int p1,
+                                                  typename C2<T>::type *__restrict__ M,
+                                                  const double *__restrict__ pas)
+{
+    far_priority();
+    constexpr int KS = 4 * MT;
+    __shared__ double2 mid[(16 + 4) * 16 * MT];  // the boxes one and two levels up
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int col = lane & 15, kq = lane >> 4, comp = col & 1;
+    double a[MT][KS];
+#pragma unroll
+    for (int t = 0; t < MT; ++t)
+#pragma unroll
+        for (int s = 0; s < 4 * (t + 1); ++s) a[t][s] = shift_term(pas, p1, 16 * t + col, 4 * s + kq);
+    // e^(i theta kq) of the lane's column, its sine signed for the component
+    // that the lane holds; four powers on it turns by 180 degrees
+    const int q = (col >> 1) & 3;
+    double cs, sn;
+    child_turn(q, kq, cs, sn);
+    sn = comp ? sn : -sn;
+    for (int D = 1; D <= u.nlev; ++D) {
+        const int nch = 1 << (2 * (u.nlev - D + 1));  // children in this workgroup
+        const int64_t box0 = (int64_t)blockIdx.x << (2 * (u.nlev - D));  // first parent
+        const typename C2<T>::type *in = M + (u.off_from + 4 * box0) * p1;
+        const double2 *lin = mid + (D == 3 ? 16 * 16 * MT : 0);
+        double2 *lout = mid + (D == 2 ? 16 * 16 * MT : 0);
+        for (int g = wv; 8 * g < nch; g += 4) {
+            const int c = 8 * g + (col >> 1);
+            const bool on = c < nch;
+            doublex4 acc[MT];
+#pragma unroll
+            for (int t = 0; t < MT; ++t) acc[t] = doublex4{0.0, 0.0, 0.0, 0.0};
+            double b[KS];
+#pragma unroll
+            for (int s = 0; s < KS; ++s) {
+                const int k = 4 * s + kq;
+                double v = 0.0;
+                if (on && k < p1)
+                    v = D == 1 ? (double)reinterpret_cast<const T *>(in + (int64_t)c * p1 + k)[comp]
+                               : reinterpret_cast<const double *>(lin + c * 16 * MT + k)[comp];
+                b[s] = v;
             }
+#pragma unroll
+            for (int s = 0; s < KS; ++s) {
+                const double o = __shfl_xor(b[s], 1);
+                b[s] = (s & 1) ? -(b[s] * cs) + o * sn : b[s] * cs - o * sn;
+#pragma unroll
+                for (int t = 0; t < MT; ++t)
+                    if (s < 4 * (t + 1))
+                        acc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[t][s], b[s], acc[t], 0, 0,
+                                                                      0);
+            }
+            typename C2<T>::type *out = M + (u.off[u.nlev - D] + box0 + (c >> 2)) * p1;
+#pragma unroll
+            for (int t = 0; t < MT; ++t)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    const int m = 16 * t + 4 * v + kq;
+                    const double o = __shfl_xor(acc[t][v], 1);
+                    double r = (v & 1) ? -(acc[t][v] * cs) - o * sn : acc[t][v] * cs + o * sn;
+                    r += __shfl_xor(r, 2);
+                    r += __shfl_xor(r, 4);
+                    if (on && q == 0 && m < p1) {
+                        reinterpret_cast<T *>(out + m)[comp] = (T)r;
+                        if (D < u.nlev)
+                            reinterpret_cast<double *>(lout + (c >> 2) * 16 * MT + m)[comp] = r;
+                    }
+                }
         }
-        part[j * PW + m] = acc;
-    }
-    __syncthreads();
-    if (tid < p1) {
-        W acc = part[tid];
-        const int ng = nd < NG ? nd : NG;
-        for (int g = 1; g < ng; ++g) {
-            acc.x += part[g * PW + tid].x;
-            acc.y += part[g * PW + tid].y;
-        }
-        M[(u.off[i] + box) * p1 + tid] = V{(T)acc.x, (T)acc.y};
+        __syncthreads();
     }
 }
 
-// Downward pass in one launch: the local expansion of leaf b gains, for
-// every ancestor level a = 2 .. Lv-1, the ancestor's own (M2L) expansion
-// shifted to the leaf, B_m += rho^m sum_{k >= m} C(k, m) d^(k-m) B_k
-// (d: leaf centre from the ancestor centre in ancestor units,
-// rho = 2^-(Lv - a)), the composition of the one-level shifts, ancestors
-// added from the coarsest.  One workgroup per leaf parent: the shared
-// ancestors' coefficients and the Pascal triangle are staged in LDS,
-// thread PW s + m serves coefficient m of sibling leaf s.
+// Downward pass over up to three levels in one launch: B_m of a child gains
+// rho^m sum_{k >= m} C(k, m) d^(k-m) B_k of its parent, m2m_kernel's turns and
+// the transpose of its matrix.  One workgroup per box of level lev0 takes the
+// levels below it in turn; only the last one's expansions (the next launch's
+// parents, or the leaves) are written.  (Each leaf from all its ancestors on
+// the vector units: 92 us beside the near field of 262k float64 blobs, order
+// 29, against 54, the evaluation 515 -> 477.)
 struct DownLevels {
-    int Lv;
-    int64_t off[13];  // coefficient offset (boxes) of each level
+    int nlev, lev0;
+    int64_t off[4];  // coefficient offset (boxes) of levels lev0 ..
 };
 
-template <class T, class TC, int PW>
-__global__ __launch_bounds__(256) void l2l_leaf_kernel(DownLevels dl, int p1,
-                                                       typename C2<T>::type *__restrict__ B,
-                                                       const TC *__restrict__ pas,
-                                                       const int32_t *__restrict__ start_t)
+template <class T, int MT>
+__global__ __launch_bounds__(256) void l2l_kernel(DownLevels dl, int p1,
+                                                  typename C2<T>::type *__restrict__ B,
+                                                  const double *__restrict__ pas)
 {
-    using V = typename C2<T>::type;
-    using W = typename C2<TC>::type;
-    __shared__ V anc[10 * PW];
-    __shared__ TC pl[PW * PW];
-    const int Lv = dl.Lv, tid = threadIdx.x;
-    const uint32_t q = blockIdx.x;  // leaf parent (level Lv - 1)
-    const int na = Lv - 2;          // ancestor levels 2 .. Lv-1
-    for (int e = tid; e < na * p1; e += 256) {
-        const int ai = e / p1, k = e - ai * p1, a = 2 + ai;
-        anc[e] = B[(dl.off[a] + (q >> (2 * (Lv - 1 - a)))) * p1 + k];
-    }
-    for (int e = tid; e < p1 * p1; e += 256) pl[e] = pas[e];
-    __syncthreads();
-    const int s = tid / PW, m = tid - s * PW;
-    if (s >= 4 || m >= p1) return;
-    const uint32_t b = 4 * q + (uint32_t)s;
-    if (start_t[b + 1] <= start_t[b]) return;
-    W acc = W{0, 0};
-    for (int ai = 0; ai < na; ++ai) {
-        const int D = Lv - (2 + ai);
-        TC dx, dy;
-        descendant_offset<TC>(b & ((1u << (2 * D)) - 1u), D, dx, dy);
-        const V *ba = anc + ai * p1;
-        W sm = W{0, 0}, dp = W{1, 0};
-        for (int k = m; k < p1; ++k) {
-            const V bk = ba[k];
-            const TC f = pl[k * p1 + m];
-            const TC tx = f * dp.x, ty = f * dp.y;
-            sm.x += tx * (TC)bk.x - ty * (TC)bk.y;
-            sm.y += tx * (TC)bk.y + ty * (TC)bk.x;
-            const TC nx = dp.x * dx - dp.y * dy;
-            dp.y = dp.x * dy + dp.y * dx;
-            dp.x = nx;
+    far_priority();
+    constexpr int KS = 4 * MT;
+    __shared__ double2 mid[(4 + 16) * 16 * MT];  // the boxes one and two levels down
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int col = lane & 15, kq = lane >> 4, comp = col & 1;
+    double a[MT][KS];
+#pragma unroll
+    for (int t = 0; t < MT; ++t)
+#pragma unroll
+        for (int s = 4 * t; s < KS; ++s) a[t][s] = shift_term(pas, p1, 4 * s + kq, 16 * t + col);
+    const int q = (col >> 1) & 3;
+    double cs, sn;
+    child_turn(q, kq, cs, sn);
+    sn = comp ? sn : -sn;
+    for (int D = 1; D <= dl.nlev; ++D) {
+        const int nch = 1 << (2 * D);  // children in this workgroup
+        const double2 *lin = mid + (D == 3 ? 4 * 16 * MT : 0);
+        double2 *lout = mid + (D == 2 ? 4 * 16 * MT : 0);
+        for (int g = wv; 8 * g < nch; g += 4) {
+            const int c = 8 * g + (col >> 1);
+            const bool on = c < nch;
+            typename C2<T>::type *out =
+                B + (dl.off[D] + ((int64_t)blockIdx.x << (2 * D)) + (on ? c : 0)) * p1;
+            double b[KS], own[MT][4];
+#pragma unroll
+            for (int s = 0; s < KS; ++s) {
+                const int k = 4 * s + kq;
+                double v = 0.0;
+                if (on && k < p1)
+                    v = D == 1 ? (double)reinterpret_cast<const T *>(
+                                     B + (dl.off[0] + blockIdx.x) * p1 + k)[comp]
+                               : reinterpret_cast<const double *>(lin + (c >> 2) * 16 * MT +
+                                                                  k)[comp];
+                b[s] = v;
+            }
+#pragma unroll
+            for (int t = 0; t < MT; ++t)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    const int m = 16 * t + 4 * v + kq;
+                    own[t][v] =
+                        on && m < p1 ? (double)reinterpret_cast<const T *>(out + m)[comp] : 0.0;
+                }
+            doublex4 acc[MT];
+#pragma unroll
+            for (int t = 0; t < MT; ++t) acc[t] = doublex4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+            for (int s = 0; s < KS; ++s) {
+                const double o = __shfl_xor(b[s], 1);
+                b[s] = (s & 1) ? -(b[s] * cs) - o * sn : b[s] * cs + o * sn;
+#pragma unroll
+                for (int t = 0; t < MT; ++t)
+                    if (s >= 4 * t)
+                        acc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[t][s], b[s], acc[t], 0, 0,
+                                                                      0);
+            }
+#pragma unroll
+            for (int t = 0; t < MT; ++t)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    const int m = 16 * t + 4 * v + kq;
+                    const double o = __shfl_xor(acc[t][v], 1);
+                    const double r = own[t][v] + ((v & 1) ? -(acc[t][v] * cs) + o * sn
+                                                          : acc[t][v] * cs - o * sn);
+                    if (!on || m >= p1) continue;
+                    if (D < dl.nlev)
+                        reinterpret_cast<double *>(lout + c * 16 * MT + m)[comp] = r;
+                    else
+                        reinterpret_cast<T *>(out + m)[comp] = (T)r;
+                }
         }
-        const TC rho = (TC)1 / (TC)(1u << D);
-        TC rm = (TC)1;
-        for (int k = 0; k < m; ++k) rm *= rho;
-        acc.x += rm * sm.x;
-        acc.y += rm * sm.y;
+        __syncthreads();
     }
-    V *bl = B + (dl.off[Lv] + b) * p1;
-    const V cur = bl[m];
-    bl[m] = V{(T)((TC)cur.x + acc.x), (T)((TC)cur.y + acc.y)};
 }
 
 // ---------------------------------------------------------------- M2L ----
@@ -284,6 +361,7 @@ __global__ __launch_bounds__(64) void m2l_kernel(
     const int32_t *__restrict__ il_offs, const typename C2<T>::type *__restrict__ U, int R,
     const T *__restrict__ binom /* [p1][p1] */)
 {
+    far_priority();
     using V = typename C2<T>::type;
     __shared__ V Ap[64];
     const int li = m2l_level_of(lv);
@@ -378,6 +456,7 @@ __global__ __launch_bounds__(64) void m2l_box_kernel(
     const int2 *__restrict__ il_tau, const int32_t *__restrict__ il_offs,
     const typename C2<T>::type *__restrict__ U, int R, const T *__restrict__ binom /* [P1][P1] */)
 {
+    far_priority();
     using V = typename C2<T>::type;
     const int li = m2l_level_of(lv);
     const int l = lv.lev0 + li;
@@ -615,11 +694,11 @@ __global__ void out_scatter_f32(const float4 *__restrict__ src, const int32_t *_
 // the XCD leaf ranges split by target count, written in sorted target
 // order: nsum[i] = (a, b) of target i.  Absolute coordinates and
 // pair_f64's operation order.
-// Three workgroups on a CU (141 VGPRs): held to 128 VGPRs four fit and the
-// kernel alone is faster (262k blobs in leaves of 16: 317 against 459 us), but
-// they fill the registers and the far field beside it waits for them: the
-// evaluation took 585 us against 564.
-__global__ __launch_bounds__(256) void p2p_near_f64s(
+// Held to 128 VGPRs, four workgroups on a CU (141 unbound, three): 1M blobs,
+// 1e-12: the evaluation takes 1520 us against 1563, 120k 289 against 314.
+// (That leaves the far field no registers beside four of them; without its
+// higher priority it fell so far behind that three were the better.)
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void p2p_near_f64s(
     const double4 *__restrict__ src, const int32_t *__restrict__ start_s,
     const double2 *__restrict__ tgt, const int32_t *__restrict__ start_t, int Lvl,
     const int32_t *__restrict__ split, const int2 *__restrict__ near, int nnear, PairParams pp,
@@ -971,67 +1050,24 @@ int fmm_level(int64_t nb, int leaf, int ndirect)
     return std::max(0, std::min(L, 11));
 }
 
-
-
-// Multi-level M2M and leaf L2L launches: thread width PW = the smallest
-// compiled width >= p1.
-template <class T, class TC, int PW>
-static int launch_up(Lane *L, int p1, UpLevels u, void *M, const TC *pas)
+// f(integral constant MT) for the tiles of 16 that hold p1 coefficients
+template <class F>
+static int shift_dispatch(int p1, const F &f)
 {
-    using V = typename C2<T>::type;
-    u.blk[0] = 0;
-    for (int i = 0; i < u.nlev; ++i) u.blk[i + 1] = u.blk[i] + (int64_t(1) << (2 * (u.lev0 + i)));
-    m2m_multi_kernel<T, TC, PW><<<(unsigned)u.blk[u.nlev], 256, 0, L->stream>>>(u, p1, (V *)M,
-                                                                               pas);
+    if (p1 <= 16)
+        f(std::integral_constant<int, 1>());
+    else if (p1 <= 32)
+        f(std::integral_constant<int, 2>());
+    else if (p1 <= 41)
+        f(std::integral_constant<int, 3>());
+    else {
+        set_error("expansion order %d too large (max 40)", p1 - 1);
+        return PHF_ERR_UNSUPPORTED;
+    }
     PHF_HIP(hipGetLastError());
     return PHF_OK;
 }
 
-template <class T, class TC>
-static int shift_up_multi(Lane *L, int p1, const UpLevels &u, void *M, const TC *pas)
-{
-#define PHF_UP(P) \
-    if (p1 <= P) return launch_up<T, TC, P>(L, p1, u, M, pas);
-    PHF_UP(9)
-    PHF_UP(13)
-    PHF_UP(17)
-    PHF_UP(21)
-    PHF_UP(25)
-    PHF_UP(33)
-    PHF_UP(41)
-#undef PHF_UP
-    set_error("expansion order %d too large (max 40)", p1 - 1);
-    return PHF_ERR_UNSUPPORTED;
-}
-
-template <class T, class TC, int PW>
-static int launch_down(Lane *L, int p1, const DownLevels &dl, void *B, const TC *pas,
-                       const int32_t *start)
-{
-    using V = typename C2<T>::type;
-    l2l_leaf_kernel<T, TC, PW><<<(unsigned)(int64_t(1) << (2 * (dl.Lv - 1))), 256, 0,
-                                 L->stream>>>(dl, p1, (V *)B, pas, start);
-    PHF_HIP(hipGetLastError());
-    return PHF_OK;
-}
-
-template <class T, class TC>
-static int shift_down_leaf(Lane *L, int p1, const DownLevels &dl, void *B, const TC *pas,
-                           const int32_t *start)
-{
-#define PHF_DOWN(P) \
-    if (p1 <= P) return launch_down<T, TC, P>(L, p1, dl, B, pas, start);
-    PHF_DOWN(9)
-    PHF_DOWN(13)
-    PHF_DOWN(17)
-    PHF_DOWN(21)
-    PHF_DOWN(25)
-    PHF_DOWN(33)
-    PHF_DOWN(41)
-#undef PHF_DOWN
-    set_error("expansion order %d too large (max 40)", p1 - 1);
-    return PHF_ERR_UNSUPPORTED;
-}
 
 // M2L of every level >= 2 in one launch: the generic coefficient-per-lane
 // kernel (G = 64 / p1 boxes per wave) for any order.
@@ -1201,7 +1237,7 @@ void fmm_plans_release(Lane *L)
 
 // The plan of (a, dom): the lane's own, or a new one.  While a graph is being
 // recorded (spl) the tables go to the recording instead, which owns them.
-template <class T, class TC>
+template <class T>
 static int fmm_plan(Lane *L, const FmmArgs &a, const Domain &dom, const PairParams &pp, bool far,
                     FmmSplit *spl, const FmmPlan **out)
 {
@@ -1211,7 +1247,7 @@ static int fmm_plan(Lane *L, const FmmArgs &a, const Domain &dom, const PairPara
     if (!L->fmm_plans) L->fmm_plans = new FmmPlanCache;
     FmmPlanCache &c = *L->fmm_plans;
     std::vector<uint8_t> key =
-        plan_key(a, dom, (int)(sizeof(T) + 16 * sizeof(TC)), far, shape_log2);
+        plan_key(a, dom, (int)sizeof(T), far, shape_log2);
     if (!spl)
         for (auto &q : c.v)
             if (q->key == key) {
@@ -1239,9 +1275,9 @@ static int fmm_plan(Lane *L, const FmmArgs &a, const Domain &dom, const PairPara
     const int R = pl->R = std::max(ls.R, 1);
     if (far) {
         // Pascal triangle C(m, k) for the multi-level shifts
-        std::vector<TC> pas((size_t)p1 * p1);
+        std::vector<double> pas((size_t)p1 * p1);
         for (int m = 0; m < p1; ++m)
-            for (int k = 0; k < p1; ++k) pas[(size_t)m * p1 + k] = (TC)binom_d(m, k);
+            for (int k = 0; k < p1; ++k) pas[(size_t)m * p1 + k] = binom_d(m, k);
         blob.add(pas, &pl->pas);
         // M2L: binomial rows C(k+m, k) and powers u^k, u = -1/offset
         std::vector<T> bin((size_t)p1 * p1);
@@ -1301,7 +1337,7 @@ static int fmm_plan(Lane *L, const FmmArgs &a, const Domain &dom, const PairPara
     return PHF_OK;
 }
 
-template <class T, class TC>
+template <class T>
 static int run_fmm_typed(Lane *L, const FmmArgs &a, const Domain &dom, const SortedPoints &S, const SortedPoints &Tg, StageTimer &tm,
                          bool *used, FmmInfo *info, FmmSplit *spl, int *nnear_out)
 {
@@ -1344,10 +1380,10 @@ static int run_fmm_typed(Lane *L, const FmmArgs &a, const Domain &dom, const Sor
     std::vector<int64_t> off(Lv + 2, 0);  // level offsets in the coefficient arrays
     for (int l = 0; l <= Lv; ++l) off[l + 1] = off[l] + (int64_t(1) << (2 * l));
     const FmmPlan *pl;
-    PHF_TRY((fmm_plan<T, TC>(L, a, dom, pp, far, spl, &pl)));
+    PHF_TRY(fmm_plan<T>(L, a, dom, pp, far, spl, &pl));
     const int2 *d_near = (const int2 *)pl->near;
     const int nnear = pl->nnear, ninner = pl->ninner;
-    const TC *d_pas = (const TC *)pl->pas;
+    const double *d_pas = (const double *)pl->pas;
     const T *d_bin = (const T *)pl->bin;
     const V *d_U = (const V *)pl->U;
     const int2 *d_il = (const int2 *)pl->il;
@@ -1375,7 +1411,7 @@ static int run_fmm_typed(Lane *L, const FmmArgs &a, const Domain &dom, const Sor
     // order (beside the far field), then the leaf expansions are added and
     // the outputs written in input order
     const int vout = a.velocity_out ? 1 : 0;
-    const int P = p2p_parts(dom.occupied, (double)a.nt, sizeof(T) == 8 ? 1536.0 : 2048.0);
+    const int P = p2p_parts(dom.occupied, (double)a.nt);
     const uint32_t nl8 = (nleaf * (uint32_t)P + 7) / 8;
     const int32_t *split = Tg.split;  // XCD leaf ranges of the targets
     const int32_t *ts = Tg.start;
@@ -1496,7 +1532,10 @@ static int run_fmm_typed(Lane *L, const FmmArgs &a, const Domain &dom, const Sor
             u.from = from;
             u.off_from = off[from];
             for (int i = 0; i < u.nlev; ++i) u.off[i] = off[u.lev0 + i];
-            PHF_TRY((shift_up_multi<T, TC>(L, p1, u, M, d_pas)));
+            PHF_TRY(shift_dispatch(p1, [&](auto mt) {
+                m2m_kernel<T, decltype(mt)::value>
+                    <<<1u << (2 * u.lev0), 256, 0, L->stream>>>(u, p1, M, d_pas);
+            }));
             from -= u.nlev;
         }
         tm.end(PHF_STAGE_M2M);
@@ -1535,11 +1574,17 @@ static int run_fmm_typed(Lane *L, const FmmArgs &a, const Domain &dom, const Sor
         // L2L: every ancestor level shifted straight to the leaves
         tm.begin(PHF_STAGE_L2L);
         used[PHF_STAGE_L2L] = true;
-        if (Lv > 2) {
+        // down to the leaves, three levels per launch, the remainder first
+        for (int lev = 2; lev < Lv;) {
             DownLevels dl{};
-            dl.Lv = Lv;
-            for (int l = 0; l <= Lv; ++l) dl.off[l] = off[l];
-            PHF_TRY((shift_down_leaf<T, TC>(L, p1, dl, B, d_pas, Tg.start)));
+            dl.nlev = (Lv - lev) % 3 ? (Lv - lev) % 3 : 3;
+            dl.lev0 = lev;
+            for (int i = 0; i <= dl.nlev; ++i) dl.off[i] = off[lev + i];
+            PHF_TRY(shift_dispatch(p1, [&](auto mt) {
+                l2l_kernel<T, decltype(mt)::value>
+                    <<<1u << (2 * lev), 256, 0, L->stream>>>(dl, p1, B, d_pas);
+            }));
+            lev += dl.nlev;
         }
         if (far_tail) PHF_TRY(far_tail(L->stream));
         tm.end(PHF_STAGE_L2L);
@@ -1607,12 +1652,9 @@ static int fmm_enqueue(Lane *L, const FmmArgs &a, const Domain &dom_in, StageTim
         PHF_ALLOC(info->d_counts, L->arena, unsigned long long, 2);
         PHF_HIP(hipMemsetAsync(info->d_counts, 0, 2 * sizeof(unsigned long long), L->stream));
     }
-    if (a.prec == PHF_PREC_F32C) {
-        if (a.p > 16)
-            return run_fmm_typed<float, double>(L, a, dom, S, Tg, tm, used, info, spl, nnear);
-        return run_fmm_typed<float, float>(L, a, dom, S, Tg, tm, used, info, spl, nnear);
-    }
-    return run_fmm_typed<double, double>(L, a, dom, S, Tg, tm, used, info, spl, nnear);
+    if (a.prec == PHF_PREC_F32C)
+        return run_fmm_typed<float>(L, a, dom, S, Tg, tm, used, info, spl, nnear);
+    return run_fmm_typed<double>(L, a, dom, S, Tg, tm, used, info, spl, nnear);
 }
 
 // ------------------------------------------------------ captured graphs --

@@ -229,18 +229,15 @@ __device__ __forceinline__ void p2p_part(int32_t &t0, int32_t &t1, int q, int P)
     t1 = min(t1, t0 + len);
 }
 
-// Workgroups per leaf of the near field: enough for `groups` in all (2048:
-// eight on each of the 256 CUs), each with at least two chunks of targets.  With one per leaf, 768
+// Workgroups per leaf of the near field: enough for eight on each of the 256
+// CUs, each with at least two chunks of targets.  With one per leaf, 768
 // leaves of 157 blobs kept the CUs busy for 67% of the kernel (the last leaves
 // run alone); staging a leaf's sources again costs little against its pairs.
 // 120k float64 blobs, 768 leaves: 323 us with one workgroup per leaf, 267 us
 // with two.
-// (float64 leaves are split only to 1536 workgroups, two rounds of the chip's
-// 768: the far field waits behind more of them.  65k blobs, 1024 leaves of 64:
-// the evaluation takes 229 us in two parts, 216 us in one.)
-inline int p2p_parts(double leaves, double targets, double groups)
+inline int p2p_parts(double leaves, double targets)
 {
-    const double want = groups / (leaves > 1.0 ? leaves : 1.0);
+    const double want = 2048.0 / (leaves > 1.0 ? leaves : 1.0);
     const double most = targets / (leaves > 1.0 ? leaves : 1.0) / 32.0;
     const double p = want < most ? want : most;
     return p <= 1.0 ? 1 : p >= 8.0 ? 8 : (int)p;
