@@ -222,10 +222,11 @@ int phf_population_control(const double *x, const double *y, const double *w, in
  *   (src/python/panels/__panelsClass.py:715-822): rows == n is the square
  *   'fixed' system (scipy lu_factor/lu_solve, :961/:782); rows > n is the
  *   'prescribed' least-squares system [A; L] x = [RHS; -gTotal]
- *   (numpy.linalg.lstsq, :800-822).  B is row-major rows x n.  Float32 LU
- *   with partial pivoting (MFMA trailing updates) + float64 iterative
- *   refinement (normal equations with semi-normal float64 residuals when
- *   rows > n).  info may be NULL. */
+ *   (numpy.linalg.lstsq, :800-822).  B is row-major rows x n.  A float32
+ *   factorisation (Cholesky of B^T B; for rows == n also the LU with partial
+ *   pivoting of B, above n = 1024 or where B^T B does not serve) + float64
+ *   iterative refinement (semi-normal float64 residuals when rows > n).  info
+ *   may be NULL. */
 int phf_panel_influence(const double *xCP, const double *yCP, const double *xs,
                         const double *ys, const double *xe, const double *ye,
                         const double *cosA, const double *sinA, int64_t m, double *A);
@@ -335,7 +336,7 @@ int phf_system_get_velocity(phf_system *s, double *vx, double *vy);
  * A phf_panels object holds one panel discretisation (start/end points of m
  * straight vortex panels), its geometry (__panelsClass.py:1036-1058: panel
  * lengths, angles, collocation points CP = mid - 0.1 L n), its influence
- * matrix and the float32 LU factors of A ('fixed') or of the least-squares
+ * matrix and the float32 factors of A ('fixed') or of the least-squares
  * system [A; L] ('prescribed', Kelvin row sum_j L_j s_j = -gTotal) -- the
  * state of the reference's Panels object (__panelsClass.py:446-525). */
 typedef struct phf_panels_s phf_panels;
@@ -356,8 +357,8 @@ int phf_panels_solve(phf_panels *p, const double *vx, const double *vy, double *
 /* Device times (ms) of one rebuild of a panel body. */
 typedef struct {
     double influence_ms; /* influence matrix (+ Kelvin row) */
-    double normal_ms;    /* float64 copies, B^T B for 'prescribed' */
-    double lu_ms;        /* float32 LU with partial pivoting (matrix cores) */
+    double normal_ms;    /* float64 copies, B^T B */
+    double lu_ms;        /* float32 factorisation (matrix cores) */
     double inverse_ms;   /* float32 inverse from the factors */
     double total_ms;     /* all of the above + grouped-velocity factors */
 } phf_panels_timing;

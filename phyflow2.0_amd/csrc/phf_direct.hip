@@ -697,8 +697,8 @@ static int target_order(Lane *L, const double *xt, const double *yt, int64_t nt,
 }
 
 // Source chunks of a direct sum over nt targets in groups of 64 * tpl:
-// enough chunks that the waves fill the chip in whole rounds, each of
-// at least 64 sources (a multiple of 16); one chunk once the target groups
+// enough chunks that the waves fill the chip in whole rounds, each of at least
+// 64 sources (16 in a small sum; a multiple of 16); one chunk once the target groups
 // alone fill the chip.  max_chunks caps the count (the partial sums take
 // nchunk * nt double2).
 static void direct_split(int64_t nt, int tpl, int64_t nb, int64_t *nchunk_out,
@@ -712,8 +712,15 @@ static void direct_split(int64_t nt, int tpl, int64_t nb, int64_t *nchunk_out,
     // waves; 61 chunks of 128 groups, 95% of a round, took 131 us where 64 take
     // 125)
     const int64_t full = 8192;
-    const int64_t most = std::max<int64_t>(
-        1, std::min<int64_t>(std::min<int64_t>(max_chunks, 65535), nb / 64));
+    // A wave takes its sources one after another, some 180 cycles each in
+    // float64, so a call of few waves ends with that chain: down to 16 sources
+    // while there are no more than 2048 waves, two per SIMD (400 x 400 float64
+    // 12.7 -> 9.8 us, 2025 x 2025 14.9 -> 11.2, 3249 x 3249 float32 16.2 ->
+    // 13.4; 4096 waves of 32 sources for 4096 x 4096 float32 took 17.4 against
+    // 15.1 us: the partial sums outweigh it)
+    const int64_t fine = std::max<int64_t>(nb / 64, std::min<int64_t>(nb / 16, 2048 / ngroups));
+    const int64_t most =
+        std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(max_chunks, 65535), fine));
     int64_t nchunk = most;
     if (most * ngroups > full) {
         double best = 0.0;

@@ -26,9 +26,9 @@ size_t lu_work_bytes(int n);
 int chol_factor_f32(Lane *L, float *A32, int n, int32_t *ipiv, int32_t *info, float *dg,
                     float *Lt = nullptr, int ldt = 0);
 
-// Float32 LU factors of B (rows == n), or of B^T B (rows > n: Cholesky in
-// LU form, the pivoted LU if B^T B is not positive definite in float32), and the
-// float32 inverse formed from them, with the float64 column-major copy of B
+// Float32 factors of B^T B (Cholesky in LU form; the pivoted LU if B^T B is not
+// positive definite in float32) or, for a square B of n > 1024 or whose B^T B
+// does not serve, the pivoted LU of B itself, and the float32 inverse formed from them, with the float64 column-major copy of B
 // for refinement residuals (arena-owned).
 struct DenseFactors {
     int64_t rows = 0, n = 0;

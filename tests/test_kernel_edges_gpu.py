@@ -94,6 +94,19 @@ def test_direct_sorted_targets(nb, nt, O):
         assert O.rel_l2([g[sub] for g in got], ref) <= 1e-13
 
 
+@pytest.mark.parametrize("prec,tol", [(F64, 1e-14), (F32C, 1e-6)])
+@pytest.mark.parametrize("nb,nt", [(1, 1), (15, 64), (16, 65), (17, 127), (33, 129), (400, 400),
+                                   (1023, 2025), (2081, 3), (8193, 1), (3249, 3249),
+                                   (5000, 8191), (16384, 16385)])
+def test_direct_source_chunks(nb, nt, prec, tol, O):
+    """Source chunks of 16 and more: remainders of chunks and target groups, one
+    round of waves and the rounds after it."""
+    x, y, w, xt, yt, ks = _flow_and_targets(nb, nt, nb + nt)
+    got = gauss.vv2parGauss_gpu(x, y, w, xt, yt, ks, 128, prec=prec)
+    ref = O.vv2par_gauss(x, y, w, xt, yt, ks)
+    assert O.rel_l2(got, ref) <= tol * max(1.0, (nb / 100) ** 0.5)
+
+
 def test_direct_sorted_degenerate(O):
     """All targets in one point or on a line: one cell, or one row of them."""
     x, y, w, xt, yt, ks = _flow_and_targets(10007, 10007, 5)
