@@ -702,7 +702,7 @@ static int target_order(Lane *L, const double *xt, const double *yt, int64_t nt,
 // alone fill the chip.  max_chunks caps the count (the partial sums take
 // nchunk * nt double2).
 static void direct_split(int64_t nt, int tpl, int64_t nb, int64_t *nchunk_out,
-                         int64_t *chunk_len_out, int64_t max_chunks = 65535)
+                         int64_t *chunk_len_out, int64_t max_chunks = 65535, bool shorten = true)
 {
     const int64_t tblock = (int64_t)kWave * tpl;
     const int64_t ngroups = (nt + tblock - 1) / tblock;
@@ -717,8 +717,10 @@ static void direct_split(int64_t nt, int tpl, int64_t nb, int64_t *nchunk_out,
     // while there are no more than 2048 waves, two per SIMD (400 x 400 float64
     // 12.7 -> 9.8 us, 2025 x 2025 14.9 -> 11.2, 3249 x 3249 float32 16.2 ->
     // 13.4; 4096 waves of 32 sources for 4096 x 4096 float32 took 17.4 against
-    // 15.1 us: the partial sums outweigh it)
-    const int64_t fine = std::max<int64_t>(nb / 64, std::min<int64_t>(nb / 16, 2048 / ngroups));
+    // 15.1 us: the partial sums outweigh it).  Not for the vorticity, whose
+    // pairs are cheaper and whose finish adds a target's parts in one thread.
+    const int64_t fine =
+        shorten ? std::max<int64_t>(nb / 64, std::min<int64_t>(nb / 16, 2048 / ngroups)) : nb / 64;
     const int64_t most =
         std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(max_chunks, 65535), fine));
     int64_t nchunk = most;
@@ -871,7 +873,7 @@ int vorticity_device(Lane *L, int prec, double ksigmasqr, const double *xb, cons
     const int64_t tblock = (int64_t)kWave * tpl;
     const int64_t ngroups = (nt + tblock - 1) / tblock;
     int64_t nchunk, chunk_len;
-    direct_split(nt, tpl, nb, &nchunk, &chunk_len);
+    direct_split(nt, tpl, nb, &nchunk, &chunk_len, 65535, false);
     double *part;
     PHF_ALLOC(part, L->arena, double, (size_t)nchunk * (size_t)nt);
     const dim3 grid((unsigned)ngroups, (unsigned)nchunk);
