@@ -179,6 +179,28 @@ struct LaneGuard {
     }
 };
 
+// The library's device is the thread's current one while this is in scope, and
+// the caller's own again afterwards: for entry points that leave it alone.
+struct DeviceScope {
+    int prev = -1;
+    hipError_t err;
+    DeviceScope()
+    {
+        const int dev = Context::get().device();
+        err = hipGetDevice(&prev);
+        if (err != hipSuccess || prev == dev)
+            prev = -1;
+        else
+            err = hipSetDevice(dev);
+    }
+    ~DeviceScope()
+    {
+        if (prev >= 0) (void)hipSetDevice(prev);
+    }
+    DeviceScope(const DeviceScope &) = delete;
+    DeviceScope &operator=(const DeviceScope &) = delete;
+};
+
 // Per-stage timing with HIP events on the lane's stream; mask selects the
 // stages that are timed (bit s for stage s).
 struct StageTimer {

@@ -298,6 +298,9 @@ struct Piece {  // one transfer into a slot
 
 int copy_out(Lane *L, std::initializer_list<HostOut> out)
 {
+    // events are made and recorded below, which takes the stream's own device
+    DeviceScope ds;
+    PHF_HIP(ds.err);
     size_t total = 0;
     for (const HostOut &o : out) total += o.bytes;
     if (total <= size_t(kPackBytes)) {
