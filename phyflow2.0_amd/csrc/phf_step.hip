@@ -344,6 +344,9 @@ static int panels_rebuild_finish(Panels *P, phf_panels_timing *timing)
     P->pending = false;
     Lane *L = &P->lane;
     hipEvent_t *ev = L->ev;
+    // the pivoted LU may be launched here, also for a caller that only asks
+    DeviceScope ds;
+    PHF_HIP(ds.err);
     PHF_HIP(hipEventSynchronize(P->ev_done));
     if (timing) {
         float a = 0, b = 0, c = 0, d = 0, e = 0;

@@ -61,3 +61,55 @@ def test_results_on_a_thread_of_another_device(H, n):
         assert H.hr_device() == dev
         assert np.array_equal(out, xyw)
     assert H.phf_system_destroy(s) == 0
+
+
+def on_launch(H, **kernels):
+    """kernels: name -> f(args), called for launches whose mangled name holds
+    it; args[i] points to the i-th argument.  Returns what must be kept."""
+    def cb(name, args):
+        for k, f in kernels.items():
+            if k.encode() in name:
+                f(args)
+    c = hostlib.LAUNCH_CB(cb)
+    H.hr_on_launch(c)
+    return c
+
+
+def arg(args, i, t):
+    return ctypes.cast(args[i], ctypes.POINTER(t)).contents
+
+
+def put_i32(args, i, v):
+    """*(int32_t *)argument i = v"""
+    ctypes.c_int32.from_address(arg(args, i, P).value).value = v
+
+
+def ring(m):
+    """Start and end points of m panels on a circle."""
+    t = np.linspace(0.0, 2.0 * np.pi, m + 1)
+    x, y = np.cos(t), np.sin(t)
+    return [np.ascontiguousarray(a) for a in (x[:-1], y[:-1], x[1:], y[1:])]
+
+
+def test_rebuild_completed_on_a_thread_of_another_device(H):
+    """A square body whose normal matrix does not serve takes the pivoted LU
+    when its rebuild is completed, whichever device that thread uses."""
+    bad = [0]
+    keep = on_launch(H, chol_check=lambda a: put_i32(a, 2, bad[0]),
+                     lu_first=lambda a: put_i32(a, 3, 0))
+    m = 40
+    g = ring(m)
+    body = P()
+    assert H.phf_panels_create(*map(ptr, g), ctypes.c_int64(m), 0, ctypes.c_double(0.0),
+                               ctypes.byref(body)) == 0, H.phf_last_error()
+    assert H.hr_launches(b"lu_first") == 0
+    bad[0] = m
+    assert H.phf_panels_update_async(body, *map(ptr, g)) == 0, H.phf_last_error()
+    H.hr_set_device(1)
+    xc, yc = np.empty(m), np.empty(m)
+    rc = H.phf_panels_info(body, None, ptr(xc), ptr(yc), None)
+    assert rc == 0, H.phf_last_error()
+    assert H.hr_device() == 1
+    assert H.hr_launches(b"lu_first") == 1
+    assert H.phf_panels_destroy(body) == 0
+    del keep
