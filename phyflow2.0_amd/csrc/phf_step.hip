@@ -599,20 +599,30 @@ int phf_system_step_rk2(phf_system *h, const phf_vel_params *vp, phf_panels *P,
                               sp->remesh_x0, sp->remesh_y0, sp->remesh_c, &ro,
                               sp->remesh_kernel));
         PHF_TRY(sys_reserve(s, ro.m));
-        s->n = ro.m;
+        s->n = 0;  // until the system's arrays hold the blobs below
+        auto take = [&]() -> int {  // the remeshed blobs as they are
+            if (ro.m > 0)
+                copy3_f64<<<(unsigned)std::min<int64_t>(div_up(ro.m, 256), 4096), 256, 0,
+                            L->stream>>>(ro.x, ro.y, ro.w, ro.m, s->x, s->y, s->w);
+            PHF_HIP(hipGetLastError());
+            s->n = ro.m;
+            return PHF_OK;
+        };
         if (sp->pc_enabled && ro.m > 0) {
             // Blobs.evolve: redistribute, then populationControl
             // (__blobsClass.py:771-781), from the remesh's buffers straight
             // into the system's arrays
             int64_t m = 0;
-            PHF_TRY(population_control_device(L, ro.x, ro.y, ro.w, ro.m, sp->pc_w_threshold,
-                                              sp->pc_total_threshold, s->x, s->y, s->w, &m,
-                                              nullptr));
+            const int rc =
+                population_control_device(L, ro.x, ro.y, ro.w, ro.m, sp->pc_w_threshold,
+                                          sp->pc_total_threshold, s->x, s->y, s->w, &m, nullptr);
+            if (rc != PHF_OK) {
+                (void)take();
+                return rc;
+            }
             s->n = m;
-        } else if (ro.m > 0) {
-            copy3_f64<<<(unsigned)std::min<int64_t>(div_up(ro.m, 256), 4096), 256, 0, L->stream>>>(
-                ro.x, ro.y, ro.w, ro.m, s->x, s->y, s->w);
-            PHF_HIP(hipGetLastError());
+        } else {
+            PHF_TRY(take());
         }
         PHF_TRY(moments_device(L, s->x, s->y, s->w, s->n, dm + 1));
         PHF_HIP(hipMemcpyAsync(&hm[1], dm + 1, sizeof(double4), hipMemcpyDeviceToHost, L->stream));

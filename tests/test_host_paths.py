@@ -113,3 +113,48 @@ def test_rebuild_completed_on_a_thread_of_another_device(H):
     assert H.hr_launches(b"lu_first") == 1
     assert H.phf_panels_destroy(body) == 0
     del keep
+
+
+class RmGeom(ctypes.Structure):
+    """The remesh's layout as phf_remesh.hip has it on the device."""
+    _fields_ = [(k, ctypes.c_int64) for k in
+                ("imin", "imax", "jmin", "jmax", "bi", "bj", "nj", "nstart", "ncell", "nscan",
+                 "m")] + [(k, ctypes.c_int32) for k in ("ok", "bits", "crowded", "pad")]
+
+
+@pytest.mark.parametrize("fail", ["pc_choose", "pc_compact"])
+def test_step_whose_population_control_fails(H, fail):
+    """A coupled step whose population control cannot run ends with an error
+    and leaves the system holding the remeshed blobs."""
+    from phyflow_amd._native import METHOD_DIRECT, StepInfo, StepParams, VelParams
+    n, m = 50, 90
+    new = np.random.default_rng(1).random((3, m))
+
+    def layout(a):
+        g = RmGeom(imin=0, jmin=0, bi=7, bj=7, nj=10, nstart=50, ncell=100, nscan=101, m=m, ok=1)
+        ctypes.memmove(arg(a, 3, P).value, ctypes.byref(g), ctypes.sizeof(g))
+
+    def gather(a):
+        for k in range(3):
+            ctypes.memmove(arg(a, 8 + k, P).value, new[k].ctypes.data, 8 * m)
+
+    def copy3(a):
+        for k in range(3):
+            ctypes.memmove(arg(a, 4 + k, P).value, arg(a, k, P).value,
+                           8 * arg(a, 3, ctypes.c_int64).value)
+
+    keep = on_launch(H, base_bounds_final=layout, gather_cells=gather, copy3_f64=copy3)
+    s, _ = system(H, n)
+    vp = VelParams(METHOD_DIRECT, 0, 0, 0, 0, 35, 0.1, 2.0, 1e-6, 0.0, 0.0)
+    sp = StepParams(dt=0.0, remesh=1, remesh_sigma=0.1, remesh_overlap=1.0, pc_enabled=1,
+                    pc_w_threshold=1e-8, pc_total_threshold=1e-8)
+    H.hr_fail(fail.encode(), 0)
+    rc = H.phf_system_step_rk2(s, ctypes.byref(vp), None, ctypes.byref(sp),
+                               ctypes.byref(StepInfo()))
+    assert rc != 0 and b"OutOfMemory" in H.phf_last_error()
+    size = ctypes.c_int64()
+    assert H.phf_system_size(s, ctypes.byref(size)) == 0 and size.value == m
+    rc, out = get(H, s, m)
+    assert rc == 0 and np.array_equal(out, new)
+    assert H.phf_system_destroy(s) == 0
+    del keep
