@@ -224,16 +224,14 @@ namespace {
 constexpr size_t kSlot = size_t(1) << 20;  // bytes per transfer at most
 constexpr int kSlots = 16;
 constexpr size_t kTask = size_t(128) << 10;  // bytes per thread's copy
-constexpr int kRings = 4;
 // Totals from which results go through a ring; the runtime's own copies are
 // quicker below (three arrays of 720 KB in all: 59 against 70 us; 1.4 MB 89
 // against 95; 2.9 MB 148 against 129; 24 MB 1,405 against 821 us, or 2,767
 // against 980 into fresh memory).
 constexpr size_t kRingBytes = size_t(2) << 20;
 
-// Pinned slots with the events that end their transfers.  At most kRings
-// exist in the process (64 MiB); one is lent to one copy_out at a time, and
-// the second and later ones are freed when they come back.
+// Pinned slots with the events that end their transfers.  One ring exists in
+// the process (16 MiB), made when first needed and kept.
 struct Ring {
     char *ptr = nullptr;
     hipEvent_t ev[kSlots] = {};
@@ -258,34 +256,18 @@ struct Ring {
     }
 };
 
-std::mutex g_ring_mu;
-Ring g_spare;  // the ring that is kept
-int g_rings = 0;
+Ring g_ring;
+std::atomic<int> g_fetches{0};  // results of kRingBytes or more under way
 
-bool ring_take(Ring *r)
-{
-    std::lock_guard<std::mutex> lk(g_ring_mu);
-    if (g_spare.ptr) {
-        *r = g_spare;
-        g_spare = Ring();
-        return true;
-    }
-    if (g_rings >= kRings || !r->make()) return false;
-    ++g_rings;
-    return true;
-}
-
-void ring_give(Ring *r)
-{
-    std::lock_guard<std::mutex> lk(g_ring_mu);
-    if (!g_spare.ptr) {
-        g_spare = *r;
-    } else {
-        r->drop();
-        --g_rings;
-    }
-    *r = Ring();
-}
+// The ring is for a fetch that is alone when it begins.  Threads that fetch at
+// the same time have the runtime's copies side by side, each on its own core,
+// and the workers only get in their way (four threads, 24 MB each: 2.4 ms a
+// fetch by the runtime, 3.1 ms with a ring each, 3.0 with one ring for the
+// first of them).
+struct Fetch {
+    const bool alone = g_fetches.fetch_add(1, std::memory_order_acq_rel) == 0;
+    ~Fetch() { g_fetches.fetch_sub(1, std::memory_order_acq_rel); }
+};
 
 struct Piece {  // one transfer into a slot
     char *host;
@@ -329,14 +311,17 @@ int copy_out(Lane *L, std::initializer_list<HostOut> out)
         }
         return PHF_OK;
     }
-    Ring ring;
-    if (total < kRingBytes || !ring_take(&ring)) {  // or all lent
+    auto plain = [&]() -> int {
         for (const HostOut &o : out)
             if (o.bytes)
                 PHF_HIP(hipMemcpyAsync(o.host, o.dev, o.bytes, hipMemcpyDeviceToHost, L->stream));
         PHF_HIP(hipStreamSynchronize(L->stream));
         return PHF_OK;
-    }
+    };
+    if (total < kRingBytes) return plain();
+    Fetch fetch;
+    if (!fetch.alone || !(g_ring.ptr || g_ring.make())) return plain();
+    const Ring ring = g_ring;
     std::vector<Piece> pc;
     int ntask = 0;
     for (const HostOut &o : out)
@@ -389,9 +374,8 @@ int copy_out(Lane *L, std::initializer_list<HostOut> out)
             send(p + kSlots);
         }
     });
-    // nothing of the ring is in use when it goes back, also after an error
+    // nothing of the ring is in use afterwards, also after an error
     const hipError_t se = hipStreamSynchronize(L->stream);
-    ring_give(&ring);
     PHF_HIP((hipError_t)err.load());
     PHF_HIP(se);
     return PHF_OK;

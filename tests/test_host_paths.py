@@ -2,8 +2,8 @@
 other current devices, failures half way, several threads.  Runs the host code
 itself on the CPU (hostlib.py); no kernel is executed."""
 import ctypes
-import os
 import threading
+import time
 
 import numpy as np
 import pytest
@@ -158,3 +158,37 @@ def test_step_whose_population_control_fails(H, fail):
     assert rc == 0 and np.array_equal(out, new)
     assert H.phf_system_destroy(s) == 0
     del keep
+
+
+def test_concurrent_results_do_not_pin_memory(H):
+    """Several threads that fetch large results at once pin one set of slots
+    between them, free none for the next fetch to pin again, and only the one
+    that pins them waits for it."""
+    n, threads, rounds = 300000, 6, 5
+    systems = [system(H, n, seed=k) for k in range(threads)]
+    barrier = threading.Barrier(threads)
+    pinned, freed = H.hr_calls(b"hipHostMalloc"), H.hr_calls(b"hipHostFree")
+    H.hr_pin_delay_us(200000)
+    bad, waits = [], []
+
+    def work(k):
+        s, xyw = systems[k]
+        for _ in range(rounds):
+            barrier.wait()
+            t = time.perf_counter()
+            rc, out = get(H, s, n)
+            waits.append(time.perf_counter() - t)
+            if rc != 0 or not np.array_equal(out, xyw):
+                bad.append(k)
+
+    ts = [threading.Thread(target=work, args=(k,)) for k in range(threads)]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    assert not bad
+    assert H.hr_calls(b"hipHostMalloc") - pinned <= 1
+    assert H.hr_calls(b"hipHostFree") == freed
+    assert sum(t > 0.15 for t in waits) <= 1
+    for s, _ in systems:
+        assert H.phf_system_destroy(s) == 0
