@@ -136,6 +136,59 @@ def test_vorticity_near(prec, tol, nb, nt, spread, O):
         assert np.all(np.abs(got - ref) <= 750 * 2.0 ** -52 * size + 1e-300)
 
 
+@pytest.mark.parametrize("prec", [F64, F32C])
+def test_vorticity_small_sums(prec, O):
+    """Sums at both ends of the second pass: targets at distances out to where
+    a term is 0 and beyond, alone in their group of 64 and in whole groups; all
+    circulations 0, and circulations whose sizes add up to infinity."""
+    nb, nt = 20011, 40009
+    x, y, w, xt, yt, ks = _flow_and_targets(nb, nt, 11)
+    d = np.sqrt(ks * np.linspace(0.0, 1500.0, 4001))  # right of the unit square
+    xt[:4001], yt[:4001] = 1.0 + d, 0.5
+    xt[5000:5200], yt[5000:5200] = -40.0, 0.5  # beyond every term
+    sub = np.r_[0:4001:7, 5000:5200:9, 6000:nt:97]
+    got = gauss.ww2parGauss_gpu(x, y, w, xt, yt, ks, 128, prec=prec)
+    ref = O.ww2par_gauss(x, y, w, xt[sub], yt[sub], ks)
+    size = O.ww2par_gauss(x, y, np.abs(w), xt[sub], yt[sub], ks)
+    # float32: some 1e-6 of the terms, and of the exponent r2 / ks times the
+    # rounding of r2, until a term leaves float32's normal numbers
+    big = size if prec == F64 else np.maximum(size, 2.0 ** -126 * np.max(size) * nb)
+    tol = 750 * 2.0 ** -52 if prec == F64 else 104 * 2.0 ** -21
+    assert np.all(np.abs(got[sub] - ref) <= tol * big + (1e-300 if prec == F64 else 0.0))
+    assert not got[5000:5200].any()
+    assert not gauss.ww2parGauss_gpu(x, y, 0 * w, xt, yt, ks, 128, prec=prec).any()
+    if prec == F64:
+        big = np.where(np.arange(nb) % 2 == 0, 2e304, -2e304)
+        got = gauss.ww2parGauss_gpu(x, y, big, xt, yt, ks, 128)[sub]
+        size = O.ww2par_gauss(x, y, np.full(nb, 1.0), xt[sub], yt[sub], ks)
+        ref = O.ww2par_gauss(x, y, big * 5e-305, xt[sub], yt[sub], ks)
+        fits = np.abs(ref) < 8e3  # of a value in float64
+        assert np.count_nonzero(fits) > 0.9 * fits.size
+        assert np.all((np.abs(got * 5e-305 - ref) <= 1e-12 * size + 1e-300)[fits])
+
+
+@pytest.mark.parametrize("prec", [F64, F32C])
+def test_vorticity_beyond_the_flow_is_not_the_whole_sum(prec):
+    """A grid that reaches beyond the blobs takes longer than one among them,
+    but not as long as every pair would (some fifteen times)."""
+    import time
+    nb, nt = 100003, 90601
+    x, y, w, xt, yt, ks = _flow_and_targets(nb, nt, 3)
+
+    def t(sx, ox):
+        a, b = xt * sx + ox, yt * sx + (1.0 - sx) / 2
+        runs = []
+        for _ in range(7):
+            t0 = time.perf_counter()
+            gauss.ww2parGauss_gpu(x, y, w, a, b, ks, 128, prec=prec)
+            runs.append(time.perf_counter() - t0)
+        return sorted(runs)[3]
+
+    inside = t(1.0, 0.0)
+    assert t(2.0, -0.5) <= 5.0 * inside
+    assert t(1.0, 2.0) <= 2.0 * inside
+
+
 @pytest.mark.parametrize("n", [1, 5461, 5462, 87381, 87382, 131072, 131073, 800001])
 def test_blobs_come_back_whole(n):
     """Results by one packed transfer, by the runtime's copies and through the
