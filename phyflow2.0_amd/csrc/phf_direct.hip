@@ -739,14 +739,35 @@ __global__ __launch_bounds__(256) void zero_part(double2 *__restrict__ part, int
 
 constexpr int DIRECT_TPL32 = 2, DIRECT_TPL64 = 1;
 
-// Pairs from which a float64 velocity sum sorts its targets (six launches,
-// some 45 us).  Call with its kernels, unsorted against sorted: 6.4e7 pairs
-// 91 against 97 us, 1.4e8 193 against 149, 6e8 731 against 439.
-constexpr double kSortPairs = 1e8;
-// Pairs from which the vorticity takes near sources only (a dozen launches).
-// Whole calls: float64 1.1e8 pairs 257 against 222 us, 8e8 1045 against 338;
-// float32 pairs cost less, 1.4e8 192 against 215 us, 8e8 425 against 285.
-constexpr double kNearPairs64 = 1e8, kNearPairs32 = 4e8;
+// Whether a float64 velocity sum sorts its targets (six launches, some 45 us,
+// and 0.1 ns a target): from 1e8 pairs, and enough sources that most are
+// outside a target's smoothing and a target's saving is more than its sort.
+// Call with its kernels, unsorted against sorted: 6.4e7 pairs 91 against 97 us,
+// 1.4e8 193 against 149, 6e8 731 against 439; 800 sources x 625,000 targets
+// 1,349 against 1,380 us, 1,600 x 312,500 997 against 987, 3,200 x 156,250 835
+// against 769; 100 x 1.1M 1,400 against 1,493.  Few targets sort at no cost:
+// 250,000 x 2,000 943 against 672 us.
+static bool sort_pays(int64_t nb, int64_t nt)
+{
+    return (double)nb * (double)nt >= 1e8 && nb >= 2048;
+}
+
+// Whether the vorticity takes near sources only (a dozen launches, two sorts):
+// from 1e8 pairs, in float32, whose pairs cost less, from 4e8, and more where
+// the sides are uneven, since either is sorted and few points make no compact
+// groups.  Whole calls, every pair against near sources, float64: 1.1e8 pairs
+// 257 against 222 us, 8e8 1,045 against 338; 400 sources x 275,000 targets 448
+// against 531, 800 x 625,000 1,020 against 959, 220,000 x 500 433 against 488,
+// 1M x 500 1,408 against 1,306.  float32: 1.4e8 192 against 215, 8e8 425
+// against 285; 1,600 x 312,500 490 against 533, 3,200 x 312,500 626 against
+// 574, 1M x 500 1,138 against 1,300, 250,000 x 2,000 586 against 492.
+static bool near_pays(int prec, int64_t nb, int64_t nt)
+{
+    const double pairs = (double)nb * (double)nt;
+    if (prec == PHF_PREC_F64)
+        return pairs >= 1e8 && pairs * (double)std::min(nb, nt) >= 2.2e11;
+    return pairs >= 4e8 && pairs * std::min((double)nb / 3.0, (double)nt) >= 5.4e11;
+}
 
 // Enqueue the pair kernel and the finishing kernel on stream st with the
 // partial sums in part (nchunk * nt double2; nchunk, chunk_len from
@@ -794,7 +815,7 @@ static int launch_direct(Lane *L, int prec, const PairParams &pp, const double *
     PHF_ALLOC(part, L->arena, double2, (size_t)nchunk * (size_t)nt);
     int32_t *perm = nullptr;
     if (prec == PHF_PREC_F64 && KIND != PAIR_CUTOFF && nt < (int64_t(1) << 31) &&
-        (double)nb * (double)nt >= kSortPairs) {
+        sort_pays(nb, nt)) {
         double4 *bb;
         PHF_ALLOC(bb, L->arena, double4, 1);
         PHF_TRY(device_bbox(L, xt, yt, nt, nullptr, nullptr, 0, bb));
@@ -855,8 +876,7 @@ int vorticity_device(Lane *L, int prec, double ksigmasqr, const double *xb, cons
         pp.eps = ksigmasqr;
         pp.eps_f = (float)ksigmasqr;
     }
-    if (!cutoff && nb < (int64_t(1) << 31) && nt < (int64_t(1) << 31) &&
-        (double)nb * (double)nt >= (prec == PHF_PREC_F64 ? kNearPairs64 : kNearPairs32))
+    if (!cutoff && nb < (int64_t(1) << 31) && nt < (int64_t(1) << 31) && near_pays(prec, nb, nt))
         return vorticity_near(L, prec, ksigmasqr, pp, xb, yb, wb, nb, xt, yt, nt, w);
     constexpr int TPL32 = 2, TPL64 = 1;
     const int tpl = prec == PHF_PREC_F32C ? TPL32 : TPL64;

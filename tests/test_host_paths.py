@@ -192,3 +192,36 @@ def test_concurrent_results_do_not_pin_memory(H):
     assert sum(t > 0.15 for t in waits) <= 1
     for s, _ in systems:
         assert H.phf_system_destroy(s) == 0
+
+
+@pytest.mark.parametrize("nb,nt,prec,sort,near", [
+    (10007, 10007, 0, 1, 1),     # even sides, 1e8 pairs
+    (9000, 9000, 0, 0, 0),       # fewer
+    (20011, 20011, 1, 0, 1),
+    (19000, 19000, 1, 0, 0),
+    (50, 2100000, 0, 0, 0),      # few sources: the targets' sort is the call
+    (400, 275000, 0, 0, 0),
+    (1600, 68750, 0, 0, 0),
+    (3200, 156250, 0, 1, 1),
+    (1600, 312500, 1, 0, 0),
+    (3200, 312500, 1, 0, 1),
+    (1100000, 100, 0, 1, 0),     # few targets: theirs is quick, the sources' is not
+    (220000, 500, 0, 1, 0),
+    (800000, 600, 1, 0, 0),
+    (250000, 2000, 1, 0, 1),
+])
+def test_which_direct_sums_sort(H, nb, nt, prec, sort, near):
+    """Direct sums sort their targets, and vorticity its sources too, where
+    the pairs saved are more than the sorts cost."""
+    r = np.random.default_rng(0)
+    b, t, o = r.random((3, nb)), r.random((2, nt)), np.empty((2, nt))
+    n = [H.hr_launches(k) for k in (b"direct_f64_sorted", b"rs_scatter", b"vort_near")]
+    args = [ptr(b[0]), ptr(b[1]), ptr(b[2]), ctypes.c_int64(nb), ptr(t[0]), ptr(t[1]),
+            ctypes.c_int64(nt), ctypes.c_double(1e-4), ctypes.c_int32(prec)]
+    assert H.phf_vv2par_gauss(*args, ptr(o[0]), ptr(o[1])) == 0, H.phf_last_error()
+    assert (H.hr_launches(b"direct_f64_sorted") > n[0]) == bool(sort)
+    assert (H.hr_launches(b"rs_scatter") > n[1]) == bool(sort)
+    n[1] = H.hr_launches(b"rs_scatter")
+    assert H.phf_ww2par_gauss(*args, ptr(o[0])) == 0, H.phf_last_error()
+    assert (H.hr_launches(b"vort_near") > n[2]) == bool(near)
+    assert (H.hr_launches(b"rs_scatter") > n[1]) == bool(near)
