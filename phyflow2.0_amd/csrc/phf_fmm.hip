@@ -1004,15 +1004,11 @@ struct TableBlob {
         if (!v.empty()) std::memcpy(host.data() + at, v.data(), sizeof(T) * v.size());
         fix.push_back({at, d});
     }
-    // To a device buffer of their own, handed to *keep, copied on stream st;
-    // wait: the copy is complete on return (launches being recorded into a
-    // graph then hold no copy), else it is ordered on st.
-    int send(Lane *L, char **keep, hipStream_t st, bool wait)
+    // To dev (at least host.size() bytes) on stream st; wait: the copy is
+    // complete on return (launches being recorded into a graph then hold no
+    // copy), else it is ordered on st.
+    int send(Lane *L, char *dev, hipStream_t st, bool wait)
     {
-        if (host.empty()) return PHF_OK;
-        char *dev;
-        PHF_HIP(hipMalloc(&dev, host.size()));
-        *keep = dev;
         if (wait) {
             PHF_HIP(hipMemcpyAsync(dev, host.data(), host.size(), hipMemcpyHostToDevice, st));
             PHF_HIP(hipStreamSynchronize(st));
@@ -1181,7 +1177,8 @@ static int fmm_near(Lane *L, const P2PLaunch &near, StageTimer &tm)
 // 120k blobs).
 struct FmmPlan {
     std::vector<uint8_t> key;
-    char *dev = nullptr;
+    char *dev = nullptr;  // the tables, cap bytes; null: in the arena or a graph's
+    size_t cap = 0;
     void *near = nullptr, *pas = nullptr, *bin = nullptr, *U = nullptr, *il = nullptr,
          *iloff = nullptr;
     int nnear = 0, ninner = 0, R = 1;
@@ -1193,6 +1190,7 @@ FmmSplit::~FmmSplit() = default;
 
 struct FmmPlanCache {
     std::vector<std::unique_ptr<FmmPlan>> v;
+    std::unique_ptr<FmmPlan> once;  // of the current call only, in the arena
     uint64_t clock = 0;
 };
 
@@ -1310,30 +1308,61 @@ static int fmm_plan(Lane *L, const FmmArgs &a, const Domain &dom, const PairPara
         blob.add(il_all, &pl->il);
         blob.add(il_offs, &pl->iloff);
     }
+    const size_t need = blob.host.size();
     if (spl) {
-        PHF_TRY(blob.send(L, spl->tables_keep, spl->side, true));
+        char *dev;
+        PHF_HIP(hipMalloc(&dev, need));
+        *spl->tables_keep = dev;
+        PHF_TRY(blob.send(L, dev, spl->side, true));
         spl->plan = std::move(pl);
         *out = spl->plan.get();
         return PHF_OK;
     }
+    // The least recently used plan makes room, and its buffer serves the new
+    // one if it is large enough: the copy below follows, on the lane's stream,
+    // every launch that reads it (a call's far field is joined to that stream).
+    // So more shapes in turn than are kept cost their tables' transfer, and
+    // neither wait for the device nor allocate.
     if (c.v.size() >= kPlans) {
         auto lru = std::min_element(c.v.begin(), c.v.end(), [](const auto &x, const auto &y) {
             return x->last < y->last;
         });
-        PHF_TRY(lane_quiesce(L));  // launches in flight may still read its tables
-        if ((*lru)->dev) (void)hipFree((*lru)->dev);
+        if ((*lru)->cap < need) {
+            PHF_TRY(lane_quiesce(L));
+            (void)hipFree((*lru)->dev);
+        } else {
+            pl->dev = (*lru)->dev;
+            pl->cap = (*lru)->cap;
+        }
         c.v.erase(lru);
+    }
+    if (!pl->dev) {
+        size_t cap = size_t(64) << 10;
+        while (cap < need) cap *= 2;
+        if (hipMalloc(&pl->dev, cap) == hipSuccess) {
+            pl->cap = cap;
+        } else {  // no memory beyond the arena's
+            (void)hipGetLastError();
+            pl->dev = nullptr;
+        }
+    }
+    if (!pl->dev) {
+        char *dev;
+        PHF_ALLOC(dev, L->arena, char, need);
+        PHF_TRY(blob.send(L, dev, L->stream, false));
+        c.once = std::move(pl);
+        *out = c.once.get();
+        return PHF_OK;
+    }
+    const int rc = blob.send(L, pl->dev, L->stream, false);
+    if (rc != PHF_OK) {
+        (void)lane_quiesce(L);
+        (void)hipFree(pl->dev);
+        return rc;
     }
     pl->last = ++c.clock;
     c.v.push_back(std::move(pl));
-    FmmPlan *q = c.v.back().get();
-    const int rc = blob.send(L, &q->dev, L->stream, false);
-    if (rc != PHF_OK) {
-        if (q->dev) (void)hipFree(q->dev);
-        c.v.pop_back();
-        return rc;
-    }
-    *out = q;
+    *out = c.v.back().get();
     return PHF_OK;
 }
 

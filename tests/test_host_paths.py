@@ -225,3 +225,55 @@ def test_which_direct_sums_sort(H, nb, nt, prec, sort, near):
     assert H.phf_ww2par_gauss(*args, ptr(o[0])) == 0, H.phf_last_error()
     assert (H.hr_launches(b"vort_near") > n[2]) == bool(near)
     assert (H.hr_launches(b"rs_scatter") > n[1]) == bool(near)
+
+
+def fmm(H, n, order):
+    """One fmm2d call of n blobs in the unit square at an expansion order."""
+    from phyflow_amd._native import FmmOpts
+    r = np.random.default_rng(n).random((3, n))
+    o = np.empty((2, n))
+    return H.phf_fmm2d(ptr(r[0]), ptr(r[1]), ptr(r[2]), ctypes.c_int64(n), ptr(r[0]), ptr(r[1]),
+                       ctypes.c_int64(n), 35, ctypes.c_double(0.01), ctypes.c_double(0.05),
+                       ctypes.c_double(1e-6), ctypes.byref(FmmOpts(order, 32, 0, 0)), ptr(o[0]),
+                       ptr(o[1]))
+
+
+def unit_box(a):
+    """What bbox_final writes for points in the unit square."""
+    box = np.array([0.0, 1.0, 0.0, 1.0])
+    ctypes.memmove(arg(a, 2, P).value, box.ctypes.data, 32)
+
+
+def test_more_tree_shapes_than_a_lane_keeps(H):
+    """Calls that take more tree shapes in turn than a lane keeps the tables of
+    neither allocate nor free, nor wait for the device more than a call whose
+    tables are there."""
+    keep = on_launch(H, bbox_final=unit_box)
+    names = (b"hipMalloc", b"hipFree", b"hipStreamSynchronize")
+
+    def calls(orders):
+        n = [H.hr_calls(k) for k in names]
+        for p in orders:
+            assert fmm(H, 4000, p) == 0, H.phf_last_error()
+        return [H.hr_calls(k) - a for k, a in zip(names, n)]
+
+    shapes = [6, 17, 9, 30, 12, 21, 7, 24, 14]
+    for _ in range(4):
+        calls(shapes)
+    kept = calls([shapes[-1]] * len(shapes))
+    assert kept[:2] == [0, 0]
+    assert calls(shapes) == kept
+    del keep
+
+
+def test_tables_without_memory_beyond_the_arena(H):
+    """A new tree shape needs no more device memory than the call's workspace:
+    its tables go there when they cannot have a buffer of their own."""
+    keep = on_launch(H, bbox_final=unit_box)
+    assert fmm(H, 4000, 35) == 0, H.phf_last_error()
+    for p in range(25, 35):
+        H.hr_fail(b"hipMalloc", 0)
+        assert fmm(H, 4000, p) == 0, H.phf_last_error()
+    H.hr_fail(b"", -1)
+    assert fmm(H, 4000, 36) == 0, H.phf_last_error()
+    del keep
