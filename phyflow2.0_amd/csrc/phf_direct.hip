@@ -816,10 +816,18 @@ static int launch_direct(Lane *L, int prec, const PairParams &pp, const double *
     int32_t *perm = nullptr;
     if (prec == PHF_PREC_F64 && KIND != PAIR_CUTOFF && nt < (int64_t(1) << 31) &&
         sort_pays(nb, nt)) {
-        double4 *bb;
-        PHF_ALLOC(bb, L->arena, double4, 1);
-        PHF_TRY(device_bbox(L, xt, yt, nt, nullptr, nullptr, 0, bb));
-        PHF_TRY(target_order(L, xt, yt, nt, bb, &perm));
+        const int rc = [&]() -> int {
+            double4 *bb;
+            PHF_ALLOC(bb, L->arena, double4, 1);
+            PHF_TRY(device_bbox(L, xt, yt, nt, nullptr, nullptr, 0, bb));
+            return target_order(L, xt, yt, nt, bb, &perm);
+        }();
+        if (rc == PHF_ERR_NOMEM) {  // no room for the sort: the targets as they are
+            clear_error();
+            perm = nullptr;
+        } else {
+            PHF_TRY(rc);
+        }
     }
     return enqueue_direct<KIND>(L->stream, prec, pp, xb, yb, wb, nb, xt, yt, nt, nchunk,
                                 chunk_len, part, o0, o1, perm);
@@ -876,8 +884,14 @@ int vorticity_device(Lane *L, int prec, double ksigmasqr, const double *xb, cons
         pp.eps = ksigmasqr;
         pp.eps_f = (float)ksigmasqr;
     }
-    if (!cutoff && nb < (int64_t(1) << 31) && nt < (int64_t(1) << 31) && near_pays(prec, nb, nt))
-        return vorticity_near(L, prec, ksigmasqr, pp, xb, yb, wb, nb, xt, yt, nt, w);
+    if (!cutoff && nb < (int64_t(1) << 31) && nt < (int64_t(1) << 31) && near_pays(prec, nb, nt)) {
+        const Arena::Mark m0 = L->arena.mark();
+        const int rc = vorticity_near(L, prec, ksigmasqr, pp, xb, yb, wb, nb, xt, yt, nt, w);
+        if (rc != PHF_ERR_NOMEM) return rc;
+        // no room for its workspace: every pair
+        L->arena.jump(L->arena.mark(), m0);
+        clear_error();
+    }
     constexpr int TPL32 = 2, TPL64 = 1;
     const int tpl = prec == PHF_PREC_F32C ? TPL32 : TPL64;
     const int64_t tblock = (int64_t)kWave * tpl;

@@ -2,6 +2,7 @@
 other current devices, failures half way, several threads.  Runs the host code
 itself on the CPU (hostlib.py); no kernel is executed."""
 import ctypes
+import shutil
 import threading
 import time
 
@@ -18,10 +19,25 @@ def ptr(a):
 
 
 @pytest.fixture(scope="module")
-def H(tmp_path_factory):
-    h = hostlib.load(hostlib.build(str(tmp_path_factory.mktemp("hostlib"))))
+def libpath(tmp_path_factory):
+    return hostlib.build(str(tmp_path_factory.mktemp("hostlib")))
+
+
+def opened(path):
+    h = hostlib.load(path)
     assert h.phf_init() == 0, h.phf_last_error()
     return h
+
+
+@pytest.fixture(scope="module")
+def H(libpath):
+    return opened(libpath)
+
+
+@pytest.fixture
+def fresh(libpath, tmp_path):
+    """The library with nothing allocated yet."""
+    return opened(shutil.copy(libpath, tmp_path / "fresh.so"))
 
 
 @pytest.fixture(autouse=True)
@@ -213,16 +229,12 @@ def test_concurrent_results_do_not_pin_memory(H):
 def test_which_direct_sums_sort(H, nb, nt, prec, sort, near):
     """Direct sums sort their targets, and vorticity its sources too, where
     the pairs saved are more than the sorts cost."""
-    r = np.random.default_rng(0)
-    b, t, o = r.random((3, nb)), r.random((2, nt)), np.empty((2, nt))
     n = [H.hr_launches(k) for k in (b"direct_f64_sorted", b"rs_scatter", b"vort_near")]
-    args = [ptr(b[0]), ptr(b[1]), ptr(b[2]), ctypes.c_int64(nb), ptr(t[0]), ptr(t[1]),
-            ctypes.c_int64(nt), ctypes.c_double(1e-4), ctypes.c_int32(prec)]
-    assert H.phf_vv2par_gauss(*args, ptr(o[0]), ptr(o[1])) == 0, H.phf_last_error()
+    assert direct(H, nb, nt, "velocity", prec) == 0, H.phf_last_error()
     assert (H.hr_launches(b"direct_f64_sorted") > n[0]) == bool(sort)
     assert (H.hr_launches(b"rs_scatter") > n[1]) == bool(sort)
     n[1] = H.hr_launches(b"rs_scatter")
-    assert H.phf_ww2par_gauss(*args, ptr(o[0])) == 0, H.phf_last_error()
+    assert direct(H, nb, nt, "vorticity", prec) == 0, H.phf_last_error()
     assert (H.hr_launches(b"vort_near") > n[2]) == bool(near)
     assert (H.hr_launches(b"rs_scatter") > n[1]) == bool(near)
 
@@ -277,3 +289,28 @@ def test_tables_without_memory_beyond_the_arena(H):
     H.hr_fail(b"", -1)
     assert fmm(H, 4000, 36) == 0, H.phf_last_error()
     del keep
+
+
+def direct(H, nb, nt, field, prec=0):
+    r = np.random.default_rng(0)
+    b, t, o = r.random((3, nb)), r.random((2, nt)), np.empty((2, nt))
+    args = [ptr(b[0]), ptr(b[1]), ptr(b[2]), ctypes.c_int64(nb), ptr(t[0]), ptr(t[1]),
+            ctypes.c_int64(nt), ctypes.c_double(1e-4), ctypes.c_int32(prec)]
+    if field == "velocity":
+        return H.phf_vv2par_gauss(*args, ptr(o[0]), ptr(o[1]))
+    return H.phf_ww2par_gauss(*args, ptr(o[0]))
+
+
+@pytest.mark.parametrize("field,nt", [("velocity", 800000), ("vorticity", 2400000)])
+def test_direct_sum_without_memory_for_its_sort(fresh, field, nt):
+    """A sum that would sort, but finds the device's memory taken (its second
+    block here), is done as it comes."""
+    H = fresh
+    H.hr_fail(b"hipMalloc", 1)
+    assert direct(H, 2100, nt, field) == 0, H.phf_last_error()
+    assert H.phf_last_error() == b""
+    assert H.hr_launches(b"direct_f64_sorted") + H.hr_launches(b"vort_near") == 0
+    assert H.hr_calls(b"hipMalloc") == (2 if field == "velocity" else 3)
+    # with room it does sort
+    assert direct(H, 2100, nt, field) == 0, H.phf_last_error()
+    assert H.hr_launches(b"direct_f64_sorted") + H.hr_launches(b"vort_near") > 0
