@@ -21,14 +21,15 @@ namespace {
 constexpr int kWorkers = 6;
 
 struct Job {
-    const std::function<void(int)> *fn;
+    void (*fn)(void *, int);
+    void *ctx;
     int n;
     std::atomic<int> next{0}, done{0};
     // takes tasks until none is left
     void work()
     {
         int mine = 0;
-        for (int i; (i = next.fetch_add(1, std::memory_order_relaxed)) < n; ++mine) (*fn)(i);
+        for (int i; (i = next.fetch_add(1, std::memory_order_relaxed)) < n; ++mine) fn(ctx, i);
         if (mine) done.fetch_add(mine, std::memory_order_release);
     }
 };
@@ -43,7 +44,7 @@ class Workers {
         static Workers *w = new Workers();
         return *w;
     }
-    void run(const std::shared_ptr<Job> &job)
+    void add(const std::shared_ptr<Job> &job)
     {
         {
             std::lock_guard<std::mutex> lk(mu_);
@@ -52,7 +53,10 @@ class Workers {
             pending_.fetch_add(1, std::memory_order_release);
         }
         cv_.notify_all();
-        job->work();
+    }
+    // takes the job, whose tasks are all taken, off the list and waits for them
+    void finish(const std::shared_ptr<Job> &job)
+    {
         {
             std::lock_guard<std::mutex> lk(mu_);
             for (size_t i = 0; i < jobs_.size(); ++i)
@@ -119,16 +123,25 @@ class Workers {
 
 }  // namespace
 
-void host_parallel(int n, const std::function<void(int)> &fn)
+void host_parallel(int n, void (*fn)(void *, int), void *ctx)
 {
     if (n <= 1) {
-        if (n == 1) fn(0);
+        if (n == 1) fn(ctx, 0);
         return;
     }
-    auto job = std::make_shared<Job>();
-    job->fn = &fn;
-    job->n = n;
-    Workers::get().run(job);
+    std::shared_ptr<Job> job;
+    try {
+        job = std::make_shared<Job>();
+        job->fn = fn;
+        job->ctx = ctx;
+        job->n = n;
+        Workers::get().add(job);
+    } catch (...) {  // no memory for it: the caller works alone
+        for (int i = 0; i < n; ++i) fn(ctx, i);
+        return;
+    }
+    job->work();
+    Workers::get().finish(job);
 }
 
 // ------------------------------------------------------------- validation --
@@ -178,14 +191,22 @@ int check_host_array(const double *p, int64_t n, const char *name, bool finite)
 // and the pack is one thread's copy.
 static constexpr int64_t kPackBytes = 128 << 10;
 
+// whether the lane has its staging (no memory left to pin: the runtime's copies)
+static bool have_pin(Lane *L)
+{
+    if (L->pin.ensure(kPackBytes) == PHF_OK) return true;
+    (void)hipGetLastError();
+    clear_error();
+    return false;
+}
+
 int copy_in(Lane *L, std::initializer_list<HostIn> in)
 {
     int64_t total = 0;
     for (const HostIn &a : in) total += a.n > 0 ? a.n : 1;
     double *d;
     PHF_ALLOC(d, L->arena, double, (size_t)total);
-    const bool pack = total * (int64_t)sizeof(double) <= kPackBytes;
-    if (pack) PHF_TRY(L->pin.ensure(kPackBytes));
+    const bool pack = total * (int64_t)sizeof(double) <= kPackBytes && have_pin(L);
     double *pin = reinterpret_cast<double *>(L->pin.ptr);
     int64_t at = 0;
     for (const HostIn &a : in) {
@@ -285,8 +306,15 @@ int copy_out(Lane *L, std::initializer_list<HostOut> out)
     PHF_HIP(ds.err);
     size_t total = 0;
     for (const HostOut &o : out) total += o.bytes;
+    auto plain = [&]() -> int {
+        for (const HostOut &o : out)
+            if (o.bytes)
+                PHF_HIP(hipMemcpyAsync(o.host, o.dev, o.bytes, hipMemcpyDeviceToHost, L->stream));
+        PHF_HIP(hipStreamSynchronize(L->stream));
+        return PHF_OK;
+    };
     if (total <= size_t(kPackBytes)) {
-        PHF_TRY(L->pin.ensure(kPackBytes));
+        if (!have_pin(L)) return plain();
         // neighbours on the device come in one transfer
         size_t at = 0, run = 0;
         const char *from = nullptr;
@@ -311,34 +339,30 @@ int copy_out(Lane *L, std::initializer_list<HostOut> out)
         }
         return PHF_OK;
     }
-    auto plain = [&]() -> int {
-        for (const HostOut &o : out)
-            if (o.bytes)
-                PHF_HIP(hipMemcpyAsync(o.host, o.dev, o.bytes, hipMemcpyDeviceToHost, L->stream));
-        PHF_HIP(hipStreamSynchronize(L->stream));
-        return PHF_OK;
-    };
     if (total < kRingBytes) return plain();
     Fetch fetch;
     if (!fetch.alone || !(g_ring.ptr || g_ring.make())) return plain();
     const Ring ring = g_ring;
     std::vector<Piece> pc;
+    std::vector<int> piece_of;  // of every task
+    std::unique_ptr<std::atomic<int>[]> left;
+    std::unique_ptr<std::atomic<bool>[]> sent;
     int ntask = 0;
-    for (const HostOut &o : out)
-        for (size_t at = 0; at < o.bytes; at += kSlot) {
-            const size_t b = std::min(kSlot, o.bytes - at);
-            pc.push_back({static_cast<char *>(o.host) + at, static_cast<const char *>(o.dev) + at,
-                          b, ntask});
-            ntask += (int)((b + kTask - 1) / kTask);
-        }
-    const int np = (int)pc.size();
-    std::vector<int> piece_of((size_t)ntask);
-    for (int p = 0; p < np; ++p) {
-        const int end = p + 1 < np ? pc[(size_t)p + 1].task0 : ntask;
-        for (int t = pc[(size_t)p].task0; t < end; ++t) piece_of[(size_t)t] = p;
+    try {
+        for (const HostOut &o : out)
+            for (size_t at = 0; at < o.bytes; at += kSlot) {
+                const size_t b = std::min(kSlot, o.bytes - at);
+                pc.push_back({static_cast<char *>(o.host) + at,
+                              static_cast<const char *>(o.dev) + at, b, ntask});
+                ntask += (int)((b + kTask - 1) / kTask);
+                piece_of.resize((size_t)ntask, (int)pc.size() - 1);
+            }
+        left.reset(new std::atomic<int>[pc.size()]);
+        sent.reset(new std::atomic<bool>[pc.size()]);
+    } catch (...) {  // no memory for the bookkeeping
+        return plain();
     }
-    std::unique_ptr<std::atomic<int>[]> left(new std::atomic<int>[(size_t)np]);
-    std::unique_ptr<std::atomic<bool>[]> sent(new std::atomic<bool>[(size_t)np]);
+    const int np = (int)pc.size();
     std::atomic<int> err{(int)hipSuccess};
     auto send = [&](int p) {
         const Piece &q = pc[(size_t)p];

@@ -5,15 +5,22 @@
 
 #include "phf_common.hpp"
 
-#include <functional>
 #include <initializer_list>
+#include <type_traits>
 
 namespace phf {
 
 // fn(0) .. fn(n - 1), taken in order by the calling thread and a few worker
 // threads shared by the process; returns when all are done.  fn must not
 // throw.  Several callers may be in it at once.
-void host_parallel(int n, const std::function<void(int)> &fn);
+void host_parallel(int n, void (*fn)(void *, int), void *ctx);
+template <class F>
+void host_parallel(int n, F &&fn)
+{
+    using T = std::remove_reference_t<F>;
+    host_parallel(
+        n, [](void *c, int i) { (*static_cast<T *>(c))(i); }, &fn);
+}
 
 // n doubles of host memory into the device slice *dev each: one transfer
 // through the lane's pinned staging when they are small, else one each.

@@ -48,5 +48,6 @@ def load(path):
     h = ctypes.CDLL(path, mode=os.RTLD_LOCAL | os.RTLD_NOW)
     h.phf_last_error.restype = ctypes.c_char_p
     h.hr_calls.restype = h.hr_launches.restype = ctypes.c_long
+    h.hr_fail_new.argtypes = [ctypes.c_long]
     h.hr_fail.argtypes = [ctypes.c_char_p, ctypes.c_long]
     return h

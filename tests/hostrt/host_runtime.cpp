@@ -9,7 +9,8 @@
 //   - memory of both kinds is malloc'ed and counted; copies are done at once;
 //   - a launch does nothing but report its kernel's name and arguments to the
 //     test's callback (hr_on_launch), which may write what the kernel would;
-//   - any entry point can be made to fail once (hr_fail).
+//   - any entry point can be made to fail once (hr_fail), and so can the
+//     library's own allocations on the calling thread (hr_fail_new).
 #include <hip/hip_runtime_api.h>
 
 #include <chrono>
@@ -17,6 +18,7 @@
 #include <cstring>
 #include <map>
 #include <mutex>
+#include <new>
 #include <string>
 #include <thread>
 
@@ -31,6 +33,7 @@ long g_fail_after = -1;
 long g_delay_us = 0;  // of hipHostMalloc
 void (*g_launch_cb)(const char *, void **) = nullptr;
 thread_local int t_device = 0;
+thread_local long t_new = -1;
 thread_local hipError_t t_last = hipSuccess;
 thread_local struct {
     dim3 grid, block;
@@ -38,12 +41,20 @@ thread_local struct {
     hipStream_t stream;
 } t_cfg;
 
+// the runtime's own allocations do not fail
+struct NoFail {
+    const long saved = t_new;
+    NoFail() { t_new = -1; }
+    ~NoFail() { t_new = saved; }
+};
+
 struct Obj {
     int device;
 };
 
 hipError_t enter(const char *name)
 {
+    const NoFail nf;
     std::lock_guard<std::mutex> lk(g_mu);
     ++g_calls[name];
     if (g_fail_after >= 0 && g_fail_name == name && g_fail_after-- == 0)
@@ -60,6 +71,7 @@ hipError_t enter(const char *name)
 template <class T>
 T make()
 {
+    const NoFail nf;
     return reinterpret_cast<T>(new Obj{t_device});
 }
 
@@ -69,11 +81,34 @@ int device_of(T t)
     return reinterpret_cast<Obj *>(t)->device;
 }
 
+void *allocate(size_t n)
+{
+    if (t_new >= 0 && t_new-- == 0) throw std::bad_alloc();
+    void *p = std::malloc(n ? n : 1);
+    if (!p) throw std::bad_alloc();
+    return p;
+}
+
 }  // namespace
+
+void *operator new(size_t n) { return allocate(n); }
+void *operator new[](size_t n) { return allocate(n); }
+void operator delete(void *p) noexcept { std::free(p); }
+void operator delete[](void *p) noexcept { std::free(p); }
+void operator delete(void *p, size_t) noexcept { std::free(p); }
+void operator delete[](void *p, size_t) noexcept { std::free(p); }
 
 extern "C" {
 
 // ----------------------------------------------------------- for tests --
+// the (after + 1)-th allocation of this thread from now on fails; returns
+// whether the one asked for last is still to come
+int hr_fail_new(long after)
+{
+    const int waiting = t_new >= 0;
+    t_new = after;
+    return waiting;
+}
 long hr_calls(const char *name)
 {
     std::lock_guard<std::mutex> lk(g_mu);
@@ -304,6 +339,7 @@ hipError_t __hipPopCallConfiguration(dim3 *grid, dim3 *block, size_t *shared, hi
 hipError_t hipLaunchKernel(const void *f, dim3 grid, dim3, void **args, size_t, hipStream_t s)
 {
     ENTER();
+    const NoFail nf;
     if (s && device_of(s) != t_device) return t_last = hipErrorInvalidHandle;
     if (grid.x == 0 || grid.y == 0 || grid.z == 0)
         return t_last = hipErrorInvalidConfiguration;

@@ -45,6 +45,7 @@ def _clean(H):
     yield
     H.hr_on_launch(None)
     H.hr_fail(b"", -1)
+    H.hr_fail_new(-1)
     H.hr_pin_delay_us(0)
     H.hr_set_device(0)
 
@@ -314,3 +315,46 @@ def test_direct_sum_without_memory_for_its_sort(fresh, field, nt):
     # with room it does sort
     assert direct(H, 2100, nt, field) == 0, H.phf_last_error()
     assert H.hr_launches(b"direct_f64_sorted") + H.hr_launches(b"vort_near") > 0
+
+
+@pytest.mark.parametrize("what", ["get", "set"])
+def test_no_host_memory_for_the_workers(H, what):
+    """The checks and copies that share worker threads do without them, and
+    without the pinned slots, when the host has no memory for their
+    bookkeeping: no exception leaves the C entry, and the data are right."""
+    n = 300000
+    s, xyw = system(H, n)
+    for k in range(100):
+        # the runtime's own objects are made in calls before this one
+        assert get(H, s, n)[0] == 0
+        out = np.zeros((3, n))
+        o = [ptr(a) for a in out]
+        x = [ptr(a) for a in xyw]
+        H.hr_fail_new(k)
+        if what == "get":
+            rc = H.phf_system_get(s, *o)
+        else:
+            rc = H.phf_system_set(s, *x, ctypes.c_int64(n))
+        left = H.hr_fail_new(-1)
+        assert rc == 0, H.phf_last_error()
+        assert np.array_equal(get(H, s, n)[1] if what == "set" else out, xyw)
+        if left:
+            break
+    assert left and k > 1  # each of the call's allocations has failed once
+    assert H.phf_system_destroy(s) == 0
+
+
+def test_no_memory_to_pin(fresh):
+    """Small arrays go without the pinned staging when it cannot be had."""
+    H = fresh
+    n = 100
+    r, o = np.random.default_rng(0).random((3, n)), np.empty((2, n))
+    H.hr_fail(b"hipHostMalloc", 0)
+    args = [ptr(r[0]), ptr(r[1]), ptr(r[2]), ctypes.c_int64(n), ptr(r[0]), ptr(r[1]),
+            ctypes.c_int64(n), ctypes.c_double(1e-4), 0, ptr(o[0]), ptr(o[1])]
+    assert H.phf_vv2par_gauss(*args) == 0, H.phf_last_error()
+    s, xyw = system(H, n)
+    H.hr_fail(b"hipHostMalloc", 0)
+    rc, out = get(H, s, n)
+    assert rc == 0 and H.phf_last_error() == b"" and np.array_equal(out, xyw)
+    assert H.phf_system_destroy(s) == 0
