@@ -223,10 +223,10 @@ int phf_population_control(const double *x, const double *y, const double *w, in
  *   'fixed' system (scipy lu_factor/lu_solve, :961/:782); rows > n is the
  *   'prescribed' least-squares system [A; L] x = [RHS; -gTotal]
  *   (numpy.linalg.lstsq, :800-822).  B is row-major rows x n.  A float32
- *   factorisation (Cholesky of B^T B; for rows == n also the LU with partial
- *   pivoting of B, above n = 1024 or where B^T B does not serve) + float64
- *   iterative refinement (semi-normal float64 residuals when rows > n).  info
- *   may be NULL. */
+ *   factorisation (the LU with partial pivoting of B for rows == n; for rows > n
+ *   the Cholesky of B^T B, or its LU above n = 1024 and where it is not positive
+ *   definite in float32) + float64 iterative refinement (semi-normal float64
+ *   residuals when rows > n).  info may be NULL. */
 int phf_panel_influence(const double *xCP, const double *yCP, const double *xs,
                         const double *ys, const double *xe, const double *ye,
                         const double *cosA, const double *sinA, int64_t m, double *A);

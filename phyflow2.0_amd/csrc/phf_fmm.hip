@@ -28,8 +28,8 @@
 // stores points as float32 offsets from their leaf centre (formed in
 // float64; leaf sides and centre differences are exact in float32 because
 // the domain side carries 5 significant bits), runs P2P with compensated
-// per-target sums, P2M/M2L/L2P in float32, and M2M/L2L in float64 when the
-// order exceeds 16.
+// per-target sums and P2M/M2L/L2P in float32, and keeps the expansions in
+// float32; M2M/L2L compute in float64 from and to them.
 #include "phf_fmm.hpp"
 #include "phf_host.hpp"
 #include "phf_fmm_dev.hpp"
@@ -1367,8 +1367,9 @@ static int fmm_plan(Lane *L, const FmmArgs &a, const Domain &dom, const PairPara
 }
 
 template <class T>
-static int run_fmm_typed(Lane *L, const FmmArgs &a, const Domain &dom, const SortedPoints &S, const SortedPoints &Tg, StageTimer &tm,
-                         bool *used, FmmInfo *info, FmmSplit *spl, int *nnear_out)
+static int run_fmm_typed(Lane *L, const FmmArgs &a, const Domain &dom, const SortedPoints &S,
+                         const SortedPoints &Tg, StageTimer &tm, bool *used, FmmInfo *info,
+                         FmmSplit *spl, int *nnear_out)
 {
     using V = typename C2<T>::type;
     const int Lv = dom.L, p1 = a.p + 1;
@@ -1600,10 +1601,9 @@ static int run_fmm_typed(Lane *L, const FmmArgs &a, const Domain &dom, const Sor
                                     d_bin));
         }
         tm.end(PHF_STAGE_M2L);
-        // L2L: every ancestor level shifted straight to the leaves
         tm.begin(PHF_STAGE_L2L);
         used[PHF_STAGE_L2L] = true;
-        // down to the leaves, three levels per launch, the remainder first
+        // L2L down to the leaves, three levels per launch, the remainder first
         for (int lev = 2; lev < Lv;) {
             DownLevels dl{};
             dl.nlev = (Lv - lev) % 3 ? (Lv - lev) % 3 : 3;

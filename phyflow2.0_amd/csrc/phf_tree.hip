@@ -246,14 +246,6 @@ __global__ __launch_bounds__(SC_THREADS) void scan_apply(const uint32_t *__restr
 
 int64_t scan_sums_size(int64_t n) { return (n + SC_CHUNK - 1) / SC_CHUNK + 1; }
 
-int device_exclusive_scan(Lane *L, const uint32_t *in, int64_t n, uint32_t *out)
-{
-    if (n <= 0) return PHF_OK;
-    uint32_t *sums;
-    PHF_ALLOC(sums, L->arena, uint32_t, (size_t)scan_sums_size(n));
-    return device_exclusive_scan_ws(L, in, n, out, sums);
-}
-
 int device_exclusive_scan_ws(Lane *L, const uint32_t *in, int64_t n, uint32_t *out,
                              uint32_t *sums, const int64_t *dn)
 {

@@ -41,8 +41,7 @@ int device_bbox(Lane *L, const double *x1, const double *y1, int64_t n1, const d
 int device_bbox_parts(Lane *L, const double *x1, const double *y1, int64_t n1, const double *x2,
                       const double *y2, int64_t n2, double4 **parts, int *np);
 
-int device_exclusive_scan(Lane *L, const uint32_t *in, int64_t n, uint32_t *out);
-// variants with caller-provided workspaces (no allocation: capturable)
+// scan and sort with caller-provided workspaces (no allocation: capturable)
 int64_t scan_sums_size(int64_t n);
 // dn (device, nullable): scan only the first *dn <= n entries
 int device_exclusive_scan_ws(Lane *L, const uint32_t *in, int64_t n, uint32_t *out,

@@ -215,6 +215,17 @@ def test_blobs_come_back_whole(n):
     assert not wrong
 
 
+@pytest.mark.parametrize("n", [87381, 87382, 131072, 131073, 699050, 699051, 800001])
+def test_blobs_come_back_whole_alone(n):
+    """Fetches that are alone go through the pinned slots from 2 MiB (24 n
+    bytes) on: one slot, whole and odd ones, and as many as there are and more."""
+    from phyflow_amd.system import BlobSystem
+    data = np.random.default_rng(n).random((3, n))
+    with BlobSystem(*data) as s:
+        for _ in range(2):
+            assert np.array_equal(s.get(), data)
+
+
 @pytest.mark.parametrize("n", [1, 7, 65536, 65537, 300001])
 @pytest.mark.parametrize("bad", [np.nan, np.inf, -np.inf])
 def test_not_finite_is_refused_anywhere(n, bad):
