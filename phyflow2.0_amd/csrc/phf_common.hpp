@@ -98,6 +98,14 @@ struct Arena {
     }
     void release();
     size_t capacity() const;
+    // whether [p, p + bytes) lies within one of the blocks
+    bool within_block(const void *p, size_t bytes) const
+    {
+        const char *c = static_cast<const char *>(p);
+        for (const Block &b : blocks)
+            if (c >= b.base && c + bytes <= b.base + b.cap) return true;
+        return false;
+    }
 };
 
 #define PHF_ALLOC(ptr, arena, T, count)                                      \

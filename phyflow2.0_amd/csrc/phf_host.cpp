@@ -315,12 +315,13 @@ int copy_out(Lane *L, std::initializer_list<HostOut> out)
     };
     if (total <= size_t(kPackBytes)) {
         if (!have_pin(L)) return plain();
-        // neighbours on the device come in one transfer
+        // neighbours in the arena come in one transfer; arrays that touch but are
+        // allocations of their own must not
         size_t at = 0, run = 0;
         const char *from = nullptr;
         for (const HostOut &o : out) {
             const char *d = static_cast<const char *>(o.dev);
-            if (run > 0 && d != from + run) {
+            if (run > 0 && (d != from + run || !L->arena.within_block(from, run + o.bytes))) {
                 PHF_HIP(hipMemcpyAsync(L->pin.ptr + at, from, run, hipMemcpyDeviceToHost,
                                        L->stream));
                 at += run;

@@ -6,12 +6,16 @@
 //   - two devices; every thread has a current one (0 at first), streams and
 //     events belong to the one they were made on, and recording an event on,
 //     or launching on, another device's stream is refused as HIP refuses it;
-//   - memory of both kinds is malloc'ed and counted; copies are done at once;
+//   - memory of both kinds is host memory and counted.  Device allocations are
+//     whole pages, one after the other, so that neighbours touch; a copy that
+//     does not lie within one is refused as HIP refuses it.  Copies are done
+//     at once;
 //   - a launch does nothing but report its kernel's name and arguments to the
 //     test's callback (hr_on_launch), which may write what the kernel would;
 //   - any entry point can be made to fail once (hr_fail), and so can the
 //     library's own allocations on the calling thread (hr_fail_new).
 #include <hip/hip_runtime_api.h>
+#include <sys/mman.h>
 
 #include <chrono>
 #include <cstdlib>
@@ -41,6 +45,10 @@ thread_local struct {
     hipStream_t stream;
 } t_cfg;
 
+struct Obj {
+    int device;
+};
+
 // the runtime's own allocations do not fail
 struct NoFail {
     const long saved = t_new;
@@ -48,9 +56,23 @@ struct NoFail {
     ~NoFail() { t_new = saved; }
 };
 
-struct Obj {
-    int device;
-};
+// device memory: pages of one reserved range, never handed out twice
+constexpr size_t kPage = 4096, kRange = size_t(1) << 38;
+char *g_base = nullptr, *g_next = nullptr;
+std::map<char *, size_t> g_blocks;  // live allocations
+
+// whether [p, p + n) is no device memory, or lies within one allocation
+bool in_one_block(const void *p, size_t n)
+{
+    const NoFail nf;
+    std::lock_guard<std::mutex> lk(g_mu);
+    char *c = static_cast<char *>(const_cast<void *>(p));
+    if (!g_base || c < g_base || c >= g_base + kRange) return true;
+    auto it = g_blocks.upper_bound(c);
+    if (it == g_blocks.begin()) return false;
+    --it;
+    return c + n <= it->first + it->second;
+}
 
 hipError_t enter(const char *name)
 {
@@ -171,6 +193,7 @@ const char *hipGetErrorName(hipError_t e)
 {
     return e == hipErrorOutOfMemory     ? "hipErrorOutOfMemory"
            : e == hipErrorInvalidHandle ? "hipErrorInvalidHandle"
+           : e == hipErrorInvalidValue  ? "hipErrorInvalidValue"
                                         : "hipError";
 }
 hipError_t hipGetLastError()
@@ -184,13 +207,30 @@ hipError_t hipGetLastError()
 hipError_t hipMalloc(void **p, size_t n)
 {
     ENTER();
-    *p = nullptr;
-    return posix_memalign(p, 4096, n ? n : 1) == 0 ? hipSuccess : hipErrorOutOfMemory;
+    const NoFail nf;
+    std::lock_guard<std::mutex> lk(g_mu);
+    if (!g_base) {
+        void *m = mmap(nullptr, kRange, PROT_READ | PROT_WRITE,
+                       MAP_PRIVATE | MAP_ANONYMOUS | MAP_NORESERVE, -1, 0);
+        if (m == MAP_FAILED) return hipErrorOutOfMemory;
+        g_base = g_next = static_cast<char *>(m);
+    }
+    const size_t b = (n + kPage - 1) / kPage * kPage;
+    if (n == 0 || g_next + b > g_base + kRange) return hipErrorOutOfMemory;
+    *p = g_next;
+    g_blocks[g_next] = n;
+    g_next += b;
+    return hipSuccess;
 }
 hipError_t hipFree(void *p)
 {
     ENTER();
-    std::free(p);
+    const NoFail nf;
+    std::lock_guard<std::mutex> lk(g_mu);
+    auto it = g_blocks.find(static_cast<char *>(p));
+    if (it == g_blocks.end()) return p ? hipErrorInvalidValue : hipSuccess;
+    madvise(p, (it->second + kPage - 1) / kPage * kPage, MADV_DONTNEED);
+    g_blocks.erase(it);
     return hipSuccess;
 }
 hipError_t hipHostMalloc(void **p, size_t n, unsigned)
@@ -215,12 +255,14 @@ hipError_t hipMemcpy(void *d, const void *s, size_t n, hipMemcpyKind)
 hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind, hipStream_t)
 {
     ENTER();
+    if (!in_one_block(d, n) || !in_one_block(s, n)) return hipErrorInvalidValue;
     std::memmove(d, s, n);
     return hipSuccess;
 }
 hipError_t hipMemsetAsync(void *d, int v, size_t n, hipStream_t)
 {
     ENTER();
+    if (!in_one_block(d, n)) return hipErrorInvalidValue;
     std::memset(d, v, n);
     return hipSuccess;
 }

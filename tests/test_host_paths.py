@@ -358,3 +358,14 @@ def test_no_memory_to_pin(fresh):
     rc, out = get(H, s, n)
     assert rc == 0 and H.phf_last_error() == b"" and np.array_equal(out, xyw)
     assert H.phf_system_destroy(s) == 0
+
+
+@pytest.mark.parametrize("n", [1, 512, 1024, 2048, 3072, 4096, 5120])
+def test_small_results_of_touching_allocations(H, n):
+    """Arrays of whole pages can be neighbours in memory and allocations of
+    their own all the same."""
+    s, xyw = system(H, n)
+    rc, out = get(H, s, n)
+    assert rc == 0, H.phf_last_error()
+    assert np.array_equal(out, xyw)
+    assert H.phf_system_destroy(s) == 0

@@ -226,6 +226,22 @@ def test_blobs_come_back_whole_alone(n):
             assert np.array_equal(s.get(), data)
 
 
+@pytest.mark.parametrize("n", [511, 512, 1024, 2048, 3072, 4096, 4608, 5120, 5461])
+def test_systems_of_whole_pages(n, O):
+    """Small systems whose arrays are whole pages, and so may touch in memory
+    without being one allocation: blobs and velocities come back."""
+    from phyflow_amd.system import BlobSystem, vel_params
+    s = W.uniform_system(n, seed=n)
+    xopt, cutoff = W.oseen_params(s["sigma"])
+    q = O.direct_oseen(s["x"], s["y"], s["w"], s["x"], s["y"], xopt, cutoff)
+    with BlobSystem(s["x"], s["y"], s["w"]) as b:
+        assert np.array_equal(b.get(), [s["x"], s["y"], s["w"]])
+        v = b.velocity(vel_params(s["sigma"]))
+        assert np.array_equal(v, b.last_velocity())
+        # (-qi, -qr) / 2 pi at the default tolerance 1e-6
+        assert O.rel_l2(v, [-q[1] / (2 * np.pi), -q[0] / (2 * np.pi)]) <= 1e-6
+
+
 @pytest.mark.parametrize("n", [1, 7, 65536, 65537, 300001])
 @pytest.mark.parametrize("bad", [np.nan, np.inf, -np.inf])
 def test_not_finite_is_refused_anywhere(n, bad):
