@@ -1046,7 +1046,8 @@ static int batch_enqueue_typed(Lane *L, const BatchPlan &P, BatchBuffers &Bf, co
     const VC *m2m = reinterpret_cast<const VC *>(Bf.m2m);
     const VC *l2l = reinterpret_cast<const VC *>(Bf.l2l);
     if (P.Lmax >= 2) {
-        PHF_TRY(p2m_dispatch(p1, (double)P.N, (double)P.nleaf, [&](auto ni, auto r) {
+        const bool many = P.nleaf >= 12288;
+        PHF_TRY(p2m_dispatch(p1, (double)P.N, (double)P.nleaf, many, [&](auto ni, auto r) {
             constexpr int R = decltype(r)::value;
             batch_p2m<T, decltype(ni)::value, R>
                 <<<div_up(P.nleaf, 64 / R), 256, 0, L->stream>>>(

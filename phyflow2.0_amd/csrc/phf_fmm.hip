@@ -1544,7 +1544,7 @@ static int run_fmm_typed(Lane *L, const FmmArgs &a, const Domain &dom, const Sor
         // P2M
         tm.begin(PHF_STAGE_P2M);
         used[PHF_STAGE_P2M] = true;
-        PHF_TRY(p2m_dispatch(p1, (double)a.nb, dom.occupied, [&](auto ni, auto r) {
+        PHF_TRY(p2m_dispatch(p1, (double)a.nb, dom.occupied, false, [&](auto ni, auto r) {
             constexpr int R = decltype(r)::value;
             p2m_kernel<T, decltype(ni)::value, R>
                 <<<(nleaf + 64 / R - 1) / (64 / R), 256, 0, L->stream>>>(

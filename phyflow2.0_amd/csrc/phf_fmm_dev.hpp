@@ -39,15 +39,17 @@ __device__ __forceinline__ int box_count(const int32_t *__restrict__ start, uint
 
 // ----------------------------------------------------------------- P2M --
 // Multipole expansion sum_j w_j ((z_j - c) inv_s)^k, k < p1 <= 4 NI, of the
-// points [s0, s1) by 4 R lanes of a wave (R = 16 or 4), without LDS.  Lane
-// 4 r + q takes the points j = r (mod R) and the powers k = q (mod 4): it
-// forms z^q from z and z^2, steps by z^4 through its NI powers and keeps their
-// sums in registers; the R lanes of a power are then added by a butterfly.
-// Four residues of
-// k balance the products repeated in every lane of a point (2 squarings, 2
-// selected) against the butterfly (4 steps of NI).  (With a table of
-// 64 x p1 powers in LDS and each column added by one lane, a leaf was a
-// serial chain of 64 LDS reads with 64 - p1 lanes idle.)
+// points [s0, s1) by 4 R lanes of a wave (R = 16 or 4), without LDS.  The
+// points fall into sixteen classes j (mod 16), added in index order each and
+// then pairwise in class order, whatever R is, so that a leaf's expansion does
+// not depend on what else is in the launch.  Lane 4 r + q takes 16 / R classes
+// and the powers k = q (mod 4): it forms z^q from z and z^2, steps by z^4
+// through its NI powers and keeps their sums in registers; the R lanes of a
+// power are then added by a butterfly.  Four residues of k balance the products
+// repeated in every lane of a point (2 squarings, 2 selected) against the
+// butterfly (4 steps of NI).  (With a table of 64 x p1 powers in LDS and each
+// column added by one lane, a leaf was a serial chain of 64 LDS reads with
+// 64 - p1 lanes idle.)
 // Beside the near field of 1M blobs, order 16: 65 us with the table, 19 us so
 // and at the far field's wave priority.
 // float32 records are relative to the leaf centre; (cx, cy) is the centre
@@ -58,46 +60,86 @@ __device__ __forceinline__ void p2m_leaf(const void *__restrict__ src, int32_t s
                                          typename C2<T>::type *__restrict__ out)
 {
     using V = typename C2<T>::type;
-    const int lane = threadIdx.x & (4 * R - 1), q = lane & 3, r = lane >> 2;
-    V acc[NI];
-#pragma unroll
-    for (int i = 0; i < NI; ++i) acc[i] = cmk<T>(0, 0);
-    // the loads of U points go out together (R U points of the leaf)
-    constexpr int U = 4;
     using Rec = std::conditional_t<sizeof(T) == 4, float4, double4>;
+    constexpr int KC = 16 / R;  // classes of a lane, KC r ..
+    const int lane = threadIdx.x & (4 * R - 1), q = lane & 3, r = lane >> 2;
     const Rec *rec = reinterpret_cast<const Rec *>(src);
-    for (int32_t j0 = s0 + r; j0 < s1; j0 += R * U) {
-        Rec pt[U];
+    auto zero = [](V *a) {
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int32_t j = j0 + R * u;
-            pt[u] = rec[j < s1 ? j : s0];
+        for (int i = 0; i < NI; ++i) a[i] = cmk<T>(0, 0);
+    };
+    auto add = [](V *a, const V *b) {
+#pragma unroll
+        for (int i = 0; i < NI; ++i) {
+            a[i].x += b[i].x;
+            a[i].y += b[i].y;
         }
+    };
+    auto point = [&](const Rec &pt, V *a) {
+        V z;
+        if (sizeof(T) == 4)
+            z = cmk<T>((T)pt.x * inv_s, (T)pt.y * inv_s);
+        else
+            z = cmk<T>((T)((pt.x - cx) * inv_s), (T)((pt.y - cy) * inv_s));
+        V t = cmk<T>((T)pt.z, 0);
+        const V z2 = cmul(z, z), z4 = cmul(z2, z2);
+        if (q & 1) t = cmul(t, z);
+        if (q & 2) t = cmul(t, z2);
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            if (j0 + R * u >= s1) break;
-            V z;
-            if (sizeof(T) == 4)
-                z = cmk<T>((T)pt[u].x * inv_s, (T)pt[u].y * inv_s);
-            else
-                z = cmk<T>((T)((pt[u].x - cx) * inv_s), (T)((pt[u].y - cy) * inv_s));
-            V t = cmk<T>((T)pt[u].z, 0);
-            const V z2 = cmul(z, z), z4 = cmul(z2, z2);
-            if (q & 1) t = cmul(t, z);
-            if (q & 2) t = cmul(t, z2);
+        for (int i = 0; i < NI; ++i) {
+            a[i].x += t.x;
+            a[i].y += t.y;
+            if (i + 1 < NI) t = cmul(t, z4);
+        }
+    };
+    // the points j, j + 16, .. of a class; the loads of U points go out together
+    auto points = [&](int32_t j0, V *a) {
+        constexpr int U = KC == 1 ? 4 : 3;
+        for (; j0 < s1; j0 += 16 * U) {
+            Rec pt[U];
 #pragma unroll
-            for (int i = 0; i < NI; ++i) {
-                acc[i].x += t.x;
-                acc[i].y += t.y;
-                if (i + 1 < NI) t = cmul(t, z4);
+            for (int u = 0; u < U; ++u) {
+                const int32_t j = j0 + 16 * u;
+                pt[u] = rec[j < s1 ? j : s0];
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                if (j0 + 16 * u >= s1) break;
+                point(pt[u], a);
             }
         }
-    }
+    };
     if (__ballot(s1 > s0) == 0) {  // nothing to add up
 #pragma unroll
         for (int i = 0; i < NI; ++i)
             if (r == i % R && 4 * i + q < p1) out[4 * i + q] = cmk<T>(0, 0);
         return;
+    }
+    V acc[NI];
+    zero(acc);
+    if constexpr (KC == 1) {
+        points(s0 + r, acc);
+    } else {
+        const int32_t j0 = s0 + KC * r;
+        Rec first[KC];  // the first point of each class, loaded together
+#pragma unroll
+        for (int c = 0; c < KC; ++c) {
+            const int32_t j = j0 + c;
+            first[c] = rec[j < s1 ? j : s1 > s0 ? s0 : 0];
+        }
+        auto cls = [&](int c, V *a) {
+            zero(a);
+            if (j0 + c < s1) point(first[c], a);
+            points(j0 + c + 16, a);
+        };
+        V b[NI], c[NI];
+        cls(0, acc);
+        cls(1, b);
+        add(acc, b);
+        cls(2, b);
+        cls(3, c);
+        add(b, c);
+        add(acc, b);
     }
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
@@ -116,12 +158,17 @@ void set_error(const char *fmt, ...) __attribute__((format(printf, 1, 2)));
 // f(integral constants NI, R) for the compiled NI that holds p1 powers and the
 // lanes of a leaf: a wave (R = 16), or sixteen lanes (R = 4) where the mean
 // leaf has fewer than 24 points, which a wave takes in little more than one
-// round of its 16 points and then spends on the butterfly.
+// round of its 16 points and then spends on the butterfly; and, where the
+// chip is full of leaves (many), since sixteen lanes go four times as long but
+// with an eighth of the butterfly.  In a batch, nothing beside it, 1,024 leaves
+// of 64 float32 points, order 13: 4.8 us by waves, 8.0 by sixteen lanes; 8,192
+// leaves 9.0 and 9.8, 16,384 15.4 and 12.7, 131,072 128.6 and 76.4 (107.8 with
+// the table).
 template <class F>
-inline int p2m_dispatch(int p1, double points, double leaves, const F &f)
+inline int p2m_dispatch(int p1, double points, double leaves, bool many, const F &f)
 {
     auto lanes = [&](auto ni) {
-        if (points < 24.0 * leaves)
+        if (points < 24.0 * leaves || many)
             f(ni, std::integral_constant<int, 4>());
         else
             f(ni, std::integral_constant<int, 16>());

@@ -228,3 +228,32 @@ def test_batch_step_graph_replays():
         b.step(use_graph=False)
         for i in range(len(systems)):
             assert all(np.array_equal(a, e) for a, e in zip(g1[i], b.get_remeshed(i)))
+
+
+@pytest.mark.parametrize("order", [8, 13, 16, 20, 29, 40])
+@pytest.mark.parametrize("prec", [PREC_F64, PREC_F32C])
+def test_alone_equals_in_sparse_and_full_mixes(prec, order):
+    """How many lanes a leaf's multipoles take follows from the whole batch
+    (few points a leaf, more leaves than fill the chip); their sums do not: a
+    system comes out with the same bits alone, among many tiny ones and among
+    many large ones."""
+    def flow(n, seed):
+        s = W.uniform_system(n, seed=seed)
+        # uneven leaves, empty ones among them
+        return dict(s, x=s["x"] ** 1.5, sigma=min(s["sigma"], 0.01))
+
+    def run(systems):
+        with BatchSystems([s["x"].size for s in systems], [s["sigma"] for s in systems],
+                          prec=prec, order=order) as b:
+            for i, s in enumerate(systems):
+                b.set_system(i, s["x"], s["y"], s["w"])
+            b.velocity()
+            return [b.get_velocity(i) for i in (0, 1)]
+
+    two = [flow(30011, 1), flow(2003, 2)]
+    sparse = [flow(5 + k % 7, k) for k in range(2500)]
+    full = [flow(70001, 3)] * 13
+    alone = [run([s, flow(1, 0)])[0] for s in two]
+    for mix in (two, two + sparse, two + full):
+        for got, ref in zip(run(mix), alone):
+            assert np.array_equal(got, ref), (len(mix), prec, order)
