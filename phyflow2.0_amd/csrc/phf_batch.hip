@@ -239,8 +239,8 @@ __global__ __launch_bounds__(256) void batch_p2m(const BatchSys *__restrict__ sy
     const BatchDom d = dom[s];
     double cx, cy;
     leaf_center(b, d.x0, d.y0, d.s, cx, cy);
-    p2m_leaf<T, NI, R>(src, start[g], start[g + 1], cx, cy, (T)(1.0 / d.s), p1,
-                    M + (lvl[L * (S + 1) + s] + b) * p1);
+    p2m_leaf<T, NI, R, true>(src, start[g], start[g + 1], cx, cy, (T)(1.0 / d.s), p1,
+                             M + (lvl[L * (S + 1) + s] + b) * p1);
 }
 
 // --------------------------------------------------------- M2M / L2L ------
@@ -1046,8 +1046,8 @@ static int batch_enqueue_typed(Lane *L, const BatchPlan &P, BatchBuffers &Bf, co
     const VC *m2m = reinterpret_cast<const VC *>(Bf.m2m);
     const VC *l2l = reinterpret_cast<const VC *>(Bf.l2l);
     if (P.Lmax >= 2) {
-        const bool many = P.nleaf >= 12288;
-        PHF_TRY(p2m_dispatch(p1, (double)P.N, (double)P.nleaf, many, [&](auto ni, auto r) {
+        const bool narrow = p2m_narrow_batch((double)P.N, (double)P.nleaf);
+        PHF_TRY(p2m_dispatch(p1, narrow, [&](auto ni, auto r) {
             constexpr int R = decltype(r)::value;
             batch_p2m<T, decltype(ni)::value, R>
                 <<<div_up(P.nleaf, 64 / R), 256, 0, L->stream>>>(

@@ -102,7 +102,8 @@ __global__ __launch_bounds__(256) void p2m_kernel(const void *__restrict__ src,
     if (b >= nleaf) return;
     double cx = 0.0, cy = 0.0;
     if (sizeof(T) == 8) leaf_center(b, org->x, org->z, s, cx, cy);
-    p2m_leaf<T, NI, R>(src, start[b], start[b + 1], cx, cy, (T)inv_s, p1, M + (int64_t)b * p1);
+    p2m_leaf<T, NI, R, false>(src, start[b], start[b + 1], cx, cy, (T)inv_s, p1,
+                              M + (int64_t)b * p1);
 }
 
 // ---------------------------------------------------------- M2M / L2L ----
@@ -1544,7 +1545,7 @@ static int run_fmm_typed(Lane *L, const FmmArgs &a, const Domain &dom, const Sor
         // P2M
         tm.begin(PHF_STAGE_P2M);
         used[PHF_STAGE_P2M] = true;
-        PHF_TRY(p2m_dispatch(p1, (double)a.nb, dom.occupied, false, [&](auto ni, auto r) {
+        PHF_TRY(p2m_dispatch(p1, p2m_narrow((double)a.nb, dom.occupied), [&](auto ni, auto r) {
             constexpr int R = decltype(r)::value;
             p2m_kernel<T, decltype(ni)::value, R>
                 <<<(nleaf + 64 / R - 1) / (64 / R), 256, 0, L->stream>>>(
@@ -1698,12 +1699,14 @@ static int fmm_enqueue(Lane *L, const FmmArgs &a, const Domain &dom_in, StageTim
 // slices).  A call replays the most recent entry without waiting for the
 // bounding box: kernels read the domain corner on the device, and the
 // bounding box comes back with the results, so that the caller can check
-// that the points kept the recording's leaf level and domain side (else it
-// evaluates again with a fresh recording).
+// that the points kept the recording's leaf level, domain side and P2M lanes
+// (else it evaluates again with a fresh recording: the results follow from the
+// points alone).
 struct FmmGraph {
     FmmArgs a{};
     int L = 0, nnear = 0;
     double D = 0.0;
+    bool narrow = false;  // P2M's lanes, which its sums' order follows
     Arena::Mark m0, m1;
     hipGraph_t g[2] = {};
     hipGraphExec_t exec[2] = {};
@@ -1775,6 +1778,7 @@ static int fmm_record(Lane *L, const FmmArgs &a, const Domain &dom0, FmmGraph **
     e->a = a;
     e->L = dom0.L;
     e->D = dom0.D;
+    e->narrow = p2m_narrow((double)a.nb, dom0.occupied);
     e->m0 = L->arena.mark();
     StageTimer off(L, false);
     bool used[PHF_STAGE_COUNT] = {};
@@ -1969,11 +1973,13 @@ int fmm_device(Lane *L, const FmmArgs &a, StageTimer &tm, bool *used, FmmInfo *i
             }
             const int L0 = e->L;
             const double D0 = e->D;
-            info->domain_ok = [hb, a, L0, D0, shape_log2]() {
+            const bool n0 = e->narrow;
+            info->domain_ok = [hb, a, L0, D0, n0, shape_log2]() {
                 const Domain d = choose_domain(*hb, a.Lhint, (double)a.nb, (double)a.nt,
                                                a.cutoff, a.ws, shape_log2, a.p + 1,
                                                a.prec == PHF_PREC_F32C ? 16 : 64, a.leaf_side);
-                return d.L == L0 && d.D == D0;
+                return d.L == L0 && d.D == D0 &&
+                       p2m_narrow((double)a.nb, d.occupied) == n0;
             };
         }
         nnear = e->nnear;

@@ -39,29 +39,31 @@ __device__ __forceinline__ int box_count(const int32_t *__restrict__ start, uint
 
 // ----------------------------------------------------------------- P2M --
 // Multipole expansion sum_j w_j ((z_j - c) inv_s)^k, k < p1 <= 4 NI, of the
-// points [s0, s1) by 4 R lanes of a wave (R = 16 or 4), without LDS.  The
-// points fall into sixteen classes j (mod 16), added in index order each and
-// then pairwise in class order, whatever R is, so that a leaf's expansion does
-// not depend on what else is in the launch.  Lane 4 r + q takes 16 / R classes
-// and the powers k = q (mod 4): it forms z^q from z and z^2, steps by z^4
-// through its NI powers and keeps their sums in registers; the R lanes of a
-// power are then added by a butterfly.  Four residues of k balance the products
-// repeated in every lane of a point (2 squarings, 2 selected) against the
-// butterfly (4 steps of NI).  (With a table of 64 x p1 powers in LDS and each
+// points [s0, s1) by 4 R lanes of a wave (R = 16 or 4), without LDS.  Lane
+// 4 r + q takes the points j = r (mod R) and the powers k = q (mod 4): it forms
+// z^q from z and z^2, steps by z^4 through its NI powers and keeps their sums
+// in registers; the R lanes of a power are then added by a butterfly.  With MIX
+// the sums do not depend on R (which follows from the whole launch in a batch):
+// the points fall into sixteen classes j (mod 16) in either case, added in
+// index order each and then pairwise in class order, and a lane of R = 4 takes
+// four neighbouring classes (its expansions then take up to a third longer).
+// Four residues of k balance the products repeated in every lane of a point (2
+// squarings, 2 selected) against the butterfly (4 steps of NI).  (With a table of 64 x p1 powers in LDS and each
 // column added by one lane, a leaf was a serial chain of 64 LDS reads with
 // 64 - p1 lanes idle.)
 // Beside the near field of 1M blobs, order 16: 65 us with the table, 19 us so
 // and at the far field's wave priority.
 // float32 records are relative to the leaf centre; (cx, cy) is the centre
 // for float64 ones.
-template <class T, int NI, int R>
+template <class T, int NI, int R, bool MIX>
 __device__ __forceinline__ void p2m_leaf(const void *__restrict__ src, int32_t s0, int32_t s1,
                                          double cx, double cy, T inv_s, int p1,
                                          typename C2<T>::type *__restrict__ out)
 {
     using V = typename C2<T>::type;
     using Rec = std::conditional_t<sizeof(T) == 4, float4, double4>;
-    constexpr int KC = 16 / R;  // classes of a lane, KC r ..
+    constexpr int KC = MIX ? 16 / R : 1;    // classes of a lane, KC r ..
+    constexpr int STEP = KC == 1 ? R : 16;  // between a class's points
     const int lane = threadIdx.x & (4 * R - 1), q = lane & 3, r = lane >> 2;
     const Rec *rec = reinterpret_cast<const Rec *>(src);
     auto zero = [](V *a) {
@@ -92,19 +94,19 @@ __device__ __forceinline__ void p2m_leaf(const void *__restrict__ src, int32_t s
             if (i + 1 < NI) t = cmul(t, z4);
         }
     };
-    // the points j, j + 16, .. of a class; the loads of U points go out together
+    // the points j, j + STEP, .. of a class; the loads of U points go out together
     auto points = [&](int32_t j0, V *a) {
         constexpr int U = KC == 1 ? 4 : 3;
-        for (; j0 < s1; j0 += 16 * U) {
+        for (; j0 < s1; j0 += STEP * U) {
             Rec pt[U];
 #pragma unroll
             for (int u = 0; u < U; ++u) {
-                const int32_t j = j0 + 16 * u;
+                const int32_t j = j0 + STEP * u;
                 pt[u] = rec[j < s1 ? j : s0];
             }
 #pragma unroll
             for (int u = 0; u < U; ++u) {
-                if (j0 + 16 * u >= s1) break;
+                if (j0 + STEP * u >= s1) break;
                 point(pt[u], a);
             }
         }
@@ -155,20 +157,27 @@ __device__ __forceinline__ void p2m_leaf(const void *__restrict__ src, int32_t s
 
 void set_error(const char *fmt, ...) __attribute__((format(printf, 1, 2)));
 
-// f(integral constants NI, R) for the compiled NI that holds p1 powers and the
-// lanes of a leaf: a wave (R = 16), or sixteen lanes (R = 4) where the mean
-// leaf has fewer than 24 points, which a wave takes in little more than one
-// round of its 16 points and then spends on the butterfly; and, where the
-// chip is full of leaves (many), since sixteen lanes go four times as long but
-// with an eighth of the butterfly.  In a batch, nothing beside it, 1,024 leaves
-// of 64 float32 points, order 13: 4.8 us by waves, 8.0 by sixteen lanes; 8,192
-// leaves 9.0 and 9.8, 16,384 15.4 and 12.7, 131,072 128.6 and 76.4 (107.8 with
+// Whether leaves take sixteen lanes rather than a wave: where the mean leaf has
+// fewer than 24 points, which a wave takes in little more than one round of its
+// 16 points and then spends on the butterfly; and in a batch, which has nothing
+// beside it, where leaves fill the chip, since sixteen lanes go four times as
+// long but with an eighth of the butterfly.  Batches of leaves of 64 float32
+// points, order 13: 1,024 leaves 4.8 us by waves, 8.0 by sixteen lanes; 8,192
+// leaves 9.0 and 9.8, 16,384 15.4 and 15.0, 131,072 128.6 and 88.1 (108.5 with
 // the table).
+inline bool p2m_narrow(double points, double leaves) { return points < 24.0 * leaves; }
+inline bool p2m_narrow_batch(double points, double leaves)
+{
+    return p2m_narrow(points, leaves) || leaves >= 12288.0;
+}
+
+// f(integral constants NI, R) for the compiled NI that holds p1 powers and the
+// lanes of a leaf
 template <class F>
-inline int p2m_dispatch(int p1, double points, double leaves, bool many, const F &f)
+inline int p2m_dispatch(int p1, bool narrow, const F &f)
 {
     auto lanes = [&](auto ni) {
-        if (points < 24.0 * leaves || many)
+        if (narrow)
             f(ni, std::integral_constant<int, 4>());
         else
             f(ni, std::integral_constant<int, 16>());

@@ -242,6 +242,28 @@ def test_systems_of_whole_pages(n, O):
         assert O.rel_l2(v, [-q[1] / (2 * np.pi), -q[0] / (2 * np.pi)]) <= 1e-6
 
 
+@pytest.mark.parametrize("leaf", [16, 128])
+@pytest.mark.parametrize("prec", [F64, F32C])
+def test_replay_follows_from_the_points_alone(prec, leaf):
+    """A system evaluated before on points that filled its domain otherwise
+    (other lanes for P2M with 16 blobs a leaf, other parts of the near field
+    with 128) gives the bits that a fresh one gives."""
+    from phyflow_amd.system import BlobSystem, vel_params
+    n = 16000
+    s = W.uniform_system(n, seed=4)
+    p = vel_params(0.2 * s["sigma"], prec=prec, order=17, leaf=leaf, leaf_side=-1.0)
+    x, y, w = s["x"], s["y"], s["w"]
+    x[0], x[1] = 0.0, 1.0  # the same bounding box side for both
+    y[0], y[1] = 0.0, 1.0
+    flat = 0.3 * y
+    with BlobSystem(x, y, w) as a, BlobSystem(x, flat, w) as b:
+        full = a.velocity(p)
+        a.set(x, flat, w)
+        assert np.array_equal(a.velocity(p), b.velocity(p))
+        a.set(x, y, w)
+        assert np.array_equal(a.velocity(p), full)
+
+
 @pytest.mark.parametrize("n", [1, 7, 65536, 65537, 300001])
 @pytest.mark.parametrize("bad", [np.nan, np.inf, -np.inf])
 def test_not_finite_is_refused_anywhere(n, bad):
