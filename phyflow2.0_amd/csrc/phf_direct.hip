@@ -459,15 +459,15 @@ __global__ void vort_finish(const double *__restrict__ part, int nchunk, int64_t
 // of them together are below 2^-100 W, W = sum |w|: they cannot change a sum
 // of at least 2^-46 W beyond 2^-54 of its value.  Sources and targets are
 // sorted in Morton order; a wave of 64 targets takes only the blocks of 64
-// sources whose box comes within that radius of its own.  Waves with a target
+// sources whose box comes within that radius of its own.  Groups with a target
 // whose sum is too small for the argument (outside the flow, cancellation) go
 // over the blocks again, out to where a term is 0 in the class's arithmetic.
 // A plotting grid that reaches beyond the flow has many of those.
 // Whole calls, 100,003 sources and 90,601 targets in float64 / float32: every
-// pair 10.0 / 3.2 ms; this way 0.62 / 0.55 ms inside the flow, 1.32 / 0.96 ms
+// pair 10.0 / 3.2 ms; this way 0.61 / 0.55 ms inside the flow, 1.03 / 0.84 ms
 // on a grid twice as wide, 0.37 ms beside it (8.3 and 10.7 ms in either class
 // when each small sum took every source).  20,011 sources, 40,401 targets:
-// 1.01 / 0.42 ms; 0.33 / 0.32, 0.46 / 0.35, 0.22 ms.
+// 1.01 / 0.42 ms; 0.31 / 0.31, 0.50 / 0.36, 0.21 ms.
 constexpr double kVortCut = 69.4;   // exp(-69.4) < 2^-100
 // exp(-746) = 0 in float64; in float32 2^-150 = exp(-103.98) is 0, and r2 is
 // within 2^-20 of its value
@@ -507,25 +507,15 @@ __global__ __launch_bounds__(256) void vort_pack(const double *__restrict__ xb,
     }
 }
 
-// Partial sums of 64 sorted targets over the blocks b = blockIdx.y (mod
-// gridDim.y) within r2 = cut ks, so that neighbouring blocks go to different
-// waves; only for groups of targets with a bit in need, where that is given.
-// F32: the arithmetic of vort_f32c, 16 terms to a TwoSum.
+// Sum of a wave's 64 targets over the blocks b = first (mod step) within cut2
+// of their box.  F32: the arithmetic of vort_f32c, 16 terms to a TwoSum.
 template <bool F32>
-__global__ __launch_bounds__(64) void vort_near(const double4 *__restrict__ rec,
-                                                const double4 *__restrict__ box, int nblk,
-                                                const double *__restrict__ xt,
-                                                const double *__restrict__ yt,
-                                                const int32_t *__restrict__ perm, int64_t nt,
-                                                PairParams pp, double cut,
-                                                const unsigned long long *__restrict__ need,
-                                                double *__restrict__ part)
+__device__ __forceinline__ double vort_sum(const double4 *__restrict__ rec,
+                                           const double4 *__restrict__ box, int nblk, double tx,
+                                           double ty, const PairParams &pp, double cut2, int first,
+                                           int step)
 {
-    if (need && need[blockIdx.x] == 0) return;
-    const int lane = threadIdx.x;
-    const int64_t t = (int64_t)blockIdx.x * kWave + lane;
-    const int32_t o = perm[t < nt ? t : nt - 1];
-    const double tx = xt[o], ty = yt[o];
+    const int lane = threadIdx.x & 63;
     double x0 = tx, x1 = tx, y0 = ty, y1 = ty;
 #pragma unroll
     for (int d = 32; d > 0; d >>= 1) {
@@ -534,12 +524,10 @@ __global__ __launch_bounds__(64) void vort_near(const double4 *__restrict__ rec,
         y0 = fmin(y0, __shfl_xor(y0, d));
         y1 = fmax(y1, __shfl_xor(y1, d));
     }
-    const double cut2 = cut / pp.inv_ks;
-    const int ny = (int)gridDim.y;
     double a = 0.0;
     float h = 0.f, l = 0.f;
-    for (int b0 = (int)blockIdx.y; b0 < nblk; b0 += ny * kWave) {
-        const int bl = b0 + lane * ny;
+    for (int b0 = first; b0 < nblk; b0 += step * kWave) {
+        const int bl = b0 + lane * step;
         bool near = false;
         if (bl < nblk) {
             const double4 bx = box[bl];
@@ -548,7 +536,7 @@ __global__ __launch_bounds__(64) void vort_near(const double4 *__restrict__ rec,
             near = gx * gx + gy * gy < cut2;
         }
         for (unsigned long long m = __ballot(near); m; m &= m - 1) {
-            const int b = b0 + (__ffsll((long long)m) - 1) * ny;  // the same in every lane
+            const int b = b0 + (__ffsll((long long)m) - 1) * step;  // the same in every lane
             const double4 *rb = rec + (int64_t)__builtin_amdgcn_readfirstlane(b) * kVortBlk;
             if (F32) {
 #pragma unroll 1
@@ -585,7 +573,24 @@ __global__ __launch_bounds__(64) void vort_near(const double4 *__restrict__ rec,
             }
         }
     }
-    if (t < nt) part[(int64_t)blockIdx.y * nt + t] = F32 ? (double)h + (double)l : a;
+    return F32 ? (double)h + (double)l : a;
+}
+
+// Partial sums of 64 sorted targets over the near blocks b = blockIdx.y (mod
+// gridDim.y), so that neighbouring blocks go to different waves.
+template <bool F32>
+__global__ __launch_bounds__(64) void vort_near(const double4 *__restrict__ rec,
+                                                const double4 *__restrict__ box, int nblk,
+                                                const double *__restrict__ xt,
+                                                const double *__restrict__ yt,
+                                                const int32_t *__restrict__ perm, int64_t nt,
+                                                PairParams pp, double *__restrict__ part)
+{
+    const int64_t t = (int64_t)blockIdx.x * kWave + threadIdx.x;
+    const int32_t o = perm[t < nt ? t : nt - 1];
+    const double a = vort_sum<F32>(rec, box, nblk, xt[o], yt[o], pp, kVortCut / pp.inv_ks,
+                                   (int)blockIdx.y, (int)gridDim.y);
+    if (t < nt) part[(int64_t)blockIdx.y * nt + t] = a;
 }
 
 // The partials of sorted target t, scaled, to w[perm[t]]; a target whose sum
@@ -615,17 +620,33 @@ __global__ __launch_bounds__(256) void vort_near_finish(
     if (ok) w[perm[t]] = inv_pi * a / ks;
 }
 
-// the same for the targets in need
-__global__ __launch_bounds__(256) void vort_rest_finish(
-    const double *__restrict__ part, int nchunk, int64_t nt, const int32_t *__restrict__ perm,
-    double ks, double *__restrict__ w, const unsigned long long *__restrict__ need)
+// The targets in need, over every block that a term can come from: a workgroup
+// per group of 64, its waves in turn over the blocks and added in wave order.
+// (A second pass of vort_near and a finish of its own took 4 us more where
+// there are none.)
+constexpr int kRestWaves = 16;
+template <bool F32>
+__global__ __launch_bounds__(64 * kRestWaves) void vort_rest(
+    const double4 *__restrict__ rec, const double4 *__restrict__ box, int nblk,
+    const double *__restrict__ xt, const double *__restrict__ yt, const int32_t *__restrict__ perm,
+    int64_t nt, PairParams pp, double ks, double *__restrict__ w,
+    const unsigned long long *__restrict__ need)
 {
-    const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (t >= nt || !((need[t / kWave] >> (t % kWave)) & 1)) return;
+    const unsigned long long m = need[blockIdx.x];
+    if (m == 0) return;
+    __shared__ double sh[kRestWaves][kWave];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int64_t t = (int64_t)blockIdx.x * kWave + lane;
+    const int32_t o = perm[t < nt ? t : nt - 1];
+    sh[wv][lane] = vort_sum<F32>(rec, box, nblk, xt[o], yt[o], pp,
+                                 (F32 ? kVortZero32 : kVortZero64) / pp.inv_ks,
+                                 __builtin_amdgcn_readfirstlane(wv), kRestWaves);
+    __syncthreads();
+    if (wv != 0 || t >= nt || !((m >> lane) & 1)) return;
     double a = 0.0;
-    for (int c = 0; c < nchunk; ++c) a += part[(int64_t)c * nt + t];
+    for (int k = 0; k < kRestWaves; ++k) a += sh[k][lane];
     const double inv_pi = 1.0 / 3.141592653589793;
-    w[perm[t]] = inv_pi * a / ks;
+    w[o] = inv_pi * a / ks;
 }
 
 // ------------------------------------------------------------- host ------
@@ -861,19 +882,19 @@ static int vorticity_near(Lane *L, int prec, double ks, const PairParams &pp, co
     PHF_TRY(target_order(L, xt, yt, nt, bb, &pt));
     vort_pack<<<div_up(nblk, 4), 256, 0, L->stream>>>(xb, yb, wb, ps, nb, nblk, rec, box, wabs);
     const dim3 grid((unsigned)ngroups, (unsigned)nchunk);
-    auto pass = [&](double cut, const unsigned long long *groups) {
-        if (prec == PHF_PREC_F32C)
-            vort_near<true><<<grid, kWave, 0, L->stream>>>(rec, box, nblk, xt, yt, pt, nt, pp, cut,
-                                                           groups, part);
-        else
-            vort_near<false><<<grid, kWave, 0, L->stream>>>(rec, box, nblk, xt, yt, pt, nt, pp,
-                                                            cut, groups, part);
-    };
-    pass(kVortCut, nullptr);
+    const bool f32 = prec == PHF_PREC_F32C;
+    if (f32)
+        vort_near<true><<<grid, kWave, 0, L->stream>>>(rec, box, nblk, xt, yt, pt, nt, pp, part);
+    else
+        vort_near<false><<<grid, kWave, 0, L->stream>>>(rec, box, nblk, xt, yt, pt, nt, pp, part);
     vort_near_finish<<<div_up(nt, 256), 256, 0, L->stream>>>(part, nchunk, nt, pt, wabs, nblk, ks,
                                                              w, need);
-    pass(prec == PHF_PREC_F32C ? kVortZero32 : kVortZero64, need);
-    vort_rest_finish<<<div_up(nt, 256), 256, 0, L->stream>>>(part, nchunk, nt, pt, ks, w, need);
+    if (f32)
+        vort_rest<true><<<(unsigned)ngroups, 64 * kRestWaves, 0, L->stream>>>(
+            rec, box, nblk, xt, yt, pt, nt, pp, ks, w, need);
+    else
+        vort_rest<false><<<(unsigned)ngroups, 64 * kRestWaves, 0, L->stream>>>(
+            rec, box, nblk, xt, yt, pt, nt, pp, ks, w, need);
     PHF_HIP(hipGetLastError());
     return PHF_OK;
 }
