@@ -177,15 +177,16 @@ def test_step_whose_population_control_fails(H, fail):
     del keep
 
 
-def test_concurrent_results_do_not_pin_memory(H):
+def test_concurrent_results_do_not_pin_memory(fresh):
     """Several threads that fetch large results at once pin one set of slots
     between them, free none for the next fetch to pin again, and only the one
     that pins them waits for it."""
+    H = fresh
     n, threads, rounds = 300000, 6, 5
     systems = [system(H, n, seed=k) for k in range(threads)]
     barrier = threading.Barrier(threads)
     pinned, freed = H.hr_calls(b"hipHostMalloc"), H.hr_calls(b"hipHostFree")
-    H.hr_pin_delay_us(200000)
+    H.hr_pin_delay_us(1000000)
     bad, waits = [], []
 
     def work(k):
@@ -206,7 +207,7 @@ def test_concurrent_results_do_not_pin_memory(H):
     assert not bad
     assert H.hr_calls(b"hipHostMalloc") - pinned <= 1
     assert H.hr_calls(b"hipHostFree") == freed
-    assert sum(t > 0.15 for t in waits) <= 1
+    assert sum(t > 0.9 for t in waits) <= 1
     for s, _ in systems:
         assert H.phf_system_destroy(s) == 0
 
