@@ -220,7 +220,7 @@ __global__ void batch_gather(const BatchSys *__restrict__ sys, const int64_t *__
 __global__ void batch_clear_flag(int32_t *flag) { flag[0] = 0; }
 
 // --------------------------------------------------------------- P2M ------
-// p2m_leaf for 64 / R leaves per workgroup
+// p2m_wave for 64 / R leaves per workgroup
 template <class T, int NI, int R>
 __global__ __launch_bounds__(256) void batch_p2m(const BatchSys *__restrict__ sys,
                                                  const int64_t *__restrict__ loff,
@@ -231,16 +231,21 @@ __global__ __launch_bounds__(256) void batch_p2m(const BatchSys *__restrict__ sy
                                                  int p1, typename C2<T>::type *__restrict__ M)
 {
     const int64_t g = (int64_t)blockIdx.x * (64 / R) + threadIdx.x / (4 * R);
-    if (g >= nleaf) return;
-    const int s = find_seg(loff, S, g);
+    int32_t s0 = 0, s1 = 0;
+    int64_t at = -1;
+    double cx = 0.0, cy = 0.0, inv_s = 0.0;
+    const int s = find_seg(loff, S, g < nleaf ? g : nleaf - 1);
     const int L = sys[s].L;
-    if (L < 2) return;  // no far field in this system
-    const uint32_t b = (uint32_t)(g - sys[s].leafbase);
-    const BatchDom d = dom[s];
-    double cx, cy;
-    leaf_center(b, d.x0, d.y0, d.s, cx, cy);
-    p2m_leaf<T, NI, R, true>(src, start[g], start[g + 1], cx, cy, (T)(1.0 / d.s), p1,
-                             M + (lvl[L * (S + 1) + s] + b) * p1);
+    if (g < nleaf && L >= 2) {  // (else no far field in this system)
+        const uint32_t b = (uint32_t)(g - sys[s].leafbase);
+        const BatchDom d = dom[s];
+        leaf_center(b, d.x0, d.y0, d.s, cx, cy);
+        inv_s = 1.0 / d.s;
+        s0 = start[g];
+        s1 = start[g + 1];
+        at = (lvl[L * (S + 1) + s] + b) * p1;
+    }
+    p2m_wave<T, NI, R, true>(src, s0, s1, cx, cy, (T)inv_s, p1, M, at);
 }
 
 // --------------------------------------------------------- M2M / L2L ------

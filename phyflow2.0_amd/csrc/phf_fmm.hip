@@ -88,7 +88,7 @@ __global__ void gather_tgt_f64(const double *__restrict__ x, const double *__res
 __device__ __forceinline__ void far_priority() { __builtin_amdgcn_s_setprio(3); }
 
 // ---------------------------------------------------------------- P2M ----
-// p2m_leaf for 64 / R leaves per workgroup; inv_s is 1 / s.
+// p2m_wave for 64 / R leaves per workgroup; inv_s is 1 / s.
 template <class T, int NI, int R>
 __global__ __launch_bounds__(256) void p2m_kernel(const void *__restrict__ src,
                                                   const int32_t *__restrict__ start,
@@ -99,11 +99,15 @@ __global__ __launch_bounds__(256) void p2m_kernel(const void *__restrict__ src,
 {
     far_priority();
     const uint32_t b = blockIdx.x * (64 / R) + threadIdx.x / (4 * R);
-    if (b >= nleaf) return;
+    int32_t s0 = 0, s1 = 0;
+    if (b < nleaf) {
+        s0 = start[b];
+        s1 = start[b + 1];
+    }
     double cx = 0.0, cy = 0.0;
     if (sizeof(T) == 8) leaf_center(b, org->x, org->z, s, cx, cy);
-    p2m_leaf<T, NI, R, false>(src, start[b], start[b + 1], cx, cy, (T)inv_s, p1,
-                              M + (int64_t)b * p1);
+    p2m_wave<T, NI, R, false>(src, s0, s1, cx, cy, (T)inv_s, p1, M,
+                              b < nleaf ? (int64_t)b * p1 : -1);
 }
 
 // ---------------------------------------------------------- M2M / L2L ----

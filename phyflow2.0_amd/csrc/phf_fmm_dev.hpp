@@ -155,6 +155,35 @@ __device__ __forceinline__ void p2m_leaf(const void *__restrict__ src, int32_t s
     }
 }
 
+// p2m_leaf for the leaves of a wave, 64 / (4 R) of them; at < 0: none.  A leaf
+// taken by sixteen lanes is a serial chain of a quarter of its points, so the
+// whole wave takes the ones with more than `crowd`, one after another (a leaf's
+// sums depend on its own count alone; with MIX they are the same either way).
+// Leaves of 24 points on average have hardly one of 128; the full batches that
+// use sixteen lanes have leaves of 64 to 128, and their waves four of them to go
+// on with, so the line lies higher there.  float64, nearly all blobs in one
+// leaf of a tree of small ones: 8,628 blobs, order 24, 808 us by sixteen lanes
+// (280 with the table), 202 so; 41,025 blobs, order 16, 3,562 (944), 860.  Leaves
+// without a crowd among them take what they took.
+template <class T, int NI, int R, bool MIX>
+__device__ __forceinline__ void p2m_wave(const void *__restrict__ src, int32_t s0, int32_t s1,
+                                         double cx, double cy, T inv_s, int p1,
+                                         typename C2<T>::type *__restrict__ M, int64_t at)
+{
+    if constexpr (R < 16) {
+        constexpr int32_t crowd = MIX ? 256 : 128;
+        for (uint64_t m = __ballot(s1 - s0 > crowd); m;) {
+            const int l = __ffsll((unsigned long long)m) - 1;  // the leaf's first lane
+            m &= ~(((1ull << (4 * R)) - 1) << l);
+            p2m_leaf<T, NI, 16, MIX>(src, __shfl(s0, l), __shfl(s1, l), __shfl(cx, l),
+                                     __shfl(cy, l), __shfl(inv_s, l), p1,
+                                     M + __shfl((long long)at, l));
+        }
+        if (s1 - s0 > crowd) return;
+    }
+    if (at >= 0) p2m_leaf<T, NI, R, MIX>(src, s0, s1, cx, cy, inv_s, p1, M + at);
+}
+
 void set_error(const char *fmt, ...) __attribute__((format(printf, 1, 2)));
 
 // Whether leaves take sixteen lanes rather than a wave: where the mean leaf has

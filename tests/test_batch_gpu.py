@@ -257,3 +257,32 @@ def test_alone_equals_in_sparse_and_full_mixes(prec, order):
     for mix in (two, two + sparse, two + full):
         for got, ref in zip(run(mix), alone):
             assert np.array_equal(got, ref), (len(mix), prec, order)
+
+
+@pytest.mark.parametrize("prec", [PREC_F64, PREC_F32C])
+def test_crowded_leaves_alone_and_in_a_sparse_mix(prec):
+    """A wave takes a crowded leaf where the others have sixteen lanes each: the
+    same bits as where every leaf has a wave, on both sides of that count."""
+    rng = np.random.default_rng(3)
+    n = 20011
+    x, y = rng.random((2, n))
+    x[-2:], y[-2:] = [0.0, 1.0], [0.0, 1.0]
+    j = 0
+    for k, c in enumerate([200, 255, 256, 257, 900]):
+        x[j:j + c] = 0.11 + 0.125 * k + 1e-3 * x[j:j + c]
+        y[j:j + c] = 0.3 + 1e-3 * y[j:j + c]
+        j += c
+    w = rng.random(n)
+
+    def run(others):
+        with BatchSystems([n] + [q.shape[1] for q in others], [2e-3] + [0.01] * len(others),
+                          prec=prec, order=16) as b:
+            b.set_system(0, x, y, w)
+            for i, q in enumerate(others):
+                b.set_system(i + 1, *q)
+            b.velocity()
+            return b.get_velocity(0)
+
+    alone = run([])
+    sparse = run([rng.random((3, 5 + k % 7)) for k in range(2500)])
+    assert np.array_equal(alone, sparse)

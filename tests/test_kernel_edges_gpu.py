@@ -279,6 +279,56 @@ def test_not_finite_is_refused_anywhere(n, bad):
             BlobSystem(x, y, x)
 
 
+def _clumps(counts, n, seed):
+    """counts[k] of n points in a clump of side 0.01 within a leaf, the rest over
+    the unit square."""
+    rng = np.random.default_rng(seed)
+    x, y = rng.random((2, n))
+    x[-2:], y[-2:] = [0.0, 1.0], [0.0, 1.0]
+    j = 0
+    for k, c in enumerate(counts):
+        x[j:j + c] = 0.11 + 0.125 * k + 0.01 * x[j:j + c]
+        y[j:j + c] = 0.3 + 0.01 * y[j:j + c]
+        j += c
+    assert j <= n
+    return x, y, rng.random(n) + 0.5
+
+
+@pytest.mark.parametrize("order", [2, 12, 19, 31, 40])
+def test_crowded_leaves_among_small_ones(order, O):
+    """Leaves on both sides of where the whole wave takes one of those that have
+    sixteen lanes each; the bounds of test_multipole_orders."""
+    x, y, w = _clumps([127, 128, 129, 1, 257, 700], 4003, order)
+    xopt, cutoff = W.oseen_params(1e-3)
+    ref = O.direct_oseen(x, y, w, x, y, xopt, cutoff)
+    r = 0.5 ** 0.5
+    for prec, eps in ((F64, 1e-12), (F32C, 1e-6)):
+        got = gauss.fmm2d_gpu(x, y, w, x, y, 35, xopt, cutoff, 1e-6, prec=prec, order=order, leaf=8)
+        assert O.rel_l2(got, ref) <= (r / (2 - r)) ** (order + 1) + eps
+
+
+@pytest.mark.parametrize("prec", [F64, F32C])
+def test_a_crowded_leaf_is_no_longer_chain_in_a_deeper_tree(prec):
+    """Expanding one leaf with most of the blobs takes about as long in a tree
+    whose other leaves have few (sixteen lanes each, which alone would take four
+    times as long) as in one of a level less (a wave each)."""
+    from phyflow_amd.system import BlobSystem, vel_params
+    x, y, w = _clumps([9000], 10000, 1)
+
+    def ms(leaf):
+        p = vel_params(1e-4, prec=prec, order=16, leaf=leaf, leaf_side=-1.0)
+        with BlobSystem(x, y, w) as s:
+            runs = []
+            for _ in range(8):
+                s.velocity(p, fetch=False, eager=True)
+                runs.append(s.last_info["ms"]["p2m"])
+            return sorted(runs)[3], s.last_info["L"]
+
+    small, wave = ms(10), ms(40)
+    assert small[1] == wave[1] + 1
+    assert small[0] <= 2.0 * wave[0]
+
+
 def test_tree_shapes_in_turn(O):
     """More tree shapes than a lane keeps tables for, in changing order: the
     same bits every time a shape comes back, each against the direct sum.
