@@ -2065,7 +2065,7 @@ extern "C" int phf_fmm2d(const double *xb, const double *yb, const double *wb, i
         used[PHF_STAGE_P2P] = true;
         PairParams pp = make_oseen_params(xopt, cutoff);
         PHF_TRY(direct_device(L, PAIR_OSEEN, o.prec, pp, dxb, dyb, dwb, nb, dxt, dyt, nt, dqr,
-                              dqi));
+                              dqi, mostly_far(xb, yb, nb, xt, yt, nt, pp.c2)));
         tm.end(PHF_STAGE_P2P);
     } else {
         FmmArgs a{};

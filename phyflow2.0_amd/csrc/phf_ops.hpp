@@ -18,13 +18,17 @@ int download(Lane *L, const double *dev, int64_t n, double *host);
 // --- (a) all-pairs sum ----------------------------------------------------
 // o0/o1 receive, for PAIR_GAUSS_EPS, the reference velocity (vx, vy);
 // for PAIR_OSEEN the reference potentials (qr, qi).  All pointers device.
+// far: whether most pairs are beyond the kernel's core, so that a sum may sort
+// its points to skip them (mostly_far, of the host arrays).
+bool mostly_far(const double *xb, const double *yb, int64_t nb, const double *xt,
+                const double *yt, int64_t nt, double reach2);
 int direct_device(Lane *L, int kind, int prec, const PairParams &pp,
                   const double *xb, const double *yb, const double *wb,
                   int64_t nb, const double *xt, const double *yt, int64_t nt,
-                  double *o0, double *o1);
+                  double *o0, double *o1, bool far = true);
 // Gaussian induced vorticity (ww2parGauss) at the targets into w (device).
 int vorticity_device(Lane *L, int prec, double ksigmasqr, const double *xb, const double *yb,
                      const double *wb, int64_t nb, const double *xt, const double *yt, int64_t nt,
-                     double *w, bool cutoff = false);
+                     double *w, bool cutoff = false, bool far = true);
 
 }  // namespace phf

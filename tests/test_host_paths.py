@@ -241,6 +241,21 @@ def test_which_direct_sums_sort(H, nb, nt, prec, sort, near):
     assert (H.hr_launches(b"rs_scatter") > n[1]) == bool(near)
 
 
+@pytest.mark.parametrize("sigma,apart,sort,near", [
+    (0.02, 0.0, 1, 1), (0.2, 0.0, 0, 0), (1e9, 0.0, 0, 0), (0.2, 30.0, 1, 1), (1e-9, 1e300, 1, 1)])
+@pytest.mark.parametrize("nb,nt", [(20011, 20011), (5133, 90007)])
+def test_sums_of_wide_kernels_do_not_sort(H, nb, nt, sigma, apart, sort, near):
+    """Kernels as wide as the points' extent leave the sorted passes nothing to
+    skip: every pair without the sorts, for points that are not far apart."""
+    for field, prec, kernel, expect in (("velocity", 0, b"direct_f64_sorted", sort),
+                                        ("vorticity", 0, b"vort_near", near),
+                                        ("vorticity", 1, b"vort_near", near)):
+        n = H.hr_launches(kernel), H.hr_launches(b"rs_scatter")
+        assert direct(H, nb, nt, field, prec, 2 * sigma ** 2, apart) == 0, H.phf_last_error()
+        assert (H.hr_launches(kernel) > n[0]) == bool(expect), field
+        assert (H.hr_launches(b"rs_scatter") > n[1]) == bool(expect), field
+
+
 def fmm(H, n, order):
     """One fmm2d call of n blobs in the unit square at an expansion order."""
     from phyflow_amd._native import FmmOpts
@@ -293,11 +308,12 @@ def test_tables_without_memory_beyond_the_arena(H):
     del keep
 
 
-def direct(H, nb, nt, field, prec=0):
+def direct(H, nb, nt, field, prec=0, ks=1e-4, apart=0.0):
     r = np.random.default_rng(0)
     b, t, o = r.random((3, nb)), r.random((2, nt)), np.empty((2, nt))
+    t[0] += apart
     args = [ptr(b[0]), ptr(b[1]), ptr(b[2]), ctypes.c_int64(nb), ptr(t[0]), ptr(t[1]),
-            ctypes.c_int64(nt), ctypes.c_double(1e-4), ctypes.c_int32(prec)]
+            ctypes.c_int64(nt), ctypes.c_double(ks), ctypes.c_int32(prec)]
     if field == "velocity":
         return H.phf_vv2par_gauss(*args, ptr(o[0]), ptr(o[1]))
     return H.phf_ww2par_gauss(*args, ptr(o[0]))
