@@ -464,10 +464,10 @@ __global__ void vort_finish(const double *__restrict__ part, int nchunk, int64_t
 // over the blocks again, out to where a term is 0 in the class's arithmetic.
 // A plotting grid that reaches beyond the flow has many of those.
 // Whole calls, 100,003 sources and 90,601 targets in float64 / float32: every
-// pair 10.0 / 3.2 ms; this way 0.61 / 0.55 ms inside the flow, 1.03 / 0.84 ms
-// on a grid twice as wide, 0.37 ms beside it (8.3 and 10.7 ms in either class
+// pair 10.0 / 3.2 ms; this way 0.64 / 0.53 ms inside the flow, 0.70 / 0.65 ms
+// on a grid twice as wide, 0.40 ms beside it (8.3 and 10.7 ms in either class
 // when each small sum took every source).  20,011 sources, 40,401 targets:
-// 1.01 / 0.42 ms; 0.31 / 0.31, 0.50 / 0.36, 0.21 ms.
+// 1.01 / 0.42 ms; 0.36 / 0.26, 0.38 / 0.30, 0.22 ms.
 constexpr double kVortCut = 69.4;   // exp(-69.4) < 2^-100
 // exp(-746) = 0 in float64; in float32 2^-150 = exp(-103.98) is 0, and r2 is
 // within 2^-20 of its value
@@ -507,18 +507,20 @@ __global__ __launch_bounds__(256) void vort_pack(const double *__restrict__ xb,
     }
 }
 
-// Sum of a wave's 64 targets over the blocks b = first (mod step) within cut2
-// of their box.  F32: the arithmetic of vort_f32c, 16 terms to a TwoSum.
-template <bool F32>
+// Sum of a wave's TG targets (lane mod TG) over the blocks b = first (mod step)
+// within cut2 of their box; lane / TG takes that part of a block's sources.
+// F32: the arithmetic of vort_f32c, 16 terms to a TwoSum.
+template <bool F32, int TG>
 __device__ __forceinline__ double vort_sum(const double4 *__restrict__ rec,
                                            const double4 *__restrict__ box, int nblk, double tx,
                                            double ty, const PairParams &pp, double cut2, int first,
                                            int step)
 {
+    constexpr int NS = kVortBlk * TG / kWave;  // sources of a block per lane
     const int lane = threadIdx.x & 63;
     double x0 = tx, x1 = tx, y0 = ty, y1 = ty;
 #pragma unroll
-    for (int d = 32; d > 0; d >>= 1) {
+    for (int d = TG / 2; d > 0; d >>= 1) {
         x0 = fmin(x0, __shfl_xor(x0, d));
         x1 = fmax(x1, __shfl_xor(x1, d));
         y0 = fmin(y0, __shfl_xor(y0, d));
@@ -538,9 +540,10 @@ __device__ __forceinline__ double vort_sum(const double4 *__restrict__ rec,
         for (unsigned long long m = __ballot(near); m; m &= m - 1) {
             const int b = b0 + (__ffsll((long long)m) - 1) * step;  // the same in every lane
             const double4 *rb = rec + (int64_t)__builtin_amdgcn_readfirstlane(b) * kVortBlk;
+            if (TG < kWave) rb += lane / TG * NS;
             if (F32) {
 #pragma unroll 1
-                for (int k0 = 0; k0 < kVortBlk; k0 += 16) {
+                for (int k0 = 0; k0 < NS; k0 += 16) {
                     float s = 0.f;
 #pragma unroll
                     for (int k = 0; k < 16; ++k) {
@@ -553,7 +556,7 @@ __device__ __forceinline__ double vort_sum(const double4 *__restrict__ rec,
                 }
             } else {
 #pragma unroll 1
-                for (int k0 = 0; k0 < kVortBlk; k0 += 4) {
+                for (int k0 = 0; k0 < NS; k0 += 4) {
                     double r2[4], w[4];
 #pragma unroll
                     for (int k = 0; k < 4; ++k) {
@@ -588,8 +591,8 @@ __global__ __launch_bounds__(64) void vort_near(const double4 *__restrict__ rec,
 {
     const int64_t t = (int64_t)blockIdx.x * kWave + threadIdx.x;
     const int32_t o = perm[t < nt ? t : nt - 1];
-    const double a = vort_sum<F32>(rec, box, nblk, xt[o], yt[o], pp, kVortCut / pp.inv_ks,
-                                   (int)blockIdx.y, (int)gridDim.y);
+    const double a = vort_sum<F32, kWave>(rec, box, nblk, xt[o], yt[o], pp, kVortCut / pp.inv_ks,
+                                          (int)blockIdx.y, (int)gridDim.y);
     if (t < nt) part[(int64_t)blockIdx.y * nt + t] = a;
 }
 
@@ -621,10 +624,14 @@ __global__ __launch_bounds__(256) void vort_near_finish(
 }
 
 // The targets in need, over every block that a term can come from: a workgroup
-// per group of 64, its waves in turn over the blocks and added in wave order.
-// (A second pass of vort_near and a finish of its own took 4 us more where
-// there are none.)
-constexpr int kRestWaves = 16;
+// takes sixteen at a time, its waves in turn over the blocks and added in wave
+// order; lanes of targets that are not in need take the place of one that is.
+// So a few of them keep many CUs busy: 20,011 sources, 40,401 targets, sigma three
+// spacings, a grid half as wide again 876 / 436 us, 644 / 351 so (1,000 / 420 for
+// every pair; 64 at a time by sixteen waves before).  Beside a flow, where every
+// target is in need and no block near, the box tests are four times as many
+// (100,003 sources, 90,601 targets: 373 and 398 us).
+constexpr int kRestT = 16, kRestWaves = 8, kRestGrid = 2048;
 template <bool F32>
 __global__ __launch_bounds__(64 * kRestWaves) void vort_rest(
     const double4 *__restrict__ rec, const double4 *__restrict__ box, int nblk,
@@ -632,21 +639,29 @@ __global__ __launch_bounds__(64 * kRestWaves) void vort_rest(
     int64_t nt, PairParams pp, double ks, double *__restrict__ w,
     const unsigned long long *__restrict__ need)
 {
-    const unsigned long long m = need[blockIdx.x];
-    if (m == 0) return;
-    __shared__ double sh[kRestWaves][kWave];
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    const int64_t t = (int64_t)blockIdx.x * kWave + lane;
-    const int32_t o = perm[t < nt ? t : nt - 1];
-    sh[wv][lane] = vort_sum<F32>(rec, box, nblk, xt[o], yt[o], pp,
-                                 (F32 ? kVortZero32 : kVortZero64) / pp.inv_ks,
-                                 __builtin_amdgcn_readfirstlane(wv), kRestWaves);
-    __syncthreads();
-    if (wv != 0 || t >= nt || !((m >> lane) & 1)) return;
-    double a = 0.0;
-    for (int k = 0; k < kRestWaves; ++k) a += sh[k][lane];
-    const double inv_pi = 1.0 / 3.141592653589793;
-    w[o] = inv_pi * a / ks;
+    __shared__ double sh[kRestWaves][kRestT];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, i = lane % kRestT;
+    for (int64_t t0 = (int64_t)blockIdx.x * kRestT; t0 < nt; t0 += (int64_t)gridDim.x * kRestT) {
+        // (targets beyond nt are not in need)
+        const uint32_t m = (uint32_t)(need[t0 / kWave] >> (t0 % kWave)) & ((1u << kRestT) - 1);
+        if (m == 0) continue;
+        const bool mine = (m >> i) & 1;
+        const int32_t o = perm[t0 + (mine ? i : __ffs((int)m) - 1)];
+        double a = vort_sum<F32, kRestT>(rec, box, nblk, xt[o], yt[o], pp,
+                                         (F32 ? kVortZero32 : kVortZero64) / pp.inv_ks,
+                                         __builtin_amdgcn_readfirstlane(wv), kRestWaves);
+#pragma unroll
+        for (int d = kRestT; d < kWave; d <<= 1) a += __shfl_xor(a, d);
+        if (lane < kRestT) sh[wv][lane] = a;
+        __syncthreads();
+        if ((int)threadIdx.x < kRestT && mine) {
+            a = 0.0;
+            for (int k = 0; k < kRestWaves; ++k) a += sh[k][i];
+            const double inv_pi = 1.0 / 3.141592653589793;
+            w[o] = inv_pi * a / ks;
+        }
+        __syncthreads();
+    }
 }
 
 // ------------------------------------------------------------- host ------
@@ -913,6 +928,7 @@ static int vorticity_near(Lane *L, int prec, double ks, const PairParams &pp, co
     PHF_TRY(target_order(L, xt, yt, nt, bb, &pt));
     vort_pack<<<div_up(nblk, 4), 256, 0, L->stream>>>(xb, yb, wb, ps, nb, nblk, rec, box, wabs);
     const dim3 grid((unsigned)ngroups, (unsigned)nchunk);
+    const unsigned rgrid = std::min(div_up(nt, kRestT), (unsigned)kRestGrid);
     const bool f32 = prec == PHF_PREC_F32C;
     if (f32)
         vort_near<true><<<grid, kWave, 0, L->stream>>>(rec, box, nblk, xt, yt, pt, nt, pp, part);
@@ -921,10 +937,10 @@ static int vorticity_near(Lane *L, int prec, double ks, const PairParams &pp, co
     vort_near_finish<<<div_up(nt, 256), 256, 0, L->stream>>>(part, nchunk, nt, pt, wabs, nblk, ks,
                                                              w, need);
     if (f32)
-        vort_rest<true><<<(unsigned)ngroups, 64 * kRestWaves, 0, L->stream>>>(
+        vort_rest<true><<<rgrid, 64 * kRestWaves, 0, L->stream>>>(
             rec, box, nblk, xt, yt, pt, nt, pp, ks, w, need);
     else
-        vort_rest<false><<<(unsigned)ngroups, 64 * kRestWaves, 0, L->stream>>>(
+        vort_rest<false><<<rgrid, 64 * kRestWaves, 0, L->stream>>>(
             rec, box, nblk, xt, yt, pt, nt, pp, ks, w, need);
     PHF_HIP(hipGetLastError());
     return PHF_OK;

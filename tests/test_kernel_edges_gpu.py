@@ -189,6 +189,26 @@ def test_vorticity_beyond_the_flow_is_not_the_whole_sum(prec):
     assert t(1.0, 2.0) <= 2.0 * inside
 
 
+def test_a_few_small_sums_are_no_long_chain():
+    """Broad blobs and a grid that reaches a little beyond them: the targets in
+    its corners, a hundredth of all, have small sums out of most of the blobs.
+    They cost what the others cost, not as much again."""
+    import time
+    x, y, w, xt, yt, ks = _flow_and_targets(20011, 40401, 3)
+    ks = 18.0 / x.size
+
+    def t(sx):
+        a, b = (xt - 0.5) * sx + 0.5, (yt - 0.5) * sx + 0.5
+        runs = []
+        for _ in range(9):
+            t0 = time.perf_counter()
+            gauss.ww2parGauss_gpu(x, y, w, a, b, ks, 128)
+            runs.append(time.perf_counter() - t0)
+        return sorted(runs)[4]
+
+    assert t(1.5) <= 1.8 * t(1.0)
+
+
 @pytest.mark.parametrize("n", [1, 5461, 5462, 87381, 87382, 131072, 131073, 800001])
 def test_blobs_come_back_whole(n):
     """Results by one packed transfer, by the runtime's copies and through the
