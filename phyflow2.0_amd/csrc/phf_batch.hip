@@ -245,7 +245,7 @@ __global__ __launch_bounds__(256) void batch_p2m(const BatchSys *__restrict__ sy
         s1 = start[g + 1];
         at = (lvl[L * (S + 1) + s] + b) * p1;
     }
-    p2m_wave<T, NI, R, true>(src, s0, s1, cx, cy, (T)inv_s, p1, M, at);
+    p2m_wave<T, NI, R>(src, s0, s1, cx, cy, (T)inv_s, p1, M, at);
 }
 
 // --------------------------------------------------------- M2M / L2L ------
@@ -1051,12 +1051,18 @@ static int batch_enqueue_typed(Lane *L, const BatchPlan &P, BatchBuffers &Bf, co
     const VC *m2m = reinterpret_cast<const VC *>(Bf.m2m);
     const VC *l2l = reinterpret_cast<const VC *>(Bf.l2l);
     if (P.Lmax >= 2) {
-        const bool narrow = p2m_narrow_batch((double)P.N, (double)P.nleaf);
-        PHF_TRY(p2m_dispatch(p1, narrow, [&](auto ni, auto r) {
-            constexpr int R = decltype(r)::value;
-            batch_p2m<T, decltype(ni)::value, R>
-                <<<div_up(P.nleaf, 64 / R), 256, 0, L->stream>>>(
-                    Bf.sys, Bf.loff, Bf.lvl, S, Bf.dom, Bf.src, sp, P.nleaf, p1, M);
+        const bool narrow = p2m_narrow((double)P.N, (double)P.nleaf);
+        PHF_TRY(p2m_dispatch(p1, [&](auto ni) {
+            auto launch = [&](auto r) {
+                constexpr int R = decltype(r)::value;
+                batch_p2m<T, decltype(ni)::value, R>
+                    <<<div_up(P.nleaf, 64 / R), 256, 0, L->stream>>>(
+                        Bf.sys, Bf.loff, Bf.lvl, S, Bf.dom, Bf.src, sp, P.nleaf, p1, M);
+            };
+            if (narrow)
+                launch(std::integral_constant<int, 4>());
+            else
+                launch(std::integral_constant<int, 16>());
         }));
         for (int l = P.Lmax - 1; l >= 2; --l) {
             const int64_t nb = P.lvl[(size_t)l * (S + 1) + S] - P.lvl[(size_t)l * (S + 1)];

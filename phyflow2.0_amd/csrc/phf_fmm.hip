@@ -88,26 +88,49 @@ __global__ void gather_tgt_f64(const double *__restrict__ x, const double *__res
 __device__ __forceinline__ void far_priority() { __builtin_amdgcn_s_setprio(3); }
 
 // ---------------------------------------------------------------- P2M ----
-// p2m_wave for 64 / R leaves per workgroup; inv_s is 1 / s.
-template <class T, int NI, int R>
+// Expansions of four leaves, the children of one box, per workgroup: a wave each,
+// or, if none has more than `few` points, all by one wave with sixteen lanes
+// each.  A wave takes up to 32 points in two rounds and then spends its time on
+// the butterfly, which sixteen lanes have half of; but they are a serial chain of
+// a quarter of the points.  The four counts decide, so the sums follow from the
+// points alone, and a crowded leaf is not waited for by lanes of small ones.
+// float32, order 16, a wave each / by this rule: 300,000 uniform blobs in leaves
+// of 18 22.9 / 18.8 us, 1M 31.5 / 28.7; a line at 48 took 9.6 instead of 6.8 us
+// for 20,000 float64 blobs.  With one choice for the launch from the mean leaf, a
+// thin ring of 20,000 (float64) took 28 us (14 now) or followed its bounding box.
+// One leaf with nearly all blobs, float64: 8,628 blobs, order 24, 808 us by
+// sixteen lanes, 280 with the table, 202 by a wave.
+// inv_s is 1 / s.
+template <class T, int NI>
 __global__ __launch_bounds__(256) void p2m_kernel(const void *__restrict__ src,
-                                                  const int32_t *__restrict__ start,
-                                                  uint32_t nleaf, int p1,
+                                                  const int32_t *__restrict__ start, int p1,
                                                   const double4 *__restrict__ org, double s,
                                                   double inv_s,
                                                   typename C2<T>::type *__restrict__ M)
 {
+    constexpr int32_t few = 32;
     far_priority();
-    const uint32_t b = blockIdx.x * (64 / R) + threadIdx.x / (4 * R);
-    int32_t s0 = 0, s1 = 0;
-    if (b < nleaf) {
-        s0 = start[b];
-        s1 = start[b + 1];
-    }
+    const int32_t *st = start + 4 * blockIdx.x;
+    int32_t s0[5];
+#pragma unroll
+    for (int k = 0; k < 5; ++k) s0[k] = st[k];
+    int32_t most = 0;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) most = max(most, s0[k + 1] - s0[k]);
+    const int wv = threadIdx.x >> 6;
+    const bool one = most <= few;
+    if (one && wv != 0) return;
+    const int k = one ? (int)(threadIdx.x >> 4) : wv;
+    const uint32_t b = 4 * blockIdx.x + k;
     double cx = 0.0, cy = 0.0;
     if (sizeof(T) == 8) leaf_center(b, org->x, org->z, s, cx, cy);
-    p2m_wave<T, NI, R, false>(src, s0, s1, cx, cy, (T)inv_s, p1, M,
-                              b < nleaf ? (int64_t)b * p1 : -1);
+    typename C2<T>::type *out = M + (int64_t)b * p1;
+    const int32_t j0 = k == 0 ? s0[0] : k == 1 ? s0[1] : k == 2 ? s0[2] : s0[3];
+    const int32_t j1 = k == 0 ? s0[1] : k == 1 ? s0[2] : k == 2 ? s0[3] : s0[4];
+    if (one)
+        p2m_leaf<T, NI, 4, false>(src, j0, j1, cx, cy, (T)inv_s, p1, out);
+    else
+        p2m_leaf<T, NI, 16, false>(src, j0, j1, cx, cy, (T)inv_s, p1, out);
 }
 
 // ---------------------------------------------------------- M2M / L2L ----
@@ -1549,11 +1572,9 @@ static int run_fmm_typed(Lane *L, const FmmArgs &a, const Domain &dom, const Sor
         // P2M
         tm.begin(PHF_STAGE_P2M);
         used[PHF_STAGE_P2M] = true;
-        PHF_TRY(p2m_dispatch(p1, p2m_narrow((double)a.nb, dom.occupied), [&](auto ni, auto r) {
-            constexpr int R = decltype(r)::value;
-            p2m_kernel<T, decltype(ni)::value, R>
-                <<<(nleaf + 64 / R - 1) / (64 / R), 256, 0, L->stream>>>(
-                    src, sp, nleaf, p1, dom.org, dom.s, 1.0 / dom.s, M + off[Lv] * p1);
+        PHF_TRY(p2m_dispatch(p1, [&](auto ni) {
+            p2m_kernel<T, decltype(ni)::value><<<nleaf / 4, 256, 0, L->stream>>>(
+                src, sp, p1, dom.org, dom.s, 1.0 / dom.s, M + off[Lv] * p1);
         }));
         PHF_HIP(hipGetLastError());
         tm.end(PHF_STAGE_P2M);
@@ -1703,14 +1724,13 @@ static int fmm_enqueue(Lane *L, const FmmArgs &a, const Domain &dom_in, StageTim
 // slices).  A call replays the most recent entry without waiting for the
 // bounding box: kernels read the domain corner on the device, and the
 // bounding box comes back with the results, so that the caller can check
-// that the points kept the recording's leaf level, domain side and P2M lanes
-// (else it evaluates again with a fresh recording: the results follow from the
-// points alone).
+// that the points kept the recording's leaf level and domain side, from which
+// the order of every sum follows (else it evaluates again with a fresh
+// recording).
 struct FmmGraph {
     FmmArgs a{};
     int L = 0, nnear = 0;
     double D = 0.0;
-    bool narrow = false;  // P2M's lanes, which its sums' order follows
     Arena::Mark m0, m1;
     hipGraph_t g[2] = {};
     hipGraphExec_t exec[2] = {};
@@ -1782,7 +1802,6 @@ static int fmm_record(Lane *L, const FmmArgs &a, const Domain &dom0, FmmGraph **
     e->a = a;
     e->L = dom0.L;
     e->D = dom0.D;
-    e->narrow = p2m_narrow((double)a.nb, dom0.occupied);
     e->m0 = L->arena.mark();
     StageTimer off(L, false);
     bool used[PHF_STAGE_COUNT] = {};
@@ -1977,13 +1996,11 @@ int fmm_device(Lane *L, const FmmArgs &a, StageTimer &tm, bool *used, FmmInfo *i
             }
             const int L0 = e->L;
             const double D0 = e->D;
-            const bool n0 = e->narrow;
-            info->domain_ok = [hb, a, L0, D0, n0, shape_log2]() {
+            info->domain_ok = [hb, a, L0, D0, shape_log2]() {
                 const Domain d = choose_domain(*hb, a.Lhint, (double)a.nb, (double)a.nt,
                                                a.cutoff, a.ws, shape_log2, a.p + 1,
                                                a.prec == PHF_PREC_F32C ? 16 : 64, a.leaf_side);
-                return d.L == L0 && d.D == D0 &&
-                       p2m_narrow((double)a.nb, d.occupied) == n0;
+                return d.L == L0 && d.D == D0;
             };
         }
         nnear = e->nnear;

@@ -155,74 +155,61 @@ __device__ __forceinline__ void p2m_leaf(const void *__restrict__ src, int32_t s
     }
 }
 
-// p2m_leaf for the leaves of a wave, 64 / (4 R) of them; at < 0: none.  A leaf
-// taken by sixteen lanes is a serial chain of a quarter of its points, so the
-// whole wave takes the ones with more than `crowd`, one after another (a leaf's
-// sums depend on its own count alone; with MIX they are the same either way).
-// Leaves of 24 points on average have hardly one of 128; the full batches that
-// use sixteen lanes have leaves of 64 to 128, and their waves four of them to go
-// on with, so the line lies higher there.  float64, nearly all blobs in one
-// leaf of a tree of small ones: 8,628 blobs, order 24, 808 us by sixteen lanes
-// (280 with the table), 202 so; 41,025 blobs, order 16, 3,562 (944), 860.  Leaves
-// without a crowd among them take what they took.
-template <class T, int NI, int R, bool MIX>
+// p2m_leaf with MIX for the leaves of a wave, 64 / (4 R) of them; at < 0: none.
+// A leaf taken by sixteen lanes is a serial chain of a quarter of its points, so
+// the whole wave takes the ones with more than `crowd`, one after another, with
+// the same sums.  The full batches that use sixteen lanes have leaves of 64 to
+// 128, and their waves four of them to go on with: they take what they took.
+template <class T, int NI, int R>
 __device__ __forceinline__ void p2m_wave(const void *__restrict__ src, int32_t s0, int32_t s1,
                                          double cx, double cy, T inv_s, int p1,
                                          typename C2<T>::type *__restrict__ M, int64_t at)
 {
     if constexpr (R < 16) {
-        constexpr int32_t crowd = MIX ? 256 : 128;
+        constexpr int32_t crowd = 256;
         for (uint64_t m = __ballot(s1 - s0 > crowd); m;) {
             const int l = __ffsll((unsigned long long)m) - 1;  // the leaf's first lane
             m &= ~(((1ull << (4 * R)) - 1) << l);
-            p2m_leaf<T, NI, 16, MIX>(src, __shfl(s0, l), __shfl(s1, l), __shfl(cx, l),
-                                     __shfl(cy, l), __shfl(inv_s, l), p1,
-                                     M + __shfl((long long)at, l));
+            p2m_leaf<T, NI, 16, true>(src, __shfl(s0, l), __shfl(s1, l), __shfl(cx, l),
+                                      __shfl(cy, l), __shfl(inv_s, l), p1,
+                                      M + __shfl((long long)at, l));
         }
         if (s1 - s0 > crowd) return;
     }
-    if (at >= 0) p2m_leaf<T, NI, R, MIX>(src, s0, s1, cx, cy, inv_s, p1, M + at);
+    if (at >= 0) p2m_leaf<T, NI, R, true>(src, s0, s1, cx, cy, inv_s, p1, M + at);
 }
 
 void set_error(const char *fmt, ...) __attribute__((format(printf, 1, 2)));
 
-// Whether leaves take sixteen lanes rather than a wave: where the mean leaf has
-// fewer than 24 points, which a wave takes in little more than one round of its
-// 16 points and then spends on the butterfly; and in a batch, which has nothing
+// Whether a batch's leaves take sixteen lanes rather than a wave: where the mean
+// leaf has fewer than 24 points, which a wave takes in little more than one round
+// of its 16 points and then spends on the butterfly; and, as a batch has nothing
 // beside it, where leaves fill the chip, since sixteen lanes go four times as
 // long but with an eighth of the butterfly.  Batches of leaves of 64 float32
 // points, order 13: 1,024 leaves 4.8 us by waves, 8.0 by sixteen lanes; 8,192
 // leaves 9.0 and 9.8, 16,384 15.4 and 15.0, 131,072 128.6 and 88.1 (108.5 with
 // the table).
-inline bool p2m_narrow(double points, double leaves) { return points < 24.0 * leaves; }
-inline bool p2m_narrow_batch(double points, double leaves)
+inline bool p2m_narrow(double points, double leaves)
 {
-    return p2m_narrow(points, leaves) || leaves >= 12288.0;
+    return points < 24.0 * leaves || leaves >= 12288.0;
 }
 
-// f(integral constants NI, R) for the compiled NI that holds p1 powers and the
-// lanes of a leaf
+// f(integral constant NI) for the compiled NI that holds p1 powers
 template <class F>
-inline int p2m_dispatch(int p1, bool narrow, const F &f)
+inline int p2m_dispatch(int p1, const F &f)
 {
-    auto lanes = [&](auto ni) {
-        if (narrow)
-            f(ni, std::integral_constant<int, 4>());
-        else
-            f(ni, std::integral_constant<int, 16>());
-    };
     if (p1 <= 12)
-        lanes(std::integral_constant<int, 3>());
+        f(std::integral_constant<int, 3>());
     else if (p1 <= 16)
-        lanes(std::integral_constant<int, 4>());
+        f(std::integral_constant<int, 4>());
     else if (p1 <= 20)
-        lanes(std::integral_constant<int, 5>());
+        f(std::integral_constant<int, 5>());
     else if (p1 <= 24)
-        lanes(std::integral_constant<int, 6>());
+        f(std::integral_constant<int, 6>());
     else if (p1 <= 32)
-        lanes(std::integral_constant<int, 8>());
+        f(std::integral_constant<int, 8>());
     else if (p1 <= 44)
-        lanes(std::integral_constant<int, 11>());
+        f(std::integral_constant<int, 11>());
     else {
         set_error("expansion order %d too large (max 40)", p1 - 1);
         return PHF_ERR_UNSUPPORTED;

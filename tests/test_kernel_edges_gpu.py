@@ -284,6 +284,34 @@ def test_replay_follows_from_the_points_alone(prec, leaf):
         assert np.array_equal(a.velocity(p), full)
 
 
+@pytest.mark.parametrize("prec", [F64, F32C])
+def test_points_that_keep_the_domain_are_replayed(prec):
+    """Points that fill the same domain otherwise are evaluated by the launches
+    that were recorded: a system whose points change between two such states
+    every time takes about as long as one that stays, not several times that."""
+    import time
+    from phyflow_amd.system import BlobSystem, vel_params
+    n = 16000
+    s = W.uniform_system(n, seed=4)
+    p = vel_params(0.2 * s["sigma"], prec=prec, order=17, leaf=16, leaf_side=-1.0)
+    x, y, w = s["x"], s["y"], s["w"]
+    x[0], x[1] = 0.0, 1.0
+    y[0], y[1] = 0.0, 1.0
+    states = y, 0.3 * y
+
+    def t(b, turns):
+        runs = []
+        for k in range(12):
+            b.set(x, states[k % turns], w)
+            t0 = time.perf_counter()
+            b.velocity(p)
+            runs.append(time.perf_counter() - t0)
+        return sorted(runs)[6]
+
+    with BlobSystem(x, y, w) as b:
+        assert t(b, 2) <= 2.0 * t(b, 1)
+
+
 @pytest.mark.parametrize("n", [1, 7, 65536, 65537, 300001])
 @pytest.mark.parametrize("bad", [np.nan, np.inf, -np.inf])
 def test_not_finite_is_refused_anywhere(n, bad):
@@ -316,9 +344,10 @@ def _clumps(counts, n, seed):
 
 @pytest.mark.parametrize("order", [2, 12, 19, 31, 40])
 def test_crowded_leaves_among_small_ones(order, O):
-    """Leaves on both sides of where the whole wave takes one of those that have
-    sixteen lanes each; the bounds of test_multipole_orders."""
-    x, y, w = _clumps([127, 128, 129, 1, 257, 700], 4003, order)
+    """Leaves on both sides of where four have a wave each in place of sixteen
+    lanes (the clumps' leaves have some 3 points more); the bounds of
+    test_multipole_orders."""
+    x, y, w = _clumps([27, 28, 29, 30, 31, 32, 700], 4003, order)
     xopt, cutoff = W.oseen_params(1e-3)
     ref = O.direct_oseen(x, y, w, x, y, xopt, cutoff)
     r = 0.5 ** 0.5
@@ -330,8 +359,8 @@ def test_crowded_leaves_among_small_ones(order, O):
 @pytest.mark.parametrize("prec", [F64, F32C])
 def test_a_crowded_leaf_is_no_longer_chain_in_a_deeper_tree(prec):
     """Expanding one leaf with most of the blobs takes about as long in a tree
-    whose other leaves have few (sixteen lanes each, which alone would take four
-    times as long) as in one of a level less (a wave each)."""
+    whose other leaves have few (sixteen lanes, as those have, would take four
+    times as long) as in one of a level less."""
     from phyflow_amd.system import BlobSystem, vel_params
     x, y, w = _clumps([9000], 10000, 1)
 
